@@ -9,7 +9,10 @@
 //                     order (bit-exact cell indices), trilinear or Gaussian
 //                     smoothing over (2 dmax + 1)^3 cells (343 for the
 //                     default dmax = 3) of delta and eta, then the FGPA
-//   k_gather_plane_tri  the same for plane-parallel skewers and trilinear
+//   k_gather_radial   the Gaussian smoothing of radial skewers with eta: a
+//                     block per run of pixels, their stencils' cells once in
+//                     LDS with eta and v projected on the line
+//   k_gather_plane_tri  k_gather for plane-parallel skewers and trilinear
 //                     interpolation, with the eight corner loads of both
 //                     fields issued together
 //   k_missing_power   one FFT line per skewer, T skewers per block, one
@@ -283,6 +286,500 @@ __global__ __launch_bounds__(256) void k_gather(GatherArgs a) {
       const float gfield = dl + ds + prow.z * eta;
       a.flux[pix] = expf(-prow.x * expf(prow.y * prow.w * gfield));
     }
+  }
+}
+
+// ------------------------------------- Gaussian smoothing of radial lines
+// The sums over (2 DM + 1)^3 cells with weights exp(-dr^2 / (2 D^2)) along
+// radial lines of sight (make_spectra.py:39-139), NT pixels of one skewer at
+// a time, a thread each:
+//  - a radial line needs eta and v only along its own direction n, the same
+//    for all its pixels: sum_ij n_i n_j eta_ij and sum_i n_i v_i are formed
+//    once per cell, so a pixel sums one or two fields besides delta, not nine;
+//  - about D / dr = 11 consecutive pixels lie in one cell and the stencils of
+//    NT of them overlap almost whole, so the block loads their union into LDS
+//    once: per z plane a window of WX x WY cells that follows the line (delta
+//    as it is, the contracted fields in FP64);
+//  - the weights factor over the axes: a row of W cells costs W multiply-adds
+//    per field and the outer axes add 1 / W and 1 / W^2 of that; with u the
+//    pixel's distance from its cell's centre in cells, w_d = exp(-u d)
+//    exp(-d^2 / 2) up to exp(-u^2 / 2), which the normalisation cancels: one
+//    exponential per axis instead of W.
+// All sums in FP64, as k_gather's.
+//
+// It replaces a thread per pixel with W^3 loads per field, whose ten fields
+// of 49 rows each did not fit the 32 KB L1.  16 000 radial skewers (3.9e7
+// forest pixels, dmax 3) of a 166 x 2560 x 1536 slab: 115 -> 7.2 ms with six
+// eta boxes; 2 100 skewers with the velocities too: 24.9 -> 1.57 ms.  VALU
+// issue is 40 % of that (2800 instructions per wave and part, half of them
+// the row sums), L2 misses run at 3.6 TB/s (each part reads its rows' 128 B
+// lines anew); the rest is latency between the barriers at 4 waves per SIMD.
+// Measured against it: chunks of 2 to 4 pixels of one cell per lane (a
+// quarter of the LDS reads, but 190 to 256 registers and half the waves)
+// 7.6 to 11 ms, 128 pixels 8.2, 512 pixels 9.2, spans of 8192 pixels 7.5.
+constexpr int GG_NK = 128;   // z planes of one tube
+
+// exp(-d^2 / 2), d = 0 .. 6
+__constant__ const double GG_E[7] = {1.0,
+                                     0.60653065971263342,
+                                     0.1353352832366127,
+                                     0.011108996538242306,
+                                     0.00033546262790251185,
+                                     3.7266531720786709e-06,
+                                     1.5229979744712629e-08};
+
+struct LosPixel {
+  int64_t ix, iy, iz;   // containing cell, make_spectra.py:47-49
+  double tx, ty, tz;    // position in cells from the box corner
+  double R;
+};
+
+struct Los {
+  double qx, qy, qz, qr;   // the skewer
+  double cx, cy, cz;       // its direction q / qr
+  double inv_d;
+  double nn[6], nv[3];     // factors of the six eta_ij and of the three velocities
+};
+
+// t is so near an integer that the rounding of the reference's own operation
+// order decides the cell, or too large for a 32-bit index; mag bounds the
+// magnitude of the terms t is the sum of
+__device__ __forceinline__ bool los_near(double t, double mag) {
+  return !(fabs(t - rint(t)) > 1e-9 + 1e-14 * mag) || !(fabs(t) < 1.0e9);
+}
+
+// Pixel g of a radial line of sight.  Positions by products with reciprocals
+// (a few ulp from the reference's quotients); where that could change the
+// cell, by the reference's own operations (make_spectra.py:312,450-452,47-49),
+// so the cell is always the reference's.
+__device__ __forceinline__ LosPixel los_pixel(const GatherArgs& a, const Los& l, int64_t g) {
+  LosPixel q;
+  const double R = add_rn(a.sk.rmin, mul_rn((double)g, a.sk.dr));
+  q.R = R;
+  double X = R * l.cx, Y = R * l.cy, Z = R * l.cz;
+  q.tx = (X + a.hx) * l.inv_d;
+  q.ty = (Y + a.hy) * l.inv_d;
+  q.tz = (Z + a.hz - a.box.r0) * l.inv_d;
+  if (los_near(q.tx, (fabs(X) + a.hx) * l.inv_d) || los_near(q.ty, (fabs(Y) + a.hy) * l.inv_d) ||
+      los_near(q.tz, (fabs(Z) + a.hz + fabs(a.box.r0)) * l.inv_d)) {
+    X = div_rn(mul_rn(R, l.qx), l.qr);
+    Y = div_rn(mul_rn(R, l.qy), l.qr);
+    Z = div_rn(mul_rn(R, l.qz), l.qr);
+    const double D = a.box.cell;
+    q.tx = div_rn(add_rn(X, a.hx), D);
+    q.ty = div_rn(add_rn(Y, a.hy), D);
+    q.tz = div_rn(sub_rn(add_rn(Z, a.hz), a.box.r0), D);
+    q.ix = (int64_t)q.tx;
+    q.iy = (int64_t)q.ty;
+    q.iz = (int64_t)q.tz;
+  } else {
+    q.ix = (int)q.tx;
+    q.iy = (int)q.ty;
+    q.iz = (int)q.tz;
+  }
+  return q;
+}
+
+// multiple of n that brings i into [0, n)
+__device__ __forceinline__ int64_t wrap_shift(int64_t i, int n) { return i - wrap(i, n); }
+
+// i - shift as a 32-bit coordinate, saturated at +-REL_MAX
+constexpr int REL_MAX = 1 << 28;
+__device__ __forceinline__ int rel_cell(int64_t i, int64_t shift) {
+  const int64_t r = i - shift;
+  return (int)(r < -REL_MAX ? -REL_MAX : (r > REL_MAX ? REL_MAX : r));
+}
+__device__ __forceinline__ bool rel_far(int x, int y, int z) {
+  return abs(x) == REL_MAX || abs(y) == REL_MAX || abs(z) == REL_MAX;
+}
+
+__device__ __forceinline__ int wave_min_i(int v) {
+  for (int o = 32; o > 0; o >>= 1) {
+    const int w = __shfl_xor(v, o, 64);
+    v = w < v ? w : v;
+  }
+  return v;
+}
+
+// outputs of one pixel, with the FGPA when asked for
+__device__ __forceinline__ void gather_out(const GatherArgs& a, int s, int64_t pix, int64_t g, float dl, float eta,
+                                           float vpar) {
+  if (a.delta_l) a.delta_l[pix] = dl;
+  if (a.eta_par) a.eta_par[pix] = eta;
+  if (a.v_par) a.v_par[pix] = vpar;
+  if (a.flux) {
+    const int64_t row = a.sk.pset ? (int64_t)a.sk.pset[s] : g;
+    if (row < 0 || row >= a.abcg_rows) {
+      a.flux[pix] = __int_as_float(0x7fc00000);
+      if (a.status) atomicOr(&a.status[s], 2);
+    } else {
+      // F = exp(-a exp(b G (delta + c eta)))
+      const float4 prow = reinterpret_cast<const float4*>(a.abcg)[row];
+      const float gfield = dl + (a.delta_s ? a.delta_s[pix] : 0.0f) + prow.z * eta;
+      a.flux[pix] = expf(-prow.x * expf(prow.y * prow.w * gfield));
+    }
+  }
+}
+
+// LDS cells of one tube: what NT pixels of 0.2 Mpc/h span at cells of 2.19
+// Mpc/h with a line that drifts two cells over a stencil; longer spans are
+// taken in parts.  One pixel's W^3 cells always fit.
+constexpr int gg_cap(int DM, int NT) {
+  const int W = 2 * DM + 1, rows = ((W + 1) * (W + 2)) | 1;
+  return (NT / 11 + 1 + W) * rows + W;
+}
+
+// Contracted fields in LDS: G = 2 (delta, eta) or 3 (and v)
+template <int G> constexpr size_t gg_lds_bytes(int DM, int NT) {
+  return (size_t)((gg_cap(DM, NT) + 1) & ~1) * (4 + 8 * (G - 1));
+}
+
+// NF fields: 7 (delta and the six eta_ij) or 10 (those and the three
+// velocities); DM the stencil radius.  Block b takes the packed pixels
+// [b span, (b+1) span), in parts of at most NT pixels of one skewer.
+template <int NF, int DM, int NT>
+__global__ __launch_bounds__(NT)
+    __attribute__((amdgpu_waves_per_eu(DM > 4 ? 2 : (DM > 3 ? 3 : 4)))) void k_gather_radial(GatherArgs a, int span) {
+  constexpr int W = 2 * DM + 1;
+  constexpr int G = NF == 10 ? 3 : 2;
+  constexpr int CAP = gg_cap(DM, NT), CAP2 = (CAP + 1) & ~1;
+  static_assert(W * (W * W | 1) + W <= CAP, "one pixel must fit");
+  extern __shared__ double gg_lds[];
+  double* ge = gg_lds;
+  double* gv = gg_lds + CAP2;   // with velocities only
+  float* gd = reinterpret_cast<float*>(gg_lds + (G - 1) * CAP2);
+  // per z plane: the extents of the pixels' own cells in it, and of all the
+  // pixels whose stencils reach it (the window is these +- DM)
+  __shared__ int oxl[GG_NK], oxh[GG_NK], oyl[GG_NK], oyh[GG_NK];
+  __shared__ int xlo[GG_NK], xhi[GG_NK], ylo[GG_NK], pbase[GG_NK];
+  __shared__ int red[7];               // zmin, zmax, first far pixel, x and y drift, x extent
+  __shared__ int64_t shift0[3];
+  __shared__ Los l;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const smk_skewers& sk = a.sk;
+  const smk_box_view& b = a.box;
+  const int nx = b.nx, ny = b.ny, nz = b.nz;
+  const bool periodic = b.periodic;
+  const int x0 = b.nxs > 0 ? b.x0 : 0, x1 = x0 + (b.nxs > 0 ? b.nxs : nx);
+  const int64_t pix0 = (int64_t)xcd_tile(blockIdx.x, gridDim.x) * span;
+  const int64_t pend = pix0 + span < a.npix_total ? pix0 + span : a.npix_total;
+  int s = 0, s_hi = sk.n - 1;
+  if (sk.blk_s0 != nullptr) {
+    const int64_t t = pix0 / SMK_GATHER_BLOCK_PIXELS;
+    const int v0 = sk.blk_s0[t], v1 = sk.blk_s0[t + 1];
+    s = v0 < 0 ? 0 : (v0 >= sk.n ? sk.n - 1 : v0);
+    s_hi = v1 < s ? s : (v1 >= sk.n ? sk.n - 1 : v1);
+  }
+  s = __builtin_amdgcn_readfirstlane(wave_find_skewer(sk.off, s, s_hi, pix0, lane));
+
+  for (int64_t pix = pix0; pix < pend;) {
+    while (s + 1 < sk.n && sk.off[s + 1] <= pix) ++s;
+    const int64_t off = sk.off[s];
+    const int64_t send = s + 1 < sk.n && sk.off[s + 1] < pend ? sk.off[s + 1] : pend;
+    const int64_t g0 = sk.g0[s];
+    const int i0 = (int)(pix - off), i1 = (int)(send - off);
+    const int imin = sk.imin[s], imax = sk.imax[s];
+    const int f0 = imin > i0 ? imin : i0, f1 = imax < i1 ? imax : i1;
+    if (tid == 0) {
+      const double qx = sk.qx[s], qy = sk.qy[s], qz = sk.qz[s], qr = sk.qr[s];
+      l.inv_d = 1.0 / b.cell;
+      l.qx = qx;
+      l.qy = qy;
+      l.qz = qz;
+      l.qr = qr;
+      l.cx = qx / qr;
+      l.cy = qy / qr;
+      l.cz = qz / qr;
+      const double q2 = qx * qx + qy * qy + qz * qz, r = sqrt(q2);
+      l.nn[0] = qx * qx / q2;
+      l.nn[1] = qy * qy / q2;
+      l.nn[2] = qz * qz / q2;
+      l.nn[3] = 2.0 * qx * qy / q2;
+      l.nn[4] = 2.0 * qx * qz / q2;
+      l.nn[5] = 2.0 * qy * qz / q2;
+      l.nv[0] = qx / r;
+      l.nv[1] = qy / r;
+      l.nv[2] = qz / r;
+    }
+    __syncthreads();
+    for (int i = i0 + tid; i < i1; i += NT) {
+      if (i >= f0 && i < f1) continue;
+      if (a.cells) {
+        const LosPixel q = los_pixel(a, l, g0 + i);
+        a.cells[3 * (off + i) + 0] = (int32_t)q.ix;
+        a.cells[3 * (off + i) + 1] = (int32_t)q.iy;
+        a.cells[3 * (off + i) + 2] = (int32_t)q.iz;
+      }
+      gather_out(a, s, off + i, g0 + i, -1000000.0f, 0.0f, 0.0f);
+    }
+    for (int f = f0; f < f1;) {
+      const int n = f1 - f < NT ? f1 - f : NT;
+      // ---- the thread's pixel and its cell
+      const LosPixel q = los_pixel(a, l, g0 + f + (tid < n ? tid : 0));
+      int64_t sx = 0, sy = 0, sz = 0;
+      if (periodic) {
+        if (tid == 0) {
+          shift0[0] = wrap_shift(q.ix, nx);
+          shift0[1] = wrap_shift(q.iy, ny);
+          shift0[2] = wrap_shift(q.iz, nz);
+        }
+        __syncthreads();
+        sx = shift0[0];
+        sy = shift0[1];
+        sz = shift0[2];
+      }
+      const int cx = rel_cell(q.ix, sx), cy = rel_cell(q.iy, sy), cz = rel_cell(q.iz, sz);
+      bool outside = false, off_slab = false;
+      if (!periodic) {
+        // (a saturated coordinate is outside any box)
+        outside = cx < DM || cx + DM >= nx || cy < DM || cy + DM >= ny || cz < DM || cz + DM >= nz;
+      }
+      if (x0 > 0 || x1 < nx) {
+        for (int d = -DM; d <= DM; ++d) {
+          const int64_t jx = periodic ? (int64_t)wrap(cx + d + sx, nx) : cx + d;
+          off_slab = off_slab || (jx >= 0 && jx < nx && (jx < x0 || jx >= x1));
+        }
+      }
+      const bool good = tid < n && !outside && !off_slab;
+      if (tid == 0) red[2] = NT;
+      // ---- the tube: as many pixels as fit (one always does)
+      int nl = n, kmin = 0, nk = 0, WX = W, WY = W;
+      for (;;) {
+        if (tid == 0) {
+          red[0] = 0x7fffffff;
+          red[1] = -0x7fffffff;
+          red[3] = red[4] = 0;
+          red[5] = 0x7fffffff;
+          red[6] = -0x7fffffff;
+        }
+        for (int k = tid; k < GG_NK; k += NT) {
+          oxl[k] = oyl[k] = 0x7fffffff;
+          oxh[k] = oyh[k] = -0x7fffffff;
+        }
+        __syncthreads();
+        // (a pixel too far from the first one for its coordinate starts the next tube)
+        if (tid > 0 && tid < nl && rel_far(cx, cy, cz)) atomicMin(&red[2], tid);
+        if (periodic) __syncthreads();
+        nl = nl < red[2] || !periodic ? nl : red[2];
+        const bool use = good && tid < nl;
+        {
+          const int zl = wave_min_i(use ? cz : 0x7fffffff), zh = -wave_min_i(use ? -cz : 0x7fffffff);
+          if (lane == 0 && zl != 0x7fffffff) {
+            atomicMin(&red[0], zl);
+            atomicMax(&red[1], zh);
+          }
+        }
+        __syncthreads();
+        kmin = red[0];
+        nk = 0;
+        if (kmin == 0x7fffffff) break;   // none of them is in the box
+        nk = red[1] - kmin + W;
+        bool fits = false;
+        if (nk <= GG_NK) {
+          // of a run of pixels in one cell, the first one counts
+          const int px = __shfl_up(cx, 1, 64), py = __shfl_up(cy, 1, 64), pz = __shfl_up(cz, 1, 64);
+          const int pu = __shfl_up((int)use, 1, 64);
+          if (use && (lane == 0 || !pu || cx != px || cy != py || cz != pz)) {
+            const int k = cz - kmin;
+            atomicMin(&oxl[k], cx);
+            atomicMax(&oxh[k], cx);
+            atomicMin(&oyl[k], cy);
+            atomicMax(&oyh[k], cy);
+          }
+          __syncthreads();
+          for (int k = tid; k < nk; k += NT) {
+            int xl = 0x7fffffff, xh = -0x7fffffff, yl = 0x7fffffff, yh = -0x7fffffff;
+#pragma unroll
+            for (int c = 0; c < W; ++c) {
+              const int j = k - c;
+              if (j >= 0) {
+                xl = min(xl, oxl[j]);
+                xh = max(xh, oxh[j]);
+                yl = min(yl, oyl[j]);
+                yh = max(yh, oyh[j]);
+              }
+            }
+            xlo[k] = xl;
+            xhi[k] = xh;
+            ylo[k] = yl;
+            if (xl <= xh) {
+              atomicMax(&red[3], xh - xl);
+              atomicMax(&red[4], yh - yl);
+              atomicMin(&red[5], xl);
+              atomicMax(&red[6], xh);
+            }
+          }
+          __syncthreads();
+          WX = W + red[3];
+          WY = W + red[4];
+          fits = WY <= 128 && (int64_t)nk * (((int64_t)WX * WY) | 1) <= CAP;
+        }
+        if (fits) break;
+        nl = (nl + 1) / 2;
+        __syncthreads();
+      }
+      const int rows = WX * WY;
+      const int ps = rows | 1;   // plane stride, odd: planes start in different LDS banks
+      if (nk > 0) {
+        const int ncell = nk * rows;
+        // q / nk and r / WY as products: exact for q nk and r WY below 2^20
+        const uint32_t mk = (1u << 20) / (uint32_t)nk + 1, my = (1u << 20) / (uint32_t)WY + 1;
+        // Strict box: a good pixel's stencil is resident, so the tube's cells
+        // are read at 32-bit offsets from its first x plane; what a window
+        // holds beyond the resident array (never needed) reads its last cell.
+        const int64_t pz = (int64_t)ny * nz;
+        const int xmin = periodic ? 0 : red[5] - DM - x0;
+        const bool narrow = !periodic && (int64_t)(red[6] - red[5] + WX + 1) * pz < 0x3fffffff;
+        if (narrow) {
+          for (int k = tid; k < nk; k += NT)
+            pbase[k] = xlo[k] <= xhi[k]
+                           ? (int)((int64_t)(xlo[k] - DM - x0 - xmin) * pz + (int64_t)(ylo[k] - DM) * nz + kmin - DM + k)
+                           : 0;
+          __syncthreads();
+        }
+        const int64_t base0 = (int64_t)xmin * pz;
+        const int64_t left = (int64_t)(x1 - x0 - xmin) * pz - 1;
+        const uint32_t last = (uint32_t)(left < 0x3fffffff ? left : 0x3fffffff);
+        for (int q0 = tid; q0 < ncell; q0 += 2 * NT) {
+          float v[2][NF];
+          int at[2];
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const int qq = q0 + h * NT < ncell ? q0 + h * NT : q0;
+            const int r = (int)(((uint32_t)qq * mk) >> 20), k = qq - r * nk;
+            const int xo = (int)(((uint32_t)r * my) >> 20), yo = r - xo * WY;
+            at[h] = k * ps + r;
+            if (narrow) {
+              uint32_t o = (uint32_t)pbase[k] + (uint32_t)xo * (uint32_t)pz + (uint32_t)(yo * nz);
+              o = o < last ? o : last;
+              v[h][0] = (b.delta + base0)[o];
+#pragma unroll
+              for (int e = 0; e < 6; ++e) v[h][1 + e] = (b.eta[e] + base0)[o];
+              if constexpr (NF == 10) {
+#pragma unroll
+                for (int e = 0; e < 3; ++e) v[h][7 + e] = (b.vel[e] + base0)[o];
+              }
+            } else {
+              const bool have = xlo[k] <= xhi[k];
+              const int64_t jx_ = (int64_t)xlo[k] - DM + xo + sx, jy_ = (int64_t)ylo[k] - DM + yo + sy;
+              const int64_t jz_ = (int64_t)kmin - DM + k + sz;
+              const int64_t jx = periodic && have ? wrap(jx_, nx) : jx_, jy = periodic && have ? wrap(jy_, ny) : jy_;
+              const int64_t jz = periodic ? wrap(jz_, nz) : jz_;
+              // cells no good pixel needs (off the box or the slab) read cell 0
+              const bool ok = have && jx >= x0 && jx < x1 && jy >= 0 && jy < ny && jz >= 0 && jz < nz;
+              const int64_t o = ok ? ((jx - x0) * ny + jy) * nz + jz : 0;
+              v[h][0] = b.delta[o];
+#pragma unroll
+              for (int e = 0; e < 6; ++e) v[h][1 + e] = b.eta[e][o];
+              if constexpr (NF == 10) {
+#pragma unroll
+                for (int e = 0; e < 3; ++e) v[h][7 + e] = b.vel[e][o];
+              }
+            }
+          }
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            if (q0 + h * NT < ncell) {
+              gd[at[h]] = v[h][0];
+              double e = 0.0;
+#pragma unroll
+              for (int c = 0; c < 6; ++c) e += l.nn[c] * (double)v[h][1 + c];
+              ge[at[h]] = e;
+              if constexpr (NF == 10)
+                gv[at[h]] = l.nv[0] * (double)v[h][7] + l.nv[1] * (double)v[h][8] + l.nv[2] * (double)v[h][9];
+            }
+          }
+        }
+      }
+      // ---- the pixel's sums
+      double acc[G], wsum = 1.0;
+#pragma unroll
+      for (int c = 0; c < G; ++c) acc[c] = 0.0;
+      double wy[W], wz[W], wx = 1.0, ex = 1.0;
+      {
+        const double u[3] = {(double)q.ix + 0.5 - q.tx, (double)q.iy + 0.5 - q.ty, (double)q.iz + 0.5 - q.tz};
+#pragma unroll
+        for (int ax = 0; ax < 3; ++ax) {
+          const double e = exp(-u[ax]), ei = 1.0 / e;
+          double up = 1.0, dn = 1.0, t = 1.0;
+          if (ax == 1) wy[DM] = 1.0;
+          if (ax == 2) wz[DM] = 1.0;
+#pragma unroll
+          for (int d = 1; d <= DM; ++d) {
+            up *= e;
+            dn *= ei;
+            const double wu = up * GG_E[d], wd = dn * GG_E[d];
+            t += wu + wd;
+            if (ax == 1) { wy[DM + d] = wu; wy[DM - d] = wd; }
+            if (ax == 2) { wz[DM + d] = wu; wz[DM - d] = wd; }
+          }
+          wsum *= t;
+          if (ax == 0) {
+            ex = e;
+            wx = dn;   // exp(u DM): the first plane's factor, times e per plane
+          }
+        }
+      }
+      __syncthreads();
+      const bool mine = tid < nl;
+      if (nk > 0 && mine) {
+        int base[W];
+#pragma unroll
+        for (int c = 0; c < W; ++c) {
+          const int k = good ? cz - kmin + c : 0;
+          base[c] = good ? k * ps + (cx - xlo[k]) * WY + (cy - ylo[k]) : 0;
+        }
+#pragma unroll 1
+        for (int ia = 0; ia < W; ++ia) {
+          double sm[G];
+#pragma unroll
+          for (int c = 0; c < W; ++c) {
+            double row[G];
+#pragma unroll
+            for (int ib = 0; ib < W; ++ib) {
+              double v[G];
+              v[0] = (double)gd[base[c] + ib];
+              v[1] = ge[base[c] + ib];
+              if constexpr (G > 2) v[2] = gv[base[c] + ib];
+#pragma unroll
+              for (int p = 0; p < G; ++p) row[p] = ib == 0 ? wy[0] * v[p] : fma(wy[ib], v[p], row[p]);
+            }
+#pragma unroll
+            for (int p = 0; p < G; ++p) sm[p] = c == 0 ? wz[0] * row[p] : fma(wz[c], row[p], sm[p]);
+            base[c] += WY;
+          }
+          const double w = wx * GG_E[ia < DM ? DM - ia : ia - DM];
+          wx *= ex;
+#pragma unroll
+          for (int p = 0; p < G; ++p) acc[p] = fma(w, sm[p], acc[p]);
+        }
+      }
+      if (mine) {
+        const int64_t pw = off + f + tid;
+        if (a.cells) {
+          a.cells[3 * pw + 0] = (int32_t)q.ix;
+          a.cells[3 * pw + 1] = (int32_t)q.iy;
+          a.cells[3 * pw + 2] = (int32_t)q.iz;
+        }
+        float dl = __int_as_float(0x7fc00000), eta = dl, vpar = dl;
+        if (good) {
+          const double inv = 1.0 / wsum;
+          dl = (float)(acc[0] * inv);
+          // the projections are undefined at the observer (R = 0)
+          const double o = q.R == 0.0 ? __longlong_as_double(0x7ff8000000000000ll) : inv;
+          eta = (float)(acc[1] * o);
+          vpar = 0.0f;
+          if constexpr (G > 2) vpar = (float)(acc[2] * ((q.R < 0.0) != (l.qr < 0.0) ? -o : o));
+        } else if (a.status) {
+          atomicOr(&a.status[s], (outside ? 1 : 0) | (off_slab ? 4 : 0));
+        }
+        gather_out(a, s, pw, g0 + f + tid, dl, eta, vpar);
+      }
+      f += nl;
+      __syncthreads();
+    }
+    pix = send;
+    __syncthreads();
   }
 }
 
@@ -1043,17 +1540,44 @@ static int gauss_radius(int interp) {
   return r >= 0 && r <= SMK_GAUSS_DMAX ? r : -1;
 }
 
+template <int NF, int DM, int NT>
+static void launch_radial_nt(hipStream_t st, const GatherArgs& a) {
+  constexpr int G = NF == 10 ? 3 : 2;
+  int span = 2048;
+  while (span > SMK_GATHER_BLOCK_PIXELS && a.npix_total / span < 8192) span /= 2;
+  hipLaunchKernelGGL((k_gather_radial<NF, DM, NT>), dim3((uint32_t)((a.npix_total + span - 1) / span)), dim3(NT),
+                     gg_lds_bytes<G>(DM, NT), st, a, span);
+}
+
+// k_gather_radial or k_gather.  One field fits k_gather's L1 (761 us against
+// 661 for 2000 skewers at dmax 3, but 34 against 45 for 30), and so does one
+// cell per pixel (dmax 0).  A block of k_gather_radial does one skewer at a
+// time, so short skewers leave it idle: with seven fields and 2e6 pixels in
+// all, dmax 1 takes 488 us against 685 at 50 pixels per skewer and 1005
+// against 790 at 20; dmax 2 13.0 ms against 15.9 and dmax 3 21.5 against 44.1
+// at 2.
+template <int NF, int DM>
+static void launch_gather_dm(hipStream_t st, const GatherArgs& a) {
+  if constexpr (NF >= 7 && DM >= 1) {
+    if (a.npix_total >= (DM == 1 ? 40 : 2) * (int64_t)a.sk.n) {
+      launch_radial_nt<NF, DM, 256>(st, a);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((k_gather<NF, DM>), dim3((uint32_t)((a.npix_total + 255) / 256)), dim3(256), 0, st, a);
+}
+
 template <int NF>
-static void launch_gather(int r, dim3 grid, hipStream_t st, const GatherArgs& a) {
+static void launch_gather(int r, hipStream_t st, const GatherArgs& a) {
   switch (r) {
-    case -1: hipLaunchKernelGGL((k_gather<NF, -1>), grid, dim3(256), 0, st, a); break;
-    case 0: hipLaunchKernelGGL((k_gather<NF, 0>), grid, dim3(256), 0, st, a); break;
-    case 1: hipLaunchKernelGGL((k_gather<NF, 1>), grid, dim3(256), 0, st, a); break;
-    case 2: hipLaunchKernelGGL((k_gather<NF, 2>), grid, dim3(256), 0, st, a); break;
-    case 4: hipLaunchKernelGGL((k_gather<NF, 4>), grid, dim3(256), 0, st, a); break;
-    case 5: hipLaunchKernelGGL((k_gather<NF, 5>), grid, dim3(256), 0, st, a); break;
-    case 6: hipLaunchKernelGGL((k_gather<NF, 6>), grid, dim3(256), 0, st, a); break;
-    default: hipLaunchKernelGGL((k_gather<NF, 3>), grid, dim3(256), 0, st, a); break;
+    case -1: launch_gather_dm<NF, -1>(st, a); break;
+    case 0: launch_gather_dm<NF, 0>(st, a); break;
+    case 1: launch_gather_dm<NF, 1>(st, a); break;
+    case 2: launch_gather_dm<NF, 2>(st, a); break;
+    case 4: launch_gather_dm<NF, 4>(st, a); break;
+    case 5: launch_gather_dm<NF, 5>(st, a); break;
+    case 6: launch_gather_dm<NF, 6>(st, a); break;
+    default: launch_gather_dm<NF, 3>(st, a); break;
   }
 }
 
@@ -1102,15 +1626,13 @@ extern "C" int smk_forest_gather(const smk_skewers* sk, const smk_box_view* box,
     const uint64_t nblk = (uint64_t)(a.npix_total + 256 * PPT - 1) / (256 * PPT);
     hipLaunchKernelGGL(k_gather_plane_tri<PPT>, dim3((uint32_t)nblk), dim3(256), 0, (hipStream_t)stream, a);
   } else {
-    const uint64_t nblk = (uint64_t)(a.npix_total + 255) / 256;
     const bool radial = sk->geometry == SMK_GEOM_RADIAL;
     const int nf = box->eta[2] == nullptr ? 1 : (radial ? (v_par ? 10 : 7) : 2);
     const int r = interp == SMK_INTERP_TRILINEAR ? -1 : gauss_radius(interp);
-    const dim3 grid((uint32_t)nblk);
-    if (nf == 1) launch_gather<1>(r, grid, (hipStream_t)stream, a);
-    else if (nf == 2) launch_gather<2>(r, grid, (hipStream_t)stream, a);
-    else if (nf == 10) launch_gather<10>(r, grid, (hipStream_t)stream, a);
-    else launch_gather<7>(r, grid, (hipStream_t)stream, a);
+    if (nf == 1) launch_gather<1>(r, (hipStream_t)stream, a);
+    else if (nf == 2) launch_gather<2>(r, (hipStream_t)stream, a);
+    else if (nf == 10) launch_gather<10>(r, (hipStream_t)stream, a);
+    else launch_gather<7>(r, (hipStream_t)stream, a);
   }
   SMK_LAUNCH_CHECK();
   return SMK_OK;
