@@ -37,12 +37,31 @@ using namespace smk_box;
 
 namespace {
 
-__global__ void k_reduce_partials(const double* __restrict__ partial, uint64_t n, double* __restrict__ out) {
+// Status slots of the C2R passes (see k_z_c2r): SLOTS words per field, in the
+// buffer of the partial sums once these are added up.
+constexpr int SLOTS = 32;
+constexpr size_t SLOT_BYTES = (size_t)2 * SLOTS * STATUS_STRIDE * sizeof(int);
+
+// the sum of the partials (fixed order); then, with `slots`, the status slots
+// that take their place, cleared
+__global__ void k_reduce_partials(const double* partial, uint64_t n, double* __restrict__ out, int* slots) {
   __shared__ double red[16];
   double s = 0.0;
   for (uint64_t i = threadIdx.x; i < n; i += blockDim.x) s += partial[i];
   const double tot = block_sum<1024>(s, red);
   if (threadIdx.x == 0) *out = tot;
+  if (slots != nullptr && threadIdx.x < 2 * SLOTS) slots[threadIdx.x * STATUS_STRIDE] = 0;
+}
+
+// status[f] = the OR of field f's slots (block of 64 threads)
+__global__ void k_merge_status(const int* __restrict__ slots, int nfields, int* __restrict__ status) {
+  static_assert(2 * SLOTS == 64, "a wave holds the slots of both fields");
+  const int v = slots[threadIdx.x * STATUS_STRIDE];
+  const uint64_t nan = __ballot(v & 1), nz = __ballot(v & 2);
+  if ((int)threadIdx.x < nfields) {
+    const int sh = (int)threadIdx.x * SLOTS;
+    status[threadIdx.x] = (((nan >> sh) & 0xffffffffu) ? 1 : 0) | (((nz >> sh) & 0xffffffffu) ? 2 : 0);
+  }
 }
 
 __global__ void k_clear_ints(int* p, int n) {
@@ -88,10 +107,10 @@ hipError_t launch_z_r2c(int m, int vid, const float* noise, uint64_t seed, float
 }
 
 hipError_t launch_z_c2r(int m, int vid, const float2* K, float* out, const float2* tw, const float2* twr,
-                        uint64_t np, float scale, int* status, hipStream_t s) {
+                        uint64_t np, float scale, int* status, int slot_mask, hipStream_t s) {
   switch (m) {
 #define SMK_CASE(N) \
-  case N: return launch_len_c2r<N>(vid, K, out, tw, twr, np, scale, status, s);
+  case N: return launch_len_c2r<N>(vid, K, out, tw, twr, np, scale, status, slot_mask, s);
     SMK_FFT_LENGTHS(SMK_CASE)
 #undef SMK_CASE
     default: return hipErrorInvalidValue;
@@ -183,6 +202,11 @@ extern "C" int smk_box_plan_create(smk_box_plan** plan, int nx, int ny, int nz, 
   smk_box_plan* p = (smk_box_plan*)calloc(1, sizeof(smk_box_plan));
   SMK_REQUIRE(p != nullptr, SMK_ERR_OOM, "host allocation failed");
   p->nx = nx; p->ny = ny; p->nz = nz; p->m = nz / 2; p->nzh = nz / 2 + 1; p->cell = cell;
+  for (int k = 0; k < SMK_PASS_COUNT; ++k) {
+    p->vid[k] = k == SMK_PASS_Z_R2C   ? default_pencil(p->m, false)
+                : k == SMK_PASS_Z_C2R ? default_pencil(p->m, true)
+                                      : default_strided(k == SMK_PASS_Y_FWD || k == SMK_PASS_Y_INV ? ny : nx, k);
+  }
   p->n_partial = strided_blocks_max(nx, MODE_SPECTRAL, (uint64_t)p->nzh, (uint32_t)ny);
 
   auto upload = [](void** dst, const void* src, size_t bytes) -> hipError_t {
@@ -483,10 +507,17 @@ extern "C" int smk_grf_box(smk_box_plan* p, uint64_t seed, const float* noise, c
   int rc = harvest_timing(p);
   if (rc) return rc;
 
-  if (status_out) {
+  // status through slots where the partials' buffer holds them (sequential
+  // schedule: the sum that frees the buffer is before the C2R passes)
+  int* slots = status_out && var_out && p->nslab < 2 && p->n_partial * sizeof(double) >= SLOT_BYTES ? (int*)partial
+                                                                                                    : nullptr;
+  if (status_out && !slots) {
     hipLaunchKernelGGL(k_clear_ints, dim3(1), dim3(64), 0, s, status_out, 2);
     SMK_LAUNCH_CHECK();
   }
+  int* const st0 = slots ? slots : status_out;
+  int* const st1 = slots ? slots + SLOTS * STATUS_STRIDE : (status_out ? status_out + 1 : nullptr);
+  const int smask = slots ? SLOTS - 1 : 0;
   const uint64_t nb_spec = strided_blocks(p->nx, MODE_SPECTRAL, vx, (uint64_t)p->nzh, (uint32_t)p->ny);
 
   if (p->nslab < 2) {
@@ -500,23 +531,26 @@ extern "C" int smk_grf_box(smk_box_plan* p, uint64_t seed, const float* noise, c
     const StridedArgs a = spectral_args(p, A2, A1, has_aux ? A3 : nullptr, pk_params, aux_kind, aux_coef, partial, 0);
     SMK_HIP_RET(timed(p, 2, s, [&] { return launch_strided<MODE_SPECTRAL>(p->nx, vx, a, (uint64_t)p->nzh, s); }));
     if (var_out) {
-      hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(1024), 0, s, partial, nb_spec, var_out);
+      hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(1024), 0, s, partial, nb_spec, var_out, slots);
       SMK_LAUNCH_CHECK();
     }
     SMK_HIP_RET(timed(p, 3, s, [&] {
       return launch_strided<MODE_INV>(p->ny, vyi, tr_y_inv_args(p, A1, A2), (uint64_t)p->nx, s);
     }));
     SMK_HIP_RET(timed(p, 4, s, [&] {
-      return launch_z_c2r(p->m, vz, A2, delta_out, p->tw_z, p->tw_r, np, 1.0f, status_out, s);
+      return launch_z_c2r(p->m, vz, A2, delta_out, p->tw_z, p->tw_r, np, 1.0f, st0, smask, s);
     }));
     if (has_aux) {
       SMK_HIP_RET(timed(p, 5, s, [&] {
         return launch_strided<MODE_INV>(p->ny, vyi, tr_y_inv_args(p, A3, A1), (uint64_t)p->nx, s);
       }));
       SMK_HIP_RET(timed(p, 6, s, [&] {
-        return launch_z_c2r(p->m, vz, A1, aux_out, p->tw_z, p->tw_r, np, 1.0f, status_out ? status_out + 1 : nullptr,
-                            s);
+        return launch_z_c2r(p->m, vz, A1, aux_out, p->tw_z, p->tw_r, np, 1.0f, st1, smask, s);
       }));
+    }
+    if (slots) {
+      hipLaunchKernelGGL(k_merge_status, dim3(1), dim3(64), 0, s, slots, 2, status_out);
+      SMK_LAUNCH_CHECK();
     }
   } else {
     // ---- slab schedule.  Stage A (x slabs): z R2C on stream 1 feeding the
@@ -565,12 +599,12 @@ extern "C" int smk_grf_box(smk_box_plan* p, uint64_t seed, const float* noise, c
       }));
     }
     if (var_out) {
-      hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(1024), 0, s1, partial, nb_spec, var_out);
+      hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(1024), 0, s1, partial, nb_spec, var_out, (int*)nullptr);
       SMK_LAUNCH_CHECK();
     }
     hipEvent_t b_done = rec(s1);
     SMK_HIP_RET(timed(p, 4, s2, [&] {
-      return launch_z_c2r(p->m, vz, A4, delta_out, p->tw_z, p->tw_r, np, 1.0f, status_out, s2);
+      return launch_z_c2r(p->m, vz, A4, delta_out, p->tw_z, p->tw_r, np, 1.0f, st0, 0, s2);
     }));
     SMK_HIP_RET(hipStreamWaitEvent(s, b_done, 0));
     if (has_aux) {
@@ -578,8 +612,7 @@ extern "C" int smk_grf_box(smk_box_plan* p, uint64_t seed, const float* noise, c
         return launch_strided<MODE_INV>(p->ny, vyi, tr_y_inv_args(p, A3, A2), (uint64_t)p->nx, s);
       }));
       SMK_HIP_RET(timed(p, 6, s, [&] {
-        return launch_z_c2r(p->m, vz, A2, aux_out, p->tw_z, p->tw_r, np, 1.0f, status_out ? status_out + 1 : nullptr,
-                            s);
+        return launch_z_c2r(p->m, vz, A2, aux_out, p->tw_z, p->tw_r, np, 1.0f, st1, 0, s);
       }));
     }
     // join: the caller's stream waits for stream 2 (stream 1 is already joined
@@ -721,7 +754,8 @@ extern "C" int smk_fft_and_store(smk_box_plan* p, float* boxk_inout, float* box_
   hipStream_t s = (hipStream_t)stream;
   float2* K = (float2*)boxk_inout;
   const uint64_t np = (uint64_t)p->nx * p->ny;
-  if (status_out) {
+  int* slots = status_out && sumsq_out && smk_fft_and_store_workspace_bytes(p) >= SLOT_BYTES ? (int*)workspace : nullptr;
+  if (status_out && !slots) {
     hipLaunchKernelGGL(k_clear_ints, dim3(1), dim3(64), 0, s, status_out, 1);
     SMK_LAUNCH_CHECK();
   }
@@ -732,12 +766,17 @@ extern "C" int smk_fft_and_store(smk_box_plan* p, float* boxk_inout, float* box_
   SMK_HIP_RET(launch_strided<MODE_INV>(p->nx, vx, a, (uint64_t)p->ny, s));
   if (sumsq_out) {
     const uint64_t nb = strided_blocks(p->nx, MODE_INV, vx, (uint64_t)p->ny, (uint32_t)p->nzh);
-    hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(1024), 0, s, a.partial, nb, sumsq_out);
+    hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(1024), 0, s, a.partial, nb, sumsq_out, slots);
     SMK_LAUNCH_CHECK();
   }
   const float scale = (float)(1.0 / ((double)p->nx * p->ny * p->nz));
   SMK_HIP_RET(launch_strided<MODE_INV>(p->ny, p->vid[SMK_PASS_Y_INV], nat_y_args(p, K), (uint64_t)p->nx, s));
-  SMK_HIP_RET(launch_z_c2r(p->m, p->vid[SMK_PASS_Z_C2R], K, box_out, p->tw_z, p->tw_r, np, scale, status_out, s));
+  SMK_HIP_RET(launch_z_c2r(p->m, p->vid[SMK_PASS_Z_C2R], K, box_out, p->tw_z, p->tw_r, np, scale,
+                           slots ? slots : status_out, slots ? SLOTS - 1 : 0, s));
+  if (slots) {
+    hipLaunchKernelGGL(k_merge_status, dim3(1), dim3(64), 0, s, slots, 1, status_out);
+    SMK_LAUNCH_CHECK();
+  }
   return SMK_OK;
 }
 

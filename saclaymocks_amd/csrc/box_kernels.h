@@ -579,6 +579,8 @@ __device__ __forceinline__ float2 c2r_fold(float2 xk, float2 xc, int k, const fl
   return make_float2(sm.x - wd.y, sm.y + wd.x);  // sm + i*wd
 }
 
+constexpr int STATUS_STRIDE = 16;   // ints between two status slots: a 64 B line each
+
 // z pencils, C2R (unnormalised, times `scale`): the inverse M-point FFT of
 // Z' (c2r_fold) is x_{2n} + i x_{2n+1}.  XCH 0 exchanges float2 values
 // through LDS; XCH 1 the real, then the imaginary parts through a float line
@@ -587,7 +589,8 @@ __device__ __forceinline__ float2 c2r_fold(float2 xk, float2 xc, int k, const fl
 template <int M, int E, int T, int XCH>
 __global__ __launch_bounds__(T*(M / E)) void k_z_c2r(const float2* __restrict__ K, float* __restrict__ out,
                                                      const float2* __restrict__ tw, const float2* __restrict__ twr,
-                                                     uint64_t n_pencils, float scale, int* __restrict__ status) {
+                                                     uint64_t n_pencils, float scale, int* __restrict__ status,
+                                                     int slot_mask) {
   constexpr int P = M / E;
   constexpr int LL = lds_line_len(M);
   __shared__ float2 xnyq[T];
@@ -657,7 +660,10 @@ __global__ __launch_bounds__(T*(M / E)) void k_z_c2r(const float2* __restrict__ 
   const int any_nz = __syncthreads_or(flags & 2);
   if (tid == 0 && status != nullptr) {
     const int f = (any_nan ? 1 : 0) | (any_nz ? 2 : 0);
-    if (f) atomicOr(status, f);
+    // slot_mask > 0: the flags go to one of slot_mask + 1 words, a cache line
+    // each (atomics of all blocks on one word take 8 ns each: 59 us of a 256^3
+    // pass that takes 27 without them)
+    if (f) atomicOr(status + (blockIdx.x & (uint32_t)slot_mask) * STATUS_STRIDE, f);
   }
 }
 
@@ -687,9 +693,9 @@ constexpr bool dif_ok(int n, int e) {
   return false;
 }
 
-constexpr int lines_per_block(int n, int e, int xch, int max_threads) {
+constexpr int lines_per_block(int n, int e, int xch, int max_threads, int max_lines = 8) {
   const int bytes = lds_line_len(n) * (xch ? 4 : 8);
-  int T = 8;
+  int T = max_lines;
   while (T > 1 && (T * (n / e) > max_threads || T * bytes > 81920)) T >>= 1;
   return T;
 }
@@ -700,8 +706,9 @@ constexpr int half_tile(int n) {
   return (e0 % 2 == 0 && plan_ok(n, e0 / 2) && n / (e0 / 2) <= 512) ? e0 / 2 : 0;
 }
 
-// Variants (n >= 512; "swz" ones only for the unpadded 2560-point line,
-// whose LDS exchange needs a swizzle; the stash ones only in spectral mode):
+// Variants (n >= 512; "swz" ones only for the unpadded 1280- and 2560-point
+// lines, whose LDS exchange needs a swizzle; the stash ones only in spectral
+// mode):
 //   0  E0, float2 exchange            5  E0, split exchange, SWS 3 (swz)
 //   1  E0, float2, SWS 2 (swz)        6  E1, float2, SWS 2 (swz) / SWS 0
 //   2  E0, float2, SWS 3 (swz)        7  E1, float2, SWS 3 (swz)
@@ -713,6 +720,8 @@ constexpr int half_tile(int n) {
 //  14  E0, k_xspec: aux in a second register tile (3 FFTs), scalar-base
 //      addressing, log2-form spectrum, SWS 2 / 0 (spectral mode only)
 //  15  as 14, registers capped for 2 waves per SIMD (spills what is left)
+//  17  E0, split exchange, 16 lines per block (128 B runs)   18  the same, E1
+//      (both also for 256 <= n < 512)
 //  16  E0, k_xspec_dif: delta's inverse FFT in place in LDS, the aux
 //      spectrum in registers (3 FFTs); lengths whose threads per line are a
 //      product of leading radices
@@ -724,7 +733,14 @@ constexpr SVar strided_variant(int n, int mode, int vid) {
   if (e0 == 0) return none;
   const int t0 = lines_per_block(n, e0, 0, 512);
   if (vid == 0) return SVar{e0, t0, 0, 1, 0, 0};
-  if (n < 512 || tuned_elems(n) == 0) return none;
+  if (n < 256 || tuned_elems(n) == 0) return none;
+  if (vid >= 17) {
+    const int e = vid == 18 ? e1 : e0;
+    if (e == 0 || vid > 18) return none;
+    const int t = lines_per_block(n, e, 1, 1024, 16);
+    return t > 8 ? SVar{e, t, 1, 1, 0, 0} : none;
+  }
+  if (n < 512) return none;
   const bool spec = mode == MODE_SPECTRAL;
   const bool swz = !lds_padded(n);
   const int ts = lines_per_block(n, e0, 1, 1024);
@@ -747,6 +763,47 @@ constexpr SVar strided_variant(int n, int mode, int vid) {
     case 15: return spec ? SVar{e0, t0, 0, 4, swz ? 2 : 0, 2} : none;
     case 16: return (spec && dif_ok(n, e0)) ? SVar{e0, t0, 0, 5, swz ? 2 : 0, 0} : none;
     default: return none;
+  }
+}
+
+// The variant a plan starts with, per pass kind and line length.  What decides
+// is the lines per block that half of a CU's LDS holds (the transposed runs are
+// 8 B per line) against the waves that the register tile leaves: the split
+// exchange buys lines, the half tile waves.  Measured per pass, in ms against
+// variant 0, at 320^3, 384^3, ... 1280 x 1280 x 512 and 2560 x 1280 x 768:
+//   y, x forward   320 18 (0.051, 0.056)  384 18 (0.114, 0.128)
+//                  512 17 (0.327, 0.362)  640 17 (0.482, 0.518)
+//                  768 17 (0.750, 0.875)  1024 3 (1.17, 1.59)
+//                  1280 6 (4.34, 4.68)    1536 3 (2.37, 3.04)
+//                  2048 3 (3.48, 4.94)
+//   y inverse      320 18 (0.147, 0.165)  384 18 (0.251, 0.273)
+//                  640 6 (1.02, 1.11)     768 18 (1.81, 2.05)
+//                  1024 3 (2.60, 2.81)    1280 6 (9.1, 10.4)
+//                  1536 6 (5.41, 5.79)    2048 3 (7.9, 11.9)
+//   x inverse      as forward; in the numpy layout 1280 17 (2.42, 2.55 the
+//                  whole inverse), 2560 4 (4.86, 5.26)
+//   x spectral     320 18 (0.153, 0.164)  384 17 (0.263, 0.288)
+//                  512 16 (0.530, 0.634)  640 10 (1.12, 1.55)
+//                  768 3 (1.85, 2.00)     1024 14 (2.57, 2.94)
+//                  1280 12 (3.53, 4.57)   1536 3 (5.95, 7.18)
+//                  2048 14 (5.68, 6.44)   2560 1 (13.2, 17.0)
+// Lengths that are not listed have variant 0 only or lose nothing by it.
+constexpr int default_strided(int n, int kind) {
+  const bool p2 = n == 1024 || n == 2048;
+  switch (kind) {
+    case SMK_PASS_X_SPECTRAL:
+      return n == 320 ? 18 : n == 384 ? 17 : n == 512 ? 16 : n == 640 ? 10 : n == 768 || n == 1536 ? 3 : p2 ? 14
+             : n == 1280 ? 12 : n == 2560 ? 1 : 0;
+    case SMK_PASS_Y_INV:
+      return n == 320 || n == 384 || n == 768 ? 18 : n == 640 || n == 1280 || n == 1536 ? 6 : p2 ? 3 : 0;
+    case SMK_PASS_X_INV:
+      if (n == 1280) return 17;
+      if (n == 2560) return 4;
+      [[fallthrough]];
+    case SMK_PASS_Y_FWD:
+    case SMK_PASS_X_FWD:
+      return n == 320 || n == 384 ? 18 : n == 512 || n == 640 || n == 768 ? 17 : n == 1280 ? 6 : p2 || n == 1536 ? 3 : 0;
+    default: return 0;
   }
 }
 
@@ -794,6 +851,8 @@ hipError_t launch_strided_n(int vid, const StridedArgs& a, uint64_t n_outer, hip
     case 14: return launch_strided_nv<N, MODE, 14>(a, n_outer, s);
     case 15: return launch_strided_nv<N, MODE, 15>(a, n_outer, s);
     case 16: return launch_strided_nv<N, MODE, 16>(a, n_outer, s);
+    case 17: return launch_strided_nv<N, MODE, 17>(a, n_outer, s);
+    case 18: return launch_strided_nv<N, MODE, 18>(a, n_outer, s);
     default: return hipErrorInvalidValue;
   }
 }
@@ -830,6 +889,13 @@ inline bool pencil_variant_ok(int m, int vid, bool c2r) {
   return vid >= 0 && vid < SMK_NPVAR && pencil_E(m, vid) != 0 && (c2r || pencil_XCH(vid) == 0);
 }
 
+// The z passes' variant a plan starts with (ms against variant 0): R2C of 320
+// complex points 0.43 against 0.65 and 384 1.94 against 2.18; C2R of 320 1.00
+// against 1.17, 384 8.7 against 8.9 and 768 32.5 against 35.4.
+constexpr int default_pencil(int m, bool c2r) {
+  return c2r ? (m == 320 ? 1 : m == 384 || m == 768 ? 2 : 0) : (m == 320 || m == 384 ? 1 : 0);
+}
+
 template <int M, int VID>
 hipError_t launch_z_r2c_v(const float* noise, uint64_t seed, float2* K, const float2* tw, const float2* twr,
                           uint64_t p0, uint64_t np, int trans, uint32_t ny, hipStream_t s) {
@@ -849,7 +915,7 @@ hipError_t launch_z_r2c_v(const float* noise, uint64_t seed, float2* K, const fl
 
 template <int M, int VID>
 hipError_t launch_z_c2r_v(const float2* K, float* out, const float2* tw, const float2* twr, uint64_t np,
-                          float scale, int* status, hipStream_t s) {
+                          float scale, int* status, int slot_mask, hipStream_t s) {
   constexpr int E = pencil_E(M, VID);
   if constexpr (E == 0) {
     return hipErrorInvalidValue;
@@ -857,7 +923,7 @@ hipError_t launch_z_c2r_v(const float2* K, float* out, const float2* tw, const f
     constexpr int T = pencil_T(M, E);
     if ((np + T - 1) / T > 0x7fffffffull) return hipErrorInvalidConfiguration;
     hipLaunchKernelGGL((k_z_c2r<M, E, T, pencil_XCH(VID)>), dim3((uint32_t)((np + T - 1) / T)), dim3(T * (M / E)), 0, s, K, out,
-                       tw, twr, np, scale, status);
+                       tw, twr, np, scale, status, slot_mask);
     return hipGetLastError();
   }
 }
@@ -886,10 +952,10 @@ hipError_t launch_len_r2c(int vid, const float* noise, uint64_t seed, float2* K,
 
 template <int M>
 hipError_t launch_len_c2r(int vid, const float2* K, float* out, const float2* tw, const float2* twr, uint64_t np,
-                          float scale, int* status, hipStream_t s) {
-  return vid == 0   ? launch_z_c2r_v<M, 0>(K, out, tw, twr, np, scale, status, s)
-         : vid == 1 ? launch_z_c2r_v<M, 1>(K, out, tw, twr, np, scale, status, s)
-         : vid == 2 ? launch_z_c2r_v<M, 2>(K, out, tw, twr, np, scale, status, s)
+                          float scale, int* status, int slot_mask, hipStream_t s) {
+  return vid == 0   ? launch_z_c2r_v<M, 0>(K, out, tw, twr, np, scale, status, slot_mask, s)
+         : vid == 1 ? launch_z_c2r_v<M, 1>(K, out, tw, twr, np, scale, status, slot_mask, s)
+         : vid == 2 ? launch_z_c2r_v<M, 2>(K, out, tw, twr, np, scale, status, slot_mask, s)
                     : hipErrorInvalidValue;
 }
 
@@ -897,7 +963,7 @@ hipError_t launch_len_c2r(int vid, const float2* K, float* out, const float2* tw
   SPEC hipError_t launch_len_strided<N>(int, int, const StridedArgs&, uint64_t, hipStream_t);                    \
   SPEC hipError_t launch_len_r2c<N>(int, const float*, uint64_t, float2*, const float2*, const float2*, uint64_t, \
                                     uint64_t, int, uint32_t, hipStream_t);                                        \
-  SPEC hipError_t launch_len_c2r<N>(int, const float2*, float*, const float2*, const float2*, uint64_t, float, int*, \
+  SPEC hipError_t launch_len_c2r<N>(int, const float2*, float*, const float2*, const float2*, uint64_t, float, int*, int, \
                                     hipStream_t);
 #define SMK_LEN_EXTERN(N) SMK_LEN_SIGNATURES(extern template, N)
 #define SMK_LEN_INSTANTIATE(N) SMK_LEN_SIGNATURES(template, N)

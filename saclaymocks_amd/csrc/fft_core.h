@@ -305,7 +305,7 @@ __host__ __device__ constexpr int elems_per_thread(int n) {
 // power-of-two strides of the early Stockham stages across banks.  The
 // 2560-point line is left unpadded so that four lines fill exactly 80 KiB and
 // two blocks share one CU's 160 KiB.
-__host__ __device__ constexpr bool lds_padded(int n) { return n != 2560; }
+__host__ __device__ constexpr bool lds_padded(int n) { return n != 2560 && n != 1280; }
 template <int N> __host__ __device__ constexpr int lds_pos(int pos) {
   return lds_padded(N) ? pos + (pos >> 5) : pos;
 }
