@@ -546,6 +546,17 @@ int smk_qso_draw(const smk_qso_params* p, const float* p1, const float* p2, cons
                  const float* vy, const float* vz, uint64_t seed, smk_qso_record* records, int64_t capacity,
                  int64_t* count, void* stream);
 
+/* The same draw (the same records) with a scratch buffer for a bit mask of
+ * the cells that a bound on the first condition does not rule out: four times
+ * faster where few cells pass it, as fast where all do.  scratch: device
+ * memory, 8-byte aligned, of at least smk_qso_scratch_bytes (0.13 bytes per
+ * cell on long columns), or NULL: smk_qso_draw.  Calls that share a scratch
+ * buffer must not overlap. */
+size_t smk_qso_scratch_bytes(const smk_qso_params* p);
+int smk_qso_draw_scratch(const smk_qso_params* p, const float* p1, const float* p2, const float* p3, const float* vx,
+                         const float* vy, const float* vz, uint64_t seed, smk_qso_record* records, int64_t capacity,
+                         int64_t* count, void* scratch, size_t scratch_bytes, void* stream);
+
 /* ------------------------------------------------------------ P(k) tables */
 /* A cubic spline as piecewise cubics: on [x[i], x[i+1]) (positive length),
  * P(k) = ((c[i][0] t + c[i][1]) t + c[i][2]) t + c[i][3], t = k - x[i];

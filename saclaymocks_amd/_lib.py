@@ -82,6 +82,8 @@ _SIGNATURES = {
     "smk_forest_step": (_i, [_vp, _vp, _vp, _vp, _c.POINTER(_c.c_int64), _c.c_int64, _c.c_int32, _vp, _vp, _u64,
                              _vp, _c.c_int64, _c.c_int32, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "smk_qso_draw": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _u64, _vp, _c.c_int64, _vp, _vp]),
+    "smk_qso_scratch_bytes": (_sz, [_vp]),
+    "smk_qso_draw_scratch": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _u64, _vp, _c.c_int64, _vp, _vp, _sz, _vp]),
     "smk_pk_table": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _c.c_float, _vp, _vp]),
     "smk_p1d_rsd_rows": (_i, [_vp, _vp, _i, _vp, _i, _d, _i, _vp, _d, _d, _vp, _vp]),
     "smk_reduce_work_len": (_c.c_int64, [_i, _i, _i]),

@@ -1,4 +1,4 @@
-// Quasar draw on gfx950: one thread per cell of the lognormal slab.
+// Quasar draw on gfx950: the cells of the lognormal slab, columns along z.
 //
 // Reference: bin/draw_qso.py:186-462.  The reference builds ptot for the
 // whole slab with numpy, then loops over the z planes drawing two uniforms
@@ -104,17 +104,13 @@ __device__ __forceinline__ double diffmod(double a, double b, double c) {
   return fmin(d, c - d);
 }
 
-__global__ __launch_bounds__(256) void k_qso_draw(smk_qso_params p, const float* __restrict__ p1,
-                                                  const float* __restrict__ p2, const float* __restrict__ p3,
-                                                  const float* __restrict__ vx, const float* __restrict__ vy,
-                                                  const float* __restrict__ vz, uint64_t seed,
-                                                  smk_qso_record* __restrict__ rec, int64_t cap,
-                                                  unsigned long long* __restrict__ count) {
-  // block (column ix * ny + iy, 256-cell chunk of z): the column's indices
-  // are block-uniform (scalar), the cell index c = column * nz + mz
-  const uint32_t col = blockIdx.x;
-  const int mz = (int)(blockIdx.y * 256 + threadIdx.x);
-  if (mz >= p.nz) return;
+// the whole draw of one cell (column ix * ny + iy, cell mz of it)
+__device__ __forceinline__ void draw_cell(const smk_qso_params& p, const float* __restrict__ p1,
+                                          const float* __restrict__ p2, const float* __restrict__ p3,
+                                          const float* __restrict__ vx, const float* __restrict__ vy,
+                                          const float* __restrict__ vz, uint64_t seed,
+                                          smk_qso_record* __restrict__ rec, int64_t cap,
+                                          unsigned long long* __restrict__ count, uint32_t col, int mz) {
   const int ix = (int)(col / (uint32_t)p.ny), iy = (int)(col % (uint32_t)p.ny);
   const uint64_t c = (uint64_t)col * (uint64_t)p.nz + (uint64_t)mz;
   const double xc = p.x_axis[ix], yc = p.y_axis[iy], zcell = p.z_axis[mz];
@@ -187,15 +183,234 @@ __global__ __launch_bounds__(256) void k_qso_draw(smk_qso_params p, const float*
   }
 }
 
+// every cell by draw_cell: block (column, 256-cell chunk of z), a thread per cell
+__global__ __launch_bounds__(256) void k_qso_draw(smk_qso_params p, const float* __restrict__ p1,
+                                                  const float* __restrict__ p2, const float* __restrict__ p3,
+                                                  const float* __restrict__ vx, const float* __restrict__ vy,
+                                                  const float* __restrict__ vz, uint64_t seed,
+                                                  smk_qso_record* __restrict__ rec, int64_t cap,
+                                                  unsigned long long* __restrict__ count) {
+  const int mz = (int)(blockIdx.y * 256 + threadIdx.x);
+  if (mz < p.nz) draw_cell(p, p1, p2, p3, vx, vy, vz, seed, rec, cap, count, blockIdx.x, mz);
+}
+
+// The draw with a mask of candidates.  Of the cells of a slice one in 10^4 to
+// 10^2 passes the first condition, rnd1 < norm ptot; the others only need a
+// bound.  Over a chunk of CHUNK cells along z the redshift, the exponents'
+// factor t = (1 + z)^0.7 and the mix of the three fields' powers lie between
+// values that one lane finds beforehand (k_qso_bounds), so a cell costs its
+// three field values, one Philox call and three hardware exponentials
+// (k_qso_filter); the cells that stay under the bound are set in a bit mask and
+// take draw_cell, which decides as before (k_qso_masked).  The bound is above
+// norm ptot by more than the float rounding of either side, so no cell that
+// draw_cell would draw is left out.
+//
+// Measured on a slice of 160 x 2560 x 1536 cells: k_qso_draw 7.7 ms, bound by
+// its FP64 lookups per cell; this way 1.67, of which the filter 1.55 (4.9 TB/s,
+// the card's copy rate) and the bounds 0.05 (0.16 with one per 8 columns; found
+// inside the filter's blocks 0.7, as a block waits for a few lanes' chains).
+// With 10 and 100 times as many cells that pass, 10.4 and 20.5 ms against 1.97
+// and 4.4; only with all of them (75 million quasars) k_qso_draw is the faster,
+// 47 against 63.  draw_cell has a kernel of its own since in the filter's loop
+// it took 216 registers (2 waves per SIMD, 9.4 ms), as a call from there 7.0.  In k_qso_masked's loop the compiler keeps its
+// constants in registers, 199 of them if it may; 128 were faster at every
+// density.  A bit per cell never overflows; a list of cells did, or was as
+// large as a field.
+constexpr int CHUNK = 128;        // cells along z of one bound: two waves
+constexpr int BCOLS = 32;         // columns of one bound
+constexpr int COLS = 16;          // columns per block of the filter
+constexpr int ZCELLS = 1024;      // z cells per block: four per thread
+constexpr int QUEUED = 1024;      // cells of a block's queue that are drawn together
+constexpr uint64_t MASK_BLOCKS = 1024;   // as many as are resident
+
+struct DrawBound {
+  float tlo, thi;                 // (1 + z)^0.7 over the chunk, log2(e) folded in
+  float g1, g2, g3;               // largest mix coefficients, times norm
+  float pad;                      // 24 bytes
+};
+
+// the bound of the cells with x^2 + y^2 in [rxy0, rxy1] and z coordinate in [lo, hi]
+__device__ __forceinline__ DrawBound draw_bounds(const smk_qso_params& p, double rxy0, double rxy1, double lo,
+                                                 double hi) {
+  DrawBound b;
+  // distance along z: 0 if the range straddles the observer's plane
+  const double near = lo > 0.0 ? lo : (hi < 0.0 ? -hi : 0.0), far = fmax(fabs(lo), fabs(hi));
+  const double z0 = z_of_r(p, sqrt(rxy0 + near * near) / p.h), z1 = z_of_r(p, sqrt(rxy1 + far * far) / p.h);
+  const float l2e = 1.4426950408889634f;
+  b.tlo = __builtin_amdgcn_exp2f(0.7f * __builtin_amdgcn_logf((float)(1.0 + z0))) * l2e * (1.0f - 2e-5f);
+  b.thi = __builtin_amdgcn_exp2f(0.7f * __builtin_amdgcn_logf((float)(1.0 + z1))) * l2e * (1.0f + 2e-5f);
+  // c(z) over [z0, z1]: its ends and the nodes between them
+  const double ca = coef_of_z(p, z0), cb = coef_of_z(p, z1);
+  double c0 = fmin(ca, cb), c1 = fmax(ca, cb);
+  int j = 1 + uniform_guess(z0, p.coef_z[1], p.coef_z[2] - p.coef_z[1]);
+  j = j > p.coef_n - 1 ? p.coef_n - 1 : j;
+  while (j > 0 && p.coef_z[j] > z0) --j;
+  for (; j < p.coef_n && p.coef_z[j] < z1; ++j) {
+    c0 = fmin(c0, p.coef_c[j]);
+    c1 = fmax(c1, p.coef_c[j]);
+  }
+  // ptot = g1 e1 + g2 e2 + g3 e3, each g bilinear in (c, z): its largest value is at a corner
+  constexpr double R12 = 1.0 / (ZB2 - ZB1), R23 = 1.0 / (ZB3 - ZB2);
+  double g1 = 0.0, g2 = 0.0, g3 = 0.0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const double z = k & 1 ? z1 : z0, c = k & 2 ? c1 : c0;
+    g1 = fmax(g1, c * (ZB2 - z) * R12);
+    g2 = fmax(g2, c * (z - ZB1) * R12 + (1.0 - c) * (ZB3 - z) * R23);
+    g3 = fmax(g3, (1.0 - c) * (z - ZB2) * R23);
+  }
+  const double up = p.norm * (1.0 + 2e-3);
+  b.g1 = (float)(up * g1);
+  b.g2 = (float)(up * g2);
+  b.g3 = (float)(up * g3);
+  return b;
+}
+
+// one lane per bound: BCOLS columns, CHUNK cells of the z axis
+__global__ __launch_bounds__(256) void k_qso_bounds(smk_qso_params p, DrawBound* __restrict__ bound, uint64_t n_bound,
+                                                    uint32_t nch, uint32_t ncol) {
+  const uint64_t q = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+  if (q >= n_bound) return;
+  const uint32_t col0 = (uint32_t)(q / nch) * BCOLS;
+  const int m0 = (int)(q % nch) * CHUNK, m1 = p.nz - m0 < CHUNK ? p.nz : m0 + CHUNK;
+  double r0 = INFINITY, r1 = 0.0, lo = INFINITY, hi = -INFINITY;
+  for (int k = 0; k < BCOLS; ++k) {
+    const uint32_t col = col0 + (uint32_t)k < ncol ? col0 + (uint32_t)k : ncol - 1;
+    const double xc = p.x_axis[col / (uint32_t)p.ny], yc = p.y_axis[col % (uint32_t)p.ny];
+    r0 = fmin(r0, xc * xc + yc * yc);
+    r1 = fmax(r1, xc * xc + yc * yc);
+  }
+#pragma unroll 8
+  for (int mz = m0; mz < m1; ++mz) {
+    lo = fmin(lo, p.z_axis[mz]);
+    hi = fmax(hi, p.z_axis[mz]);
+  }
+  bound[q] = draw_bounds(p, r0, r1, lo, hi);
+}
+
+// mask: a bit per cell, 64 cells along z to a word, nw words to a column
+__global__ __launch_bounds__(256) void k_qso_filter(int nz, int randoms, const float* __restrict__ p1,
+                                                    const float* __restrict__ p2, const float* __restrict__ p3,
+                                                    uint64_t seed, const DrawBound* __restrict__ bounds, uint32_t nch,
+                                                    uint64_t* __restrict__ mask, uint32_t nw, uint32_t ncol) {
+  static_assert(BCOLS % COLS == 0, "a block's columns share a bound");
+  static_assert(CHUNK % 64 == 0, "a wave's cells share a bound");
+  const int tid = threadIdx.x;
+  const uint32_t col0 = blockIdx.x * COLS;
+  const int m0 = (int)blockIdx.y * ZCELLS, m1 = nz - m0 < ZCELLS ? nz : m0 + ZCELLS;
+  const DrawBound* __restrict__ bound = bounds + (uint64_t)(col0 / BCOLS) * nch;
+  for (int k = 0; k < COLS && col0 + (uint32_t)k < ncol; ++k) {
+    const uint64_t c0 = (uint64_t)(col0 + (uint32_t)k) * (uint64_t)nz;
+    const uint32_t lo = (uint32_t)c0, hi = (uint32_t)(c0 >> 32);
+    // the cells of a column share the counter's high word unless it carries
+    const bool carries = lo > 0xffffffffu - (uint32_t)nz;
+    // four cells per thread, the loads of all four ahead of their arithmetic
+    float f[4][3];
+    if (!randoms) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int mz = m0 + tid + 256 * u < m1 ? m0 + tid + 256 * u : m1 - 1;
+        f[u][0] = p1[c0 + (uint64_t)mz];
+        f[u][1] = p2[c0 + (uint64_t)mz];
+        f[u][2] = p3[c0 + (uint64_t)mz];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int mz = m0 + tid + 256 * u;
+      const int word = __builtin_amdgcn_readfirstlane(mz / 64);   // the wave's
+      if (64 * word >= m1) break;
+      bool maybe = true;
+      if (randoms) {
+        const uint64_t c = c0 + (uint64_t)mz;
+        const U4 w = philox4x32_10_c4((uint32_t)c, (uint32_t)(c >> 32), TAG_CELL, 0u, seed);
+        maybe = u53(w.x, w.y) > 1.0 - RAND_QSO_NB;
+      } else if (!carries) {
+        const DrawBound b = bound[64 * word / CHUNK];
+        const U4 w = philox4x32_10_c4(lo + (uint32_t)mz, hi, TAG_CELL, 0u, seed);
+        // rnd1 from below: its leading 27 bits, rounded down
+        const float rnd = (float)(w.x >> 5) * (7.450580596923828e-9f * (1.0f - 2.4e-7f));
+        const float e1 = __builtin_amdgcn_exp2f((f[u][0] > 0.0f ? b.thi : b.tlo) * (INV1 * f[u][0]));
+        const float e2 = __builtin_amdgcn_exp2f((f[u][1] > 0.0f ? b.thi : b.tlo) * (INV2 * f[u][1]));
+        const float e3 = __builtin_amdgcn_exp2f((f[u][2] > 0.0f ? b.thi : b.tlo) * (INV3 * f[u][2]));
+        // (a NaN or an overflowing power fails the comparison: the cell is looked at)
+        maybe = !(rnd > fmaf(b.g1, e1, fmaf(b.g2, e2, b.g3 * e3)));
+      }
+      const uint64_t m = __ballot(maybe && mz < m1);
+      if ((tid & 63) == 0) mask[(uint64_t)(col0 + (uint32_t)k) * nw + (uint32_t)word] = m;
+    }
+  }
+}
+
+// draw_cell of the cells of the mask: a block takes a range of half words,
+// queues their cells in LDS and draws them together
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_qso_masked(smk_qso_params p, const float* __restrict__ p1,
+                                                    const float* __restrict__ p2, const float* __restrict__ p3,
+                                                    const float* __restrict__ vx, const float* __restrict__ vy,
+                                                    const float* __restrict__ vz, uint64_t seed,
+                                                    smk_qso_record* __restrict__ rec, int64_t cap,
+                                                    unsigned long long* __restrict__ count,
+                                                    const uint32_t* __restrict__ mask, uint32_t nhalf, uint64_t total) {
+  __shared__ uint32_t queue[QUEUED + 256 * 32];   // half word in the range and bit
+  __shared__ int nqueue;
+  const int tid = threadIdx.x;
+  if (tid == 0) nqueue = 0;
+  __syncthreads();
+  // a range holds fewer than 2^27 half words: total / gridDim.x
+  const uint64_t per = (total + gridDim.x - 1) / gridDim.x;
+  const uint64_t h0 = per * blockIdx.x, h1 = h0 + per < total ? h0 + per : total;
+  uint32_t next = h0 + (uint64_t)tid < h1 ? mask[h0 + (uint64_t)tid] : 0u;
+  for (uint64_t hb = h0; hb < h1; hb += 256) {
+    const uint64_t h = hb + (uint64_t)tid;
+    uint32_t m = next;
+    next = h + 256 < h1 ? mask[h + 256] : 0u;   // loaded a step ahead
+    if (m != 0u) {
+      int at = atomicAdd(&nqueue, __popc(m));
+      for (; m != 0u; m &= m - 1u) queue[at++] = (uint32_t)(h - h0) * 32u + (uint32_t)(__ffs((int)m) - 1);
+    }
+    __syncthreads();
+    const int n = nqueue;
+    if (n > QUEUED || hb + 256 >= h1) {
+      for (int q = tid; q < n; q += 256) {
+        const uint64_t hh = h0 + queue[q] / 32u;
+        draw_cell(p, p1, p2, p3, vx, vy, vz, seed, rec, cap, count, (uint32_t)(hh / nhalf),
+                  (int)(hh % nhalf) * 32 + (int)(queue[q] % 32u));
+      }
+      __syncthreads();
+      if (tid == 0) nqueue = 0;
+    }
+    __syncthreads();
+  }
+}
+
 __global__ void k_clear_count(unsigned long long* c) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *c = 0ull;
 }
 
 }  // namespace
 
+// the scratch buffer: the bounds, then the mask
+static uint64_t qso_bounds(const smk_qso_params& p) {
+  const uint64_t ncol = (uint64_t)p.nx * (uint64_t)p.ny;
+  return (ncol + BCOLS - 1) / BCOLS * (((uint64_t)p.nz + CHUNK - 1) / CHUNK);
+}
+
+extern "C" size_t smk_qso_scratch_bytes(const smk_qso_params* p) {
+  if (p == nullptr || p->nx <= 0 || p->ny <= 0 || p->nz <= 0) return 0;
+  return (size_t)(qso_bounds(*p) * sizeof(DrawBound) +
+                  (uint64_t)p->nx * (uint64_t)p->ny * (((uint64_t)p->nz + 63) / 64) * sizeof(uint64_t));
+}
+
 extern "C" int smk_qso_draw(const smk_qso_params* p, const float* p1, const float* p2, const float* p3,
                             const float* vx, const float* vy, const float* vz, uint64_t seed,
                             smk_qso_record* records, int64_t capacity, int64_t* count, void* stream) {
+  return smk_qso_draw_scratch(p, p1, p2, p3, vx, vy, vz, seed, records, capacity, count, nullptr, 0, stream);
+}
+
+extern "C" int smk_qso_draw_scratch(const smk_qso_params* p, const float* p1, const float* p2, const float* p3,
+                                    const float* vx, const float* vy, const float* vz, uint64_t seed,
+                                    smk_qso_record* records, int64_t capacity, int64_t* count, void* scratch,
+                                    size_t scratch_bytes, void* stream) {
   SMK_REQUIRE(p != nullptr && count != nullptr, SMK_ERR_ARG, "NULL argument");
   SMK_REQUIRE(p->nx > 0 && p->ny > 0 && p->nz > 0, SMK_ERR_ARG, "empty slab");
   SMK_REQUIRE(p->randoms || (p1 != nullptr && p2 != nullptr && p3 != nullptr), SMK_ERR_ARG,
@@ -209,15 +424,38 @@ extern "C" int smk_qso_draw(const smk_qso_params* p, const float* p1, const floa
   SMK_REQUIRE(p->r2z_n >= 2 && p->r2z_ng >= 1 && p->coef_n >= 3 && p->dn_n >= 1 && (!p->rsd || p->dg_n >= 2) &&
                   p->r2z_step > 0.0 && p->dn_dz > 0.0,
               SMK_ERR_ARG, "bad table sizes");
+  SMK_REQUIRE(scratch == nullptr || (scratch_bytes >= smk_qso_scratch_bytes(p) && ((uintptr_t)scratch & 7) == 0),
+              SMK_ERR_ARG, "scratch too small or misaligned");
   hipStream_t s = (hipStream_t)stream;
   unsigned long long* cnt = reinterpret_cast<unsigned long long*>(count);
   hipLaunchKernelGGL(k_clear_count, dim3(1), dim3(64), 0, s, cnt);
   SMK_LAUNCH_CHECK();
   const uint64_t ncol = (uint64_t)p->nx * (uint64_t)p->ny;
-  const uint32_t nzb = (uint32_t)((p->nz + 255) / 256);
+  const uint32_t nzb = (uint32_t)(((int64_t)p->nz + 255) / 256);
   SMK_REQUIRE(ncol <= 0x7fffffffull && nzb <= 65535u, SMK_ERR_ARG, "slab too large for one launch");
-  hipLaunchKernelGGL(k_qso_draw, dim3((uint32_t)ncol, nzb), dim3(256), 0, s, *p, p1, p2, p3, vx, vy, vz, seed,
-                     records, capacity, cnt);
+  if (scratch == nullptr) {
+    hipLaunchKernelGGL(k_qso_draw, dim3((uint32_t)ncol, nzb), dim3(256), 0, s, *p, p1, p2, p3, vx, vy, vz, seed, records,
+                       capacity, cnt);
+    SMK_LAUNCH_CHECK();
+    return SMK_OK;
+  }
+  const uint64_t nb = qso_bounds(*p);
+  DrawBound* bounds = static_cast<DrawBound*>(scratch);
+  uint64_t* mask = reinterpret_cast<uint64_t*>(bounds + nb);
+  const uint32_t nch = (uint32_t)(((int64_t)p->nz + CHUNK - 1) / CHUNK), nw = (uint32_t)(((int64_t)p->nz + 63) / 64);
+  if (!p->randoms) {
+    const uint64_t blocks = (nb + 255) / 256;
+    hipLaunchKernelGGL(k_qso_bounds, dim3((uint32_t)blocks), dim3(256), 0, s, *p, bounds, nb, nch, (uint32_t)ncol);
+    SMK_LAUNCH_CHECK();
+  }
+  hipLaunchKernelGGL(k_qso_filter,
+                     dim3((uint32_t)((ncol + COLS - 1) / COLS), (uint32_t)(((int64_t)p->nz + ZCELLS - 1) / ZCELLS)),
+                     dim3(256), 0, s, p->nz, p->randoms, p1, p2, p3, seed, bounds, nch, mask, nw, (uint32_t)ncol);
+  SMK_LAUNCH_CHECK();
+  const uint64_t total = 2 * ncol * nw;
+  const uint64_t blocks = (total + 255) / 256 < MASK_BLOCKS ? (total + 255) / 256 : MASK_BLOCKS;
+  hipLaunchKernelGGL(k_qso_masked, dim3((uint32_t)blocks), dim3(256), 0, s, *p, p1, p2, p3, vx, vy, vz, seed, records,
+                     capacity, cnt, reinterpret_cast<const uint32_t*>(mask), 2 * nw, total);
   SMK_LAUNCH_CHECK();
   return SMK_OK;
 }

@@ -209,6 +209,9 @@ class Drawer:
         self.count = torch.zeros(1, dtype=torch.int64, device=self.dev)
         self.capacity = int(capacity) if capacity is not None else max(1024, int(4 * s.n_expected) + 1024)
         self.records = torch.empty((self.capacity, RECORD.itemsize), dtype=torch.uint8, device=self.dev)
+        # the draw's mask of candidate cells (smk_qso_draw_scratch)
+        self.scratch = torch.empty(int(_lib.lib().smk_qso_scratch_bytes(ctypes.byref(prm))), dtype=torch.uint8,
+                                   device=self.dev)
 
     def _t(self, a, dtype=torch.float64):
         x = torch.as_tensor(np.ascontiguousarray(a), dtype=dtype).to(self.dev)
@@ -216,8 +219,8 @@ class Drawer:
         return x.data_ptr()
 
     def launch(self, p1, p2, p3, vel=None, seed=0, stream=None):
-        """One smk_qso_draw into the record buffer (asynchronous); returns the
-        device count."""
+        """One smk_qso_draw_scratch into the record buffer (asynchronous); returns
+        the device count.  The Drawer's buffers hold one draw at a time."""
         s = self.setup
         for a in (p1, p2, p3):
             if a is not None and (a.dtype != torch.float32 or tuple(a.shape) != (s.nx, s.ny, s.nz)
@@ -226,11 +229,13 @@ class Drawer:
         if self.prm.rsd and vel is None:
             raise ValueError("rsd needs the velocity boxes")
         vx, vy, vz = vel if vel is not None else (None, None, None)
-        _lib.check(_lib.lib().smk_qso_draw(ctypes.byref(self.prm), _lib.ptr(p1), _lib.ptr(p2), _lib.ptr(p3),
-                                           _lib.ptr(vx), _lib.ptr(vy), _lib.ptr(vz),
-                                           ctypes.c_uint64(int(seed) & (2 ** 64 - 1)), _lib.ptr(self.records),
-                                           self.capacity, _lib.ptr(self.count), _lib.stream_ptr(stream)),
-                   "smk_qso_draw")
+        _lib.check(_lib.lib().smk_qso_draw_scratch(ctypes.byref(self.prm), _lib.ptr(p1), _lib.ptr(p2), _lib.ptr(p3),
+                                                   _lib.ptr(vx), _lib.ptr(vy), _lib.ptr(vz),
+                                                   ctypes.c_uint64(int(seed) & (2 ** 64 - 1)),
+                                                   _lib.ptr(self.records), self.capacity, _lib.ptr(self.count),
+                                                   _lib.ptr(self.scratch), self.scratch.numel(),
+                                                   _lib.stream_ptr(stream)),
+                   "smk_qso_draw_scratch")
         return self.count
 
     def __call__(self, p1, p2, p3, vel=None, seed=0, stream=None):
