@@ -245,8 +245,10 @@ class Drawer:
                 break
             self.capacity = n + 1024
             self.records = torch.empty((self.capacity, RECORD.itemsize), dtype=torch.uint8, device=self.dev)
-        out = np.frombuffer(self.records[:n].cpu().numpy().tobytes(), dtype=RECORD).copy()
-        return out[np.argsort(out["key"], kind="stable")]
+        out = self.records[:n].cpu().numpy().view(RECORD)[:, 0]
+        # take moves whole records; indexing and copying a structured array go
+        # field by field (2300 records: 263 and 158 us)
+        return out.take(np.argsort(out["key"], kind="stable"))
 
 
 def draw(setup, p1, p2, p3, vel=None, seed=0, capacity=None, stream=None):
