@@ -87,28 +87,230 @@ __device__ __forceinline__ double rsd_integrand(const RsdArgs& a, double kpar, d
   return kperp * r * r * f * p;
 }
 
-// One block per k_par row.  The trapezoid sum over k_perp is taken as
+// The sum over [j0, j1) of a block's row of k_perp.  The trapezoid sum is taken as
 // sum_j f_j (x_{j+1} - x_{j-1}) / 2 (half intervals at the ends), so each
 // point is evaluated once.
 template <int MODEL>
-__global__ __launch_bounds__(256) void k_p1d_rsd_rows(RsdArgs a) {
-  __shared__ double red[4];
-  const int i = blockIdx.x;
-  const double kpar = a.k_par[i];
+__device__ __forceinline__ double row_sum(const RsdArgs& a, double kpar, int j0, int j1) {
   const double lkpar = kpar > 0.0 ? log(kpar) : 0.0;
   const int n = a.n_perp;
   double acc = 0.0;
-  for (int j = threadIdx.x; j < n; j += 256) {
+  for (int j = j0 + (int)threadIdx.x; j < j1; j += 256) {
     const double x = a.k_perp[j];
     const double hi = j + 1 < n ? a.k_perp[j + 1] : x;
     const double lo = j > 0 ? a.k_perp[j - 1] : x;
     acc += (hi - lo) * rsd_integrand<MODEL>(a, kpar, lkpar, x) / 2.0;
   }
-  // wave then block reduction in a fixed order
+  return acc;
+}
+
+// log and exp in FP64 from a table and a short polynomial (P. T. P. Tang, ACM
+// TOMS 16 (1990) 378 and 15 (1989) 144): the argument is reduced to a node of
+// the table and a remainder small enough for a degree of 6 and 5.  log_t: of
+// normal numbers, error below 1.2 half ulps of the larger of |log x| and 1 / 2;
+// exp_t: arguments of [-745, 690], relative error below 3e-16.
+constexpr double LN2_HI = 0x1.62e42fefap-1, LN2_LO = 0x1.cf79abc9e3b3ap-40;   // LN2_HI: 36 bits
+
+struct MathTables {
+  // c the middles of the 128ths of [1, 2): 1 / c; log c to 36 bits after the point, and the rest
+  double rcp[128], lhi[128], llo[128];
+  double pw[64];              // 2^(i / 64)
+};
+
+__device__ __forceinline__ void fill_tables(MathTables& t, int tid) {
+  if (tid < 128) {
+    const double r = 1.0 / (1.0 + (tid + 0.5) / 128.0);
+    const double l = -log(r), hi = rint(l * 0x1p36) * 0x1p-36;
+    t.rcp[tid] = r;
+    t.lhi[tid] = hi;
+    t.llo[tid] = l - hi;
+  } else if (tid < 192) {
+    t.pw[tid - 128] = exp2((tid - 128) / 64.0);
+  }
+}
+
+__device__ __forceinline__ double log_t(const MathTables& t, double x) {
+  const uint64_t u = (uint64_t)__double_as_longlong(x);
+  const double e = (double)((int)(u >> 52) - 1023);
+  const int i = (int)(u >> 45) & 127;
+  const double m = __longlong_as_double((long long)((u & 0x000fffffffffffffull) | 0x3ff0000000000000ull));
+  const double z = fma(m, t.rcp[i], -1.0);       // |z| <= 1 / 256
+  double q = fma(z, -1.0 / 6, 1.0 / 5);
+  q = fma(z, q, -1.0 / 4);
+  q = fma(z, q, 1.0 / 3);
+  q = fma(z, q, -1.0 / 2);
+  q = fma(z * z, q, fma(e, LN2_LO, t.llo[i]));
+  return fma(e, LN2_HI, t.lhi[i]) + (z + q);     // the product's sum is exact
+}
+
+__device__ __forceinline__ double exp_t(const MathTables& t, double y) {
+  constexpr double M = 6755399441055744.0;       // 1.5 2^52: the sum rounds to an integer
+  const double s = fma(y, 64 * 1.4426950408889634, M), n = s - M;
+  const double f = fma(n, -LN2_LO / 64, fma(n, -LN2_HI / 64, y));   // |f| <= ln 2 / 128
+  const int k = (int)__double_as_longlong(s);
+  double q = fma(f, 1.0 / 120, 1.0 / 24);
+  q = fma(f, q, 1.0 / 6);
+  q = fma(f, q, 0.5);
+  q = fma(f * f, q, f);
+  const double w = t.pw[k & 63];
+  return ldexp(fma(w, q, w), k >> 6);
+}
+
+// the spline segment of the last point
+struct Segment {
+  double lo, hi;              // [lo, hi), to infinity at the ends of the spline
+  double x, c0, c1, c2, c3;
+  int iv;
+};
+
+__device__ __forceinline__ void find_segment(const smk_pk_spline& sp, double r_step, double k, Segment& s) {
+  // mostly the next one
+  int iv = s.iv + 1;
+  if (!(k >= s.hi && iv < sp.n_int && (iv + 1 == sp.n_int || k < sp.x[iv + 1]))) {
+    iv = sp.guess[(int)fmin(fmax((k - sp.g_lo) * r_step, 0.0), (double)(sp.n_guess - 1))];
+    while (iv + 1 < sp.n_int && sp.x[iv + 1] <= k) ++iv;
+    while (iv > 0 && sp.x[iv] > k) --iv;
+  }
+  const double* cc = sp.c + 4 * (int64_t)iv;
+  s.iv = iv;
+  s.x = sp.x[iv];
+  s.lo = iv > 0 ? s.x : -INFINITY;
+  s.hi = iv + 1 < sp.n_int ? sp.x[iv + 1] : INFINITY;
+  s.c0 = cc[0];
+  s.c1 = cc[1];
+  s.c2 = cc[2];
+  s.c3 = cc[3];
+}
+
+// The row's sum with fewer FP64 instructions per point (models 0 and 1): one
+// reciprocal square root gives k and mu^2, the spline's segment is kept from
+// one point of a lane to the next, and model 1's powers and exponentials
+// are one log_t and two exp_t.  ok is cleared where an argument leaves
+// their ranges or is no number: the row is then row_sum's.
+//
+// Bound by FP64 issue.  20000 rows of 20000 points, model 1: 344 instructions
+// per point and 3.5 ms with the library's square root, divisions, log and exp,
+// 110 and 1.35 ms (80% of the issue rate) here.  With the segment of every
+// point looked up in the guess table 1.40; 8 waves per SIMD instead of 6 spill
+// (1.55), 4 leave latencies bare (1.50).  The log's and exp's short forms in base 2
+// took 6 instructions less, but their constants' rounding made the rows' error
+// against exact sums four times larger; as it is, it is half of before.
+template <int MODEL>
+__device__ __forceinline__ double row_fast(const RsdArgs& a, const MathTables& t, double kpar, bool& ok) {
+  const int n = a.n_perp;
+  const double kp2 = kpar * kpar, r_step = 1.0 / a.sp.g_step;
+  const double lkpar = log(kpar), lkv = log(a.kv), rkp = 1.0 / a.kp;
+  const double cg = a.G * a.G / (2.0 * M_PI * M_PI);
+  // the rest of 1 / k_p, whose rounding would be the same in every point
+  const double rkp_lo = fma(-rkp, a.kp, 1.0) * rkp;
+  Segment s;
+  s.iv = -1;
+  s.lo = s.hi = INFINITY;
+  double acc = 0.0;
+  const auto point = [&](double x, double dx) {
+    const double k2 = fma(x, x, kp2);
+    // 1 / k by a third-order step from the hardware's estimate
+    const double y0 = __builtin_amdgcn_rsq(k2), h = k2 * y0, e = fma(-h, y0, 1.0);
+    const double c = e * fma(0.375, e, 0.5);
+    const double k = fma(h, c, h), rk = fma(y0, c, y0);
+    if (!(k >= s.lo && k < s.hi)) find_segment(a.sp, r_step, k, s);
+    const double d = k - s.x;
+    const double p = fmax(fma(fma(fma(s.c0, d, s.c1), d, s.c2), d, s.c3), 0.0);
+    ok = ok && k2 < 1e200;
+    double g = x * p;
+    if (MODEL == 1) {
+      const double d2 = cg * (k * k2) * p;
+      const double lk = 0.5 * log_t(t, k2);
+      const double y1 = fma(a.av, lk - lkv, a.bv * (lkpar - lk));
+      const double pw = exp_t(t, y1);
+      const double kk = fma(k, rkp, k * rkp_lo);
+      const double y2 = fma(d2 * fma(a.q2, d2, a.q1), 1.0 - pw, -(kk * kk));
+      ok = ok && fabs(y1) < 690.0 && y2 < 690.0;
+      g *= exp_t(t, fmax(y2, -745.0));
+    }
+    const double mu = kpar * rk, r = fma(a.beta * mu, mu, 1.0);
+    acc = fma(dx, g * (r * r), acc);
+  };
+  // each wave has a quarter of the inner points, its lanes 64 points from one
+  // to the next, mostly within a segment; the row's ends go to two other lanes
+  const int m = n - 2, nw = (m + 3) / 4, w = (int)threadIdx.x / 64, end = (w + 1) * nw < m ? (w + 1) * nw : m;
+  const double* xp = a.k_perp + 1 + w * nw + (int)(threadIdx.x & 63);
+  for (int j = w * nw + (int)(threadIdx.x & 63); j < end; j += 64, xp += 64) point(xp[0], xp[1] - xp[-1]);
+  if (threadIdx.x >= 254) {
+    const int j = threadIdx.x == 254 ? 0 : n - 1;
+    point(a.k_perp[j], a.k_perp[j > 0 ? j : 1] - a.k_perp[j > 0 ? j - 1 : 0]);
+  }
+  return acc * 0.5;
+}
+
+// the block's sum, in a fixed order, as the row's value
+__device__ __forceinline__ void store_row(const RsdArgs& a, int i, double acc, double* red) {
   for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
   __syncthreads();
   if (threadIdx.x == 0) a.out[i] = (((red[0] + red[1]) + red[2]) + red[3]) / 2.0 / M_PI;
+  __syncthreads();
+}
+
+// One block per k_par row (models 0 and 1).
+template <int MODEL>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k_p1d_rsd_rows(RsdArgs a) {
+  __shared__ double red[4];
+  __shared__ MathTables t;
+  const double kpar = a.k_par[blockIdx.x];
+  double acc = 0.0;
+  bool ok = kpar > 1e-14 && kpar < 1e100;
+  if (MODEL == 1) {
+    fill_tables(t, threadIdx.x);
+    __syncthreads();
+  }
+  if (ok) acc = row_fast<MODEL>(a, t, kpar, ok);
+  if (__syncthreads_or(!ok)) acc = row_sum<MODEL>(a, kpar, 0, a.n_perp);
+  store_row(a, blockIdx.x, acc, red);
+}
+
+// Model 2: the integrand is 0 from k_ny on.  A block finds the range of k_perp
+// within k_ny (with a margin over the rounding of k) of any of its rows, then
+// sums the rows over it.  What is no number, or large enough that a product
+// might overflow, counts as within.
+//
+// 20000 rows of 20000 points: 1.6 ms with every point evaluated, 0.21 with
+// whole waves passing over the points beyond, row by row, bound by the
+// 3.2 GB of k_perp that the rows read from L2; 0.09 with 8 rows to a block.
+// Fewer rows than 8192 go fewer to a block, so that the blocks fill the card.
+__global__ __launch_bounds__(256) void k_p1d_cut_rows(RsdArgs a, int n_par, int rows) {
+  __shared__ double red[4];
+  __shared__ int range[2];
+  const int n = a.n_perp, i0 = blockIdx.x * rows, i1 = n_par - i0 < rows ? n_par : i0 + rows;
+  if (threadIdx.x == 0) {
+    range[0] = n;
+    range[1] = 0;
+  }
+  double kp2 = INFINITY;
+  bool all = !(fabs(a.beta) < 1e100);
+  for (int i = i0; i < i1; ++i) {
+    const double k = a.k_par[i];
+    all = all || !(k * k < 1e100);
+    kp2 = fmin(kp2, k * k);
+  }
+  const double far = a.kny * a.kny * (1.0 + 1e-12);
+  __syncthreads();
+  int lo = n, hi = 0;
+  for (int j = threadIdx.x; j < n; j += 256) {
+    const double x = a.k_perp[j], k2 = fma(x, x, kp2);
+    if (all || !(k2 > far && k2 < 1e100)) {
+      lo = j < lo ? j : lo;
+      hi = j + 1;
+    }
+  }
+  if (hi > 0) {
+    atomicMin(&range[0], lo);
+    atomicMax(&range[1], hi);
+  }
+  __syncthreads();
+  lo = range[0] & ~255;   // whole turns of the block: the sum's order is that of the whole row
+  hi = range[1];
+  for (int i = i0; i < i1; ++i) store_row(a, i, row_sum<2>(a, a.k_par[i], lo, hi), red);
 }
 
 }  // namespace
@@ -139,7 +341,10 @@ extern "C" int smk_p1d_rsd_rows(const smk_pk_spline* spline, const double* k_par
   const hipStream_t st = (hipStream_t)stream;
   if (model == 0) hipLaunchKernelGGL(k_p1d_rsd_rows<0>, dim3(n_par), dim3(256), 0, st, a);
   else if (model == 1) hipLaunchKernelGGL(k_p1d_rsd_rows<1>, dim3(n_par), dim3(256), 0, st, a);
-  else hipLaunchKernelGGL(k_p1d_rsd_rows<2>, dim3(n_par), dim3(256), 0, st, a);
+  else {
+    const int rows = n_par < 2048 ? 1 : (n_par < 8192 ? n_par / 1024 : 8);   // 1024 blocks or more
+    hipLaunchKernelGGL(k_p1d_cut_rows, dim3((n_par + rows - 1) / rows), dim3(256), 0, st, a, n_par, rows);
+  }
   SMK_LAUNCH_CHECK();
   return SMK_OK;
 }
