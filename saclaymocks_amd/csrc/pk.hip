@@ -1,10 +1,10 @@
 // Per-mode P(k) tables on gfx950 (interpolate_pk.py).
 //
-// One thread per mode of the k-space box: k from the float32 axes with the
+// For each mode of the k-space box: k from the float32 axes with the
 // reference's float32 operations (correctly rounded, as numpy's), the spline
 // segment from a uniform guess table plus a short walk, a Horner cubic in
-// FP64, then float32 max(P, 0) / Vcell and its square root.  The output is
-// written once, so the kernel is bound by the 4 B per mode it stores.
+// FP64, then float32 max(P, 0) / Vcell and its square root.  And the rows of
+// the missing 1D power (p1d_missing.py).
 #include <math.h>
 
 #include "fft_core.h"
@@ -26,26 +26,212 @@ __device__ __forceinline__ double spline_eval(const smk_pk_spline& sp, double k)
   return ((cc[0] * t + cc[1]) * t + cc[2]) * t + cc[3];
 }
 
-__global__ __launch_bounds__(256) void k_pk_table(smk_pk_spline sp, const float* __restrict__ kx,
-                                                  const float* __restrict__ ky, const float* __restrict__ kz,
-                                                  int ny, int nzh, float vcell, float* __restrict__ out,
-                                                  uint64_t nmodes) {
-  const uint64_t m = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-  if (m >= nmodes) return;
-  const int l = (int)(m % (uint64_t)nzh);
-  const uint64_t rest = m / (uint64_t)nzh;
-  const int j = (int)(rest % (uint64_t)ny);
-  const int i = (int)(rest / (uint64_t)ny);
-  const float a = kx[i], b = ky[j], c = kz[l];
-  // numpy float32: (kx*kx + ky*ky) + kz*kz, then sqrt, each correctly rounded
-  // (the square root and the quotient below through FP64, which rounds them
-  // to the correctly rounded float32 results)
-  const float kk = add_rn(add_rn(mul_rn(a, a), mul_rn(b, b)), mul_rn(c, c));
-  const float kf = (float)sqrt((double)kk);
-  const double p = spline_eval(sp, (double)kf);
-  const float pf = (float)fmax(p, 0.0);
-  const float q = (float)((double)pf / (double)vcell);
-  out[m] = (float)sqrt((double)q);
+// the spline segment of the last point
+struct Segment {
+  double lo, hi;              // [lo, hi), to infinity at the ends of the spline
+  double x, c0, c1, c2, c3;
+  int iv;
+};
+
+__device__ __forceinline__ void find_segment(const smk_pk_spline& sp, double r_step, double k, Segment& s) {
+  // mostly the next one
+  int iv = s.iv + 1;
+  if (!(k >= s.hi && iv < sp.n_int && (iv + 1 == sp.n_int || k < sp.x[iv + 1]))) {
+    iv = sp.guess[(int)fmin(fmax((k - sp.g_lo) * r_step, 0.0), (double)(sp.n_guess - 1))];
+    while (iv + 1 < sp.n_int && sp.x[iv + 1] <= k) ++iv;
+    while (iv > 0 && sp.x[iv] > k) --iv;
+  }
+  const double* cc = sp.c + 4 * (int64_t)iv;
+  s.iv = iv;
+  s.x = sp.x[iv];
+  s.lo = iv > 0 ? s.x : -INFINITY;
+  s.hi = iv + 1 < sp.n_int ? sp.x[iv + 1] : INFINITY;
+  s.c0 = cc[0];
+  s.c1 = cc[1];
+  s.c2 = cc[2];
+  s.c3 = cc[3];
+}
+
+// The correctly rounded float32 square root, through FP64: a third-order step
+// from the hardware's reciprocal square root is within 2^-51, and the root of a
+// float32 is never nearer than 2^-50 to the middle of two.
+__device__ __forceinline__ float sqrt_f32(float x) {
+  const double d = (double)x, y = __builtin_amdgcn_rsq(d), h = d * y, e = fma(-h, y, 1.0);
+  const float r = (float)fma(h, e * fma(0.375, e, 0.5), h);
+  return __builtin_amdgcn_classf(x, 0x180) ? r : x;   // x if not positive and finite
+}
+
+struct TableArgs {
+  smk_pk_spline sp;
+  double r_step, r_lo, r_vcell;   // 1 / sp.g_step, -sp.g_lo / sp.g_step, 1 / vcell
+  const float *kx, *ky, *kz;
+  uint32_t ny, nzh, nch;          // nch: 64-mode pieces of a row
+  float* out;
+  uint64_t nrows, ngroup;         // groups of TABLE_ROWS rows
+  // the grid's waves as a step over (group, piece), and its group as rows (i, j)
+  uint64_t dgroup;
+  uint32_t dch, di, dj;
+};
+
+// the bin of k, of bins 0 ... last of 1 / r_step (a NaN takes 0)
+__device__ __forceinline__ uint32_t guess_bin(double k, double r_step, double r_lo, uint32_t last) {
+  const uint32_t g = (uint32_t)fmax(fma(k, r_step, r_lo), 0.0);
+  return g < last ? g : last;
+}
+
+// sqrt(max(P, 0) / vcell), P the cubic c at d; the float32 quotient is rounded
+// once: 1 / vcell is exact to 2^-53, and a quotient of float32s no nearer than
+// 2^-49 to the middle of two
+__device__ __forceinline__ float table_value(const TableArgs& a, const double* c, double d) {
+  const double p = ((c[0] * d + c[1]) * d + c[2]) * d + c[3];
+  return sqrt_f32((float)((double)fmaxf((float)p, 0.0f) * a.r_vcell));
+}
+
+__device__ __forceinline__ float table_global(const TableArgs& a, double k) {
+  int iv = a.sp.guess[guess_bin(k, a.r_step, a.r_lo, (uint32_t)a.sp.n_guess - 1)];
+  while (iv + 1 < a.sp.n_int && a.sp.x[iv + 1] <= k) ++iv;
+  while (iv > 0 && a.sp.x[iv] > k) --iv;
+  return table_value(a, a.sp.c + 4 * (int64_t)iv, k - a.sp.x[iv]);
+}
+
+constexpr int TABLE_ROWS = 4;  // rows that a wave's lanes have at a time
+constexpr int SEGS = 1760;     // segments in LDS: two blocks of 1024 threads per CU
+constexpr int BINS = 4096;     // bins of the guess table in LDS
+// Tables from here on take the LDS kernel, whose blocks first load 20 to 80 KB
+// each: 2.5 million modes take 15.9 us with and 14.5 without, 3.7 million 19.2
+// and 19.0, 6.2 million 25.9 and 27.2.
+constexpr uint64_t LDS_MODES = 4u << 20;
+
+// A wave has 64 neighbouring modes of TABLE_ROWS rows at a time, a lane one
+// column of them: k from the float32 axes as numpy's sqrt((kx*kx + ky*ky) + kz*kz),
+// each operation correctly rounded.  With LDS the block keeps the segments that
+// the guess table reaches (if no more than SEGS) and a guess of BINS bins; what
+// they do not settle goes to the spline in global memory.
+//
+// A table of 40 x 2560 x 769 takes 67 us to write.  It took 375 us with a thread
+// per mode: two 64-bit modulos, two FP64 square roots and two divisions each,
+// and a guess table of 256 KB gathered through L1.  Now 197 with LDS and 250
+// without; the instructions left (60 per mode, 7 of them conversions or
+// reciprocal roots of a quarter of the rate) take about 165.  Four modes of a
+// row per lane instead, with their index arithmetic: 248 and 340; eight rows:
+// 205, spilling.  A spline of 1e5 nodes within reach: 1563 before, 1374.
+template <bool LDS>
+__global__ __launch_bounds__(LDS ? 1024 : 256) __attribute__((amdgpu_waves_per_eu(8))) void k_pk_table(TableArgs a) {
+  __shared__ double x[LDS ? SEGS + 2 : 1];
+  __shared__ __align__(16) double c[LDS ? 4 * (SEGS + 1) : 2];
+  __shared__ uint16_t guess[LDS ? BINS : 1];   // bytes into x
+  const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63;
+  // the segments of the guess table's range, [s0, s0 + ns)
+  int s0 = 0, ns = 0, sh = 0;
+  bool lds = false;
+  if (LDS) {
+    s0 = a.sp.guess[0];
+    ns = a.sp.guess[a.sp.n_guess - 1] - s0 + 1;
+    lds = ns >= 1 && ns <= SEGS;
+    if (lds) {
+      while ((a.sp.n_guess - 1) >> sh >= BINS) ++sh;
+      for (int q = tid; q <= (a.sp.n_guess - 1) >> sh; q += nt) {
+        const int g = a.sp.guess[q << sh] - s0;
+        guess[q] = (uint16_t)(8 * (g < 0 ? 0 : (g < ns ? g : ns - 1)));
+      }
+      // (the spline's last segment has no end; segment ns is never taken)
+      for (int q = tid; q <= ns + 1; q += nt)
+        x[q] = q < ns || (q == ns && s0 + ns < a.sp.n_int) ? a.sp.x[s0 + q] : (q == ns ? INFINITY : -INFINITY);
+      for (int q = tid; q < 4 * ns; q += nt) c[q] = a.sp.c[4 * (int64_t)s0 + q];
+    }
+    __syncthreads();
+  }
+  // the scaling by a power of 2 is exact: bin >> sh
+  const double r_bin = ldexp(a.r_step, -sh), r_bin0 = ldexp(a.r_lo, -sh);
+  const uint32_t last_bin = (uint32_t)(a.sp.n_guess - 1) >> sh;
+  const uint32_t w = blockIdx.x * (nt / 64) + (uint32_t)__builtin_amdgcn_readfirstlane(tid / 64);
+  uint32_t ch = w % a.nch, i = w / a.nch * TABLE_ROWS / a.ny, j = w / a.nch * TABLE_ROWS % a.ny;
+  for (uint64_t group = w / a.nch; group < a.ngroup;) {
+    const uint64_t row = group * TABLE_ROWS;
+    const uint32_t l = ch * 64 + (uint32_t)lane;
+    const float kz = a.kz[l < a.nzh ? l : a.nzh - 1], cc = mul_rn(kz, kz);
+    double k[TABLE_ROWS];
+    float r[TABLE_ROWS];
+    uint32_t iu = i, ju = j;
+#pragma unroll
+    for (int u = 0; u < TABLE_ROWS; ++u) {
+      const float kx = a.kx[iu], ky = a.ky[ju];
+      k[u] = (double)sqrt_f32(add_rn(add_rn(mul_rn(kx, kx), mul_rn(ky, ky)), cc));
+      if (row + (uint64_t)u + 1 < a.nrows && ++ju == a.ny) {   // past the last row the last row again
+        ju = 0;
+        ++iu;
+      }
+    }
+    bool off = false;   // past the segments in LDS, or two segments past the bin's
+    if (LDS && lds) {
+      uint32_t at[TABLE_ROWS];
+      double x0[TABLE_ROWS];
+      const char *xb = reinterpret_cast<const char*>(x), *cb = reinterpret_cast<const char*>(c);
+#pragma unroll
+      for (int u = 0; u < TABLE_ROWS; ++u) at[u] = guess[guess_bin(k[u], r_bin, r_bin0, last_bin)];
+      // the bin's segment or the next one, mostly
+#pragma unroll
+      for (int u = 0; u < TABLE_ROWS; ++u) at[u] += k[u] >= *reinterpret_cast<const double*>(xb + at[u] + 8) ? 8u : 0u;
+#pragma unroll
+      for (int u = 0; u < TABLE_ROWS; ++u) {
+        x0[u] = *reinterpret_cast<const double*>(xb + at[u]);
+        const double x1 = *reinterpret_cast<const double*>(xb + at[u] + 8);
+        off |= !(k[u] >= x0[u]) | !(k[u] < x1);
+      }
+#pragma unroll
+      for (int u = 0; u < TABLE_ROWS; ++u)
+        r[u] = table_value(a, reinterpret_cast<const double*>(cb + 4 * at[u]), k[u] - x0[u]);
+    }
+    if (!lds) {
+      // the loads of all rows ahead of what waits for them
+      int iv[TABLE_ROWS];
+      double x0[TABLE_ROWS], x1[TABLE_ROWS];
+#pragma unroll
+      for (int u = 0; u < TABLE_ROWS; ++u)
+        iv[u] = a.sp.guess[guess_bin(k[u], a.r_step, a.r_lo, (uint32_t)a.sp.n_guess - 1)];
+#pragma unroll
+      for (int u = 0; u < TABLE_ROWS; ++u) {
+        x0[u] = a.sp.x[iv[u]];
+        x1[u] = a.sp.x[iv[u] + 1];
+      }
+#pragma unroll
+      for (int u = 0; u < TABLE_ROWS; ++u) {
+        if (k[u] >= x1[u] || k[u] < x0[u]) {
+          while (iv[u] + 1 < a.sp.n_int && a.sp.x[iv[u] + 1] <= k[u]) ++iv[u];
+          while (iv[u] > 0 && a.sp.x[iv[u]] > k[u]) --iv[u];
+          x0[u] = a.sp.x[iv[u]];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < TABLE_ROWS; ++u) r[u] = table_value(a, a.sp.c + 4 * (int64_t)iv[u], k[u] - x0[u]);
+    } else if (off) {
+#pragma unroll 1
+      for (int u = 0; u < TABLE_ROWS; ++u) {
+        const float v = table_global(a, u == 0 ? k[0] : (u == 1 ? k[1] : (u == 2 ? k[2] : k[3])));
+        r[0] = u == 0 ? v : r[0];
+        r[1] = u == 1 ? v : r[1];
+        r[2] = u == 2 ? v : r[2];
+        r[3] = u == 3 ? v : r[3];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < TABLE_ROWS; ++u)
+      if (l < a.nzh && row + (uint64_t)u < a.nrows) a.out[(row + (uint64_t)u) * a.nzh + l] = r[u];
+    // the next piece of this wave
+    group += a.dgroup;
+    i += a.di;
+    j += a.dj;
+    ch += a.dch;
+    if (ch >= a.nch) {
+      ch -= a.nch;
+      ++group;
+      j += TABLE_ROWS;
+    }
+    while (j >= a.ny) {
+      j -= a.ny;
+      ++i;
+    }
+  }
 }
 
 struct RsdArgs {
@@ -154,32 +340,6 @@ __device__ __forceinline__ double exp_t(const MathTables& t, double y) {
   q = fma(f * f, q, f);
   const double w = t.pw[k & 63];
   return ldexp(fma(w, q, w), k >> 6);
-}
-
-// the spline segment of the last point
-struct Segment {
-  double lo, hi;              // [lo, hi), to infinity at the ends of the spline
-  double x, c0, c1, c2, c3;
-  int iv;
-};
-
-__device__ __forceinline__ void find_segment(const smk_pk_spline& sp, double r_step, double k, Segment& s) {
-  // mostly the next one
-  int iv = s.iv + 1;
-  if (!(k >= s.hi && iv < sp.n_int && (iv + 1 == sp.n_int || k < sp.x[iv + 1]))) {
-    iv = sp.guess[(int)fmin(fmax((k - sp.g_lo) * r_step, 0.0), (double)(sp.n_guess - 1))];
-    while (iv + 1 < sp.n_int && sp.x[iv + 1] <= k) ++iv;
-    while (iv > 0 && sp.x[iv] > k) --iv;
-  }
-  const double* cc = sp.c + 4 * (int64_t)iv;
-  s.iv = iv;
-  s.x = sp.x[iv];
-  s.lo = iv > 0 ? s.x : -INFINITY;
-  s.hi = iv + 1 < sp.n_int ? sp.x[iv + 1] : INFINITY;
-  s.c0 = cc[0];
-  s.c1 = cc[1];
-  s.c2 = cc[2];
-  s.c3 = cc[3];
 }
 
 // The row's sum with fewer FP64 instructions per point (models 0 and 1): one
@@ -359,10 +519,32 @@ extern "C" int smk_pk_table(const smk_pk_spline* spline, const float* kx, const 
   SMK_REQUIRE(nxs >= 0 && ny > 0 && nzh > 0 && vcell > 0.0f, SMK_ERR_ARG, "bad table shape");
   const uint64_t nmodes = (uint64_t)nxs * (uint64_t)ny * (uint64_t)nzh;
   if (nmodes == 0) return SMK_OK;
-  const uint64_t nblk = (nmodes + 255) / 256;
-  SMK_REQUIRE(nblk <= 0x7fffffffull, SMK_ERR_ARG, "table too large for one launch");
-  hipLaunchKernelGGL(k_pk_table, dim3((uint32_t)nblk), dim3(256), 0, (hipStream_t)stream, *spline, kx, ky, kz, ny,
-                     nzh, vcell, table, nmodes);
+  TableArgs a;
+  a.sp = *spline;
+  a.r_step = 1.0 / spline->g_step;
+  a.r_lo = -spline->g_lo / spline->g_step;
+  a.r_vcell = 1.0 / (double)vcell;
+  a.kx = kx;
+  a.ky = ky;
+  a.kz = kz;
+  a.ny = (uint32_t)ny;
+  a.nzh = (uint32_t)nzh;
+  a.nch = (uint32_t)(((int64_t)nzh + 63) / 64);
+  a.out = table;
+  a.nrows = (uint64_t)nxs * (uint64_t)ny;
+  a.ngroup = (a.nrows + TABLE_ROWS - 1) / TABLE_ROWS;
+  const hipStream_t st = (hipStream_t)stream;
+  const bool lds = nmodes >= LDS_MODES;
+  // two blocks of 16 waves per CU; or as many waves as there are pieces, of which fewer than 2^18
+  const uint64_t blocks = lds ? 512 : (a.ngroup * a.nch + 3) / 4, waves = blocks * (lds ? 16 : 4);
+  a.dgroup = waves / a.nch;
+  a.dch = (uint32_t)(waves % a.nch);
+  a.di = (uint32_t)(a.dgroup * TABLE_ROWS / a.ny);
+  a.dj = (uint32_t)(a.dgroup * TABLE_ROWS % a.ny);
+  if (lds)
+    hipLaunchKernelGGL(k_pk_table<true>, dim3((uint32_t)blocks), dim3(1024), 0, st, a);
+  else
+    hipLaunchKernelGGL(k_pk_table<false>, dim3((uint32_t)blocks), dim3(256), 0, st, a);
   SMK_LAUNCH_CHECK();
   return SMK_OK;
 }
