@@ -123,12 +123,23 @@ __device__ __forceinline__ double wave_sum(double v) {
 
 // the per-skewer FGPA kernels run one wave per skewer (a forest of ~10^3
 // pixels is ~16 loads per lane; a block per skewer spent its time on block
-// barriers and the skewer's descriptor loads)
+// barriers and the skewer's descriptor loads), k_fgpa_flux several where the
+// skewers are few or long (flux_waves)
 constexpr int FLUX_WAVES = FIT_THREADS / 64;
 __device__ __forceinline__ int flux_wave() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); }
-int grid_for_waves(int n) {
-  const int b = (n + FLUX_WAVES - 1) / FLUX_WAVES;
+int grid_for_waves(int n, int w = 1) {
+  const int b = (n + FLUX_WAVES / w - 1) / (FLUX_WAVES / w);
   return b < 1 ? 1 : (b < 65536 ? b : 65536);
+}
+// Waves of k_fgpa_flux to a skewer.  Few skewers leave waves idle if each has
+// one, and a long one is a long chain on one wave: 600 skewers of 7500 pixels
+// take 60.8, 34.7 and 22.6 us with 1, 2 and 8 (16 at the copy rate), 3000 of
+// 8000 149, 124 and 122, 1500 of 1500 15.2, 13.9 and 13.2.  Short ones do not
+// fill eight: 3000 of 700 take 13.0, 11.5 and 16.2, 2000 of 650 8.8, 8.7 and
+// 11.1, and many short ones fill the card alone: 6000 of 1000 23.8, 24.3, 32.6.
+int flux_waves(const smk_skewers& sk) {
+  if (sk.npix_total >= 1400 * (int64_t)sk.n) return 8;
+  return sk.n < 4096 ? 2 : 1;
 }
 
 // F for every pixel, in FP64 so that chi2(theta) is smooth to FP64 rounding
@@ -138,9 +149,9 @@ int grid_for_waves(int n) {
 // pixels per lane whose loads are issued together in the FGPA kernels
 constexpr int FLUX_U = 8;
 
-// one skewer's flux and forest sum of F on one wave (lane's share, pixels
-// lane + 64 k in ascending k); PP: parameters per pixel; ETA: eta given
-template <bool PP, bool ETA>
+// one skewer's flux and forest sum of F on W waves (thread lane's share, pixels
+// lane + 64 W k in ascending k); PP: parameters per pixel; ETA: eta given
+template <int W, bool PP, bool ETA>
 __device__ __forceinline__ double flux_skewer(const smk_skewers& sk, int s, const float* __restrict__ delta,
                                               const float* __restrict__ eta, const double* __restrict__ abcg,
                                               int64_t rows, double* __restrict__ flux, int lane) {
@@ -148,19 +159,20 @@ __device__ __forceinline__ double flux_skewer(const smk_skewers& sk, int s, cons
   const int n = sk.npix[s], i0 = sk.imin[s], i1 = sk.imax[s];
   const double4 ps = PP ? make_double4(0.0, 0.0, 0.0, 0.0) : prow(abcg, rows, sk.pset[s]);
   double acc = 0.0;
-  for (int i = lane; i < n; i += 64 * FLUX_U) {
-    float dv[FLUX_U], ev[FLUX_U];
+  constexpr int U = W == 1 ? FLUX_U : FLUX_U / 2;   // several waves hide each other's loads
+  for (int i = lane; i < n; i += 64 * W * U) {
+    float dv[U], ev[U];
 #pragma unroll
-    for (int u = 0; u < FLUX_U; ++u) {
+    for (int u = 0; u < U; ++u) {
       // past the end: a clamped (in-bounds, unused) load, so no load waits
       // on a branch
-      const int j = i + 64 * u < n ? i + 64 * u : n - 1;
+      const int j = i + 64 * W * u < n ? i + 64 * W * u : n - 1;
       dv[u] = delta[o + j];
       ev[u] = ETA ? eta[o + j] : 0.0f;
     }
 #pragma unroll
-    for (int u = 0; u < FLUX_U; ++u) {
-      const int j = i + 64 * u;
+    for (int u = 0; u < U; ++u) {
+      const int j = i + 64 * W * u;
       if (j < n) {
         const double4 p = PP ? prow(abcg, rows, (int64_t)sk.g0[s] + j) : ps;
         const double g = (double)dv[u] + p.z * (ETA ? (double)ev[u] : 0.0);
@@ -173,22 +185,44 @@ __device__ __forceinline__ double flux_skewer(const smk_skewers& sk, int s, cons
   return acc;
 }
 
+// the sum of v over a skewer's W waves, in their order, on its first thread
+// (lane 0); called by the whole block, w its wave
+template <int W>
+__device__ __forceinline__ double skewer_sum(double v, int w, int lane, double* part) {
+  double tot = wave_sum(v);
+  if (W > 1) {
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) part[w] = tot;
+    __syncthreads();
+    if (lane == 0)
+      for (int q = 1; q < W; ++q) tot += part[w + q];
+  }
+  return tot;
+}
+
+// W waves to a skewer, FLUX_WAVES / W skewers to a block at a time.
+template <int W>
 __global__ __launch_bounds__(FIT_THREADS) void k_fgpa_flux(smk_skewers sk, const float* __restrict__ delta,
                                                            const float* __restrict__ eta,
                                                            const double* __restrict__ abcg, int64_t rows,
                                                            double* __restrict__ flux, double* __restrict__ fsum) {
-  const int lane = threadIdx.x & 63;
+  constexpr int S = FLUX_WAVES / W;
+  __shared__ double part[FLUX_WAVES];
+  const int lane = threadIdx.x % (64 * W), w = flux_wave();
   const bool per_pixel = sk.pset == nullptr;
-  for (int s = blockIdx.x * FLUX_WAVES + flux_wave(); s < sk.n; s += gridDim.x * FLUX_WAVES) {
-    double acc;
-    if (per_pixel)
-      acc = eta ? flux_skewer<true, true>(sk, s, delta, eta, abcg, rows, flux, lane)
-                : flux_skewer<true, false>(sk, s, delta, eta, abcg, rows, flux, lane);
-    else
-      acc = eta ? flux_skewer<false, true>(sk, s, delta, eta, abcg, rows, flux, lane)
-                : flux_skewer<false, false>(sk, s, delta, eta, abcg, rows, flux, lane);
-    const double tot = wave_sum(acc);
-    if (lane == 0) fsum[s] = tot;
+  for (int s0 = blockIdx.x * S; s0 < sk.n; s0 += gridDim.x * S) {
+    const int s = s0 + w / W;
+    double acc = 0.0;
+    if (s < sk.n) {
+      if (per_pixel)
+        acc = eta ? flux_skewer<W, true, true>(sk, s, delta, eta, abcg, rows, flux, lane)
+                  : flux_skewer<W, true, false>(sk, s, delta, eta, abcg, rows, flux, lane);
+      else
+        acc = eta ? flux_skewer<W, false, true>(sk, s, delta, eta, abcg, rows, flux, lane)
+                  : flux_skewer<W, false, false>(sk, s, delta, eta, abcg, rows, flux, lane);
+    }
+    const double tot = skewer_sum<W>(acc, w, lane, part);
+    if (lane == 0 && s < sk.n) fsum[s] = tot;
   }
 }
 
@@ -1538,27 +1572,28 @@ __device__ __forceinline__ JacPoint jac_point(const JacArgs& a, int64_t o, int q
 }
 
 // one skewer's flux (k_fgpa_flux's expression) and its forest sums of F
-// and of dF/d(a, b, c) at the parameters of its set, on one wave
-template <bool ETA>
+// and of dF/d(a, b, c) at the parameters of its set, on W waves as there
+template <int W, bool ETA>
 __device__ __forceinline__ void flux_jac_skewer(const smk_skewers& sk, int s, const float* __restrict__ delta,
                                                 const float* __restrict__ eta, const double* __restrict__ abcg,
                                                 int64_t rows, double* __restrict__ flux, int lane, double (&v)[4]) {
   const int64_t o = sk.off[s];
   const int n = sk.npix[s], i0 = sk.imin[s], i1 = sk.imax[s];
   const double4 p = prow(abcg, rows, sk.pset[s]);
-  for (int i = lane; i < n; i += 64 * FLUX_U) {
-    float dv[FLUX_U], ev[FLUX_U];
+  constexpr int U = W == 1 ? FLUX_U : FLUX_U / 2;
+  for (int i = lane; i < n; i += 64 * W * U) {
+    float dv[U], ev[U];
 #pragma unroll
-    for (int u = 0; u < FLUX_U; ++u) {
+    for (int u = 0; u < U; ++u) {
       // past the end: a clamped (in-bounds, unused) load, so no load waits
       // on a branch
-      const int j = i + 64 * u < n ? i + 64 * u : n - 1;
+      const int j = i + 64 * W * u < n ? i + 64 * W * u : n - 1;
       dv[u] = delta[o + j];
       ev[u] = ETA ? eta[o + j] : 0.0f;
     }
 #pragma unroll
-    for (int u = 0; u < FLUX_U; ++u) {
-      const int j = i + 64 * u;
+    for (int u = 0; u < U; ++u) {
+      const int j = i + 64 * W * u;
       if (j < n) {
         const double e = ETA ? (double)ev[u] : 0.0;
         const double g = (double)dv[u] + p.z * e;
@@ -1576,21 +1611,27 @@ __device__ __forceinline__ void flux_jac_skewer(const smk_skewers& sk, int s, co
   }
 }
 
+template <int W>
 __global__ __launch_bounds__(FIT_THREADS) void k_fgpa_flux_jac(smk_skewers sk, const float* __restrict__ delta,
                                                                const float* __restrict__ eta,
                                                                const double* __restrict__ abcg, int64_t rows,
                                                                double* __restrict__ flux,
                                                                double* __restrict__ sums) {
-  const int lane = threadIdx.x & 63;
-  for (int s = blockIdx.x * FLUX_WAVES + flux_wave(); s < sk.n; s += gridDim.x * FLUX_WAVES) {
+  constexpr int S = FLUX_WAVES / W;
+  __shared__ double part[FLUX_WAVES];
+  const int lane = threadIdx.x % (64 * W), w = flux_wave();
+  for (int s0 = blockIdx.x * S; s0 < sk.n; s0 += gridDim.x * S) {
+    const int s = s0 + w / W;
     double v[4] = {0.0, 0.0, 0.0, 0.0};
-    if (eta)
-      flux_jac_skewer<true>(sk, s, delta, eta, abcg, rows, flux, lane, v);
-    else
-      flux_jac_skewer<false>(sk, s, delta, eta, abcg, rows, flux, lane, v);
+    if (s < sk.n) {
+      if (eta)
+        flux_jac_skewer<W, true>(sk, s, delta, eta, abcg, rows, flux, lane, v);
+      else
+        flux_jac_skewer<W, false>(sk, s, delta, eta, abcg, rows, flux, lane, v);
+    }
 #pragma unroll
-    for (int k = 0; k < 4; ++k) v[k] = wave_sum(v[k]);
-    if (lane == 0) {
+    for (int k = 0; k < 4; ++k) v[k] = skewer_sum<W>(v[k], w, lane, part);
+    if (lane == 0 && s < sk.n) {
 #pragma unroll
       for (int k = 0; k < 4; ++k) sums[(int64_t)s * 4 + k] = v[k];
     }
@@ -2013,8 +2054,14 @@ extern "C" int smk_fgpa_flux(const smk_skewers* sk, const float* delta, const fl
   SMK_REQUIRE(sk != nullptr && delta != nullptr && abcg != nullptr && flux != nullptr && fsum != nullptr,
               SMK_ERR_ARG, "NULL argument");
   if (sk->n <= 0) return SMK_OK;
-  hipLaunchKernelGGL(k_fgpa_flux, dim3(grid_for_waves(sk->n)), dim3(FIT_THREADS), 0, (hipStream_t)stream, *sk, delta,
-                     eta, abcg, abcg_rows, flux, fsum);
+  const int w = flux_waves(*sk);
+#define SMK_FLUX(W)                                                                                            \
+  hipLaunchKernelGGL(k_fgpa_flux<W>, dim3(grid_for_waves(sk->n, W)), dim3(FIT_THREADS), 0, (hipStream_t)stream, \
+                     *sk, delta, eta, abcg, abcg_rows, flux, fsum)
+  if (w == 8) SMK_FLUX(8);
+  else if (w == 2) SMK_FLUX(2);
+  else SMK_FLUX(1);
+#undef SMK_FLUX
   SMK_LAUNCH_CHECK();
   return SMK_OK;
 }
@@ -2206,8 +2253,14 @@ extern "C" int smk_fgpa_flux_jac(const smk_skewers* sk, const float* delta, cons
               SMK_ERR_ARG, "NULL argument");
   SMK_REQUIRE(sk->pset != nullptr, SMK_ERR_ARG, "the fit kernels need skewers.pset");
   if (sk->n <= 0) return SMK_OK;
-  hipLaunchKernelGGL(k_fgpa_flux_jac, dim3(grid_for_waves(sk->n)), dim3(FIT_THREADS), 0, (hipStream_t)stream, *sk,
-                     delta, eta, abcg, abcg_rows, flux, sums);
+  const int w = flux_waves(*sk);   // as smk_fgpa_flux: the sums of F are its bits
+#define SMK_FLUX(W)                                                                                                \
+  hipLaunchKernelGGL(k_fgpa_flux_jac<W>, dim3(grid_for_waves(sk->n, W)), dim3(FIT_THREADS), 0, (hipStream_t)stream, \
+                     *sk, delta, eta, abcg, abcg_rows, flux, sums)
+  if (w == 8) SMK_FLUX(8);
+  else if (w == 2) SMK_FLUX(2);
+  else SMK_FLUX(1);
+#undef SMK_FLUX
   SMK_LAUNCH_CHECK();
   return SMK_OK;
 }
