@@ -927,23 +927,16 @@ __global__ __launch_bounds__(256) void k_gather_plane_tri(GatherArgs a) {
 // Re, Im ~ N(0, M); k = 0 and k = M are real with variance 2M.  M/2 Philox
 // calls per skewer (counter c), each two Box-Muller pairs: call 0 gives
 // modes 0 and M (the first pair, one normal each) and mode 1 (the second);
-// call c >= 1 gives modes 2c (first pair) and 2c + 1 (second pair).
+// call c >= 1 gives modes 2c (first pair) and 2c + 1 (second pair).  The fold
+// for the C2R transform pairs k with M - k, so the modes pass through LDS:
+// drawn where they are used, every call was made four times (600 skewers of
+// 8192 points: 33 us, now 26, a block's chain of draws and FFT stages; with 512
+// or 1024 threads to a line instead of 256 the call takes 47 and 52 us
+// against 44, and 229 and 294 against 186 for 10000 skewers).
 constexpr uint32_t MP_TAG = 0x6d697373u;
 
 __device__ __forceinline__ U4 mp_call(uint64_t seed, uint64_t id, int c) {
   return philox4x32_10_c4((uint32_t)c, (uint32_t)id, (uint32_t)(id >> 32), MP_TAG, seed);
-}
-
-__device__ __forceinline__ float2 mp_mode(uint64_t seed, uint64_t id, int k, int M, const float* __restrict__ filt) {
-  const int c = (k == M || k == 1) ? 0 : k >> 1;
-  const U4 u = mp_call(seed, id, c);
-  float n0, n1;
-  if (k == 0 || k == M || (k & 1) == 0) box_muller_hw(u.x, u.y, n0, n1);
-  else box_muller_hw(u.z, u.w, n0, n1);
-  if (k == 0) return make_float2(n0 * sqrtf(2.0f * M) * filt[k], 0.0f);
-  if (k == M) return make_float2(n1 * sqrtf(2.0f * M) * filt[k], 0.0f);
-  const float sm = sqrtf((float)M) * filt[k];
-  return make_float2(n0 * sm, n1 * sm);
 }
 
 template <int M, int T>
@@ -972,16 +965,36 @@ __global__ __launch_bounds__(T* (M / elems_per_thread(M))) void k_missing_power(
   float2 v[E];
   if (noise == nullptr) {
     const uint64_t id = sk.noise_id ? sk.noise_id[s] : (uint64_t)s;
+    // the modes into the line, each from one Philox call of its pair: k at
+    // line[k], and the two real ones, k = 0 and M, as line[0]
+    const float sr = sqrtf((float)M), s2 = sqrtf(2.0f * M);
+#pragma unroll
+    for (int h = 0; h < E / 2; ++h) {
+      const int c = p + P * h;
+      const U4 u = mp_call(seed, id, c);
+      float n0, n1, n2, n3;
+      box_muller_hw(u.x, u.y, n0, n1);
+      box_muller_hw(u.z, u.w, n2, n3);
+      const float f0 = filt[2 * c] * (c == 0 ? s2 : sr), f0i = c == 0 ? filt[M] * s2 : f0, f1 = filt[2 * c + 1] * sr;
+      line[2 * c] = make_float2(n0 * f0, n1 * f0i);
+      line[2 * c + 1] = make_float2(n2 * f1, n3 * f1);
+    }
+    __syncthreads();
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       const int k = p + P * e;
-      const float2 yk = mp_mode(seed, id, k, M, filt);
-      const float2 yc = cconj(mp_mode(seed, id, M - k, M, filt));
+      float2 yk = line[k];
+      float2 yc = cconj(line[(M - k) % M]);
+      if (k == 0) {
+        yc = make_float2(yk.y, 0.0f);
+        yk.y = 0.0f;
+      }
       const float2 sm = cadd(yk, yc);
       const float2 d = csub(yk, yc);
       const float2 wd = cmul(cconj(twr[k]), d);
       v[e] = make_float2(sm.x - wd.y, sm.y + wd.x);
     }
+    __syncthreads();
   } else {
     // forward R2C of the fed noise, times the filter, then the C2R pre-step
     const float2* src = reinterpret_cast<const float2*>(noise + (valid ? noise_off[s] : 0));
@@ -1142,7 +1155,7 @@ __device__ __forceinline__ void step_missing_power(const StepArgs& a, int s, int
   const int tid = threadIdx.x;
   const float* __restrict__ filt = a.filt + a.foff[C] + (a.fset ? (int64_t)a.fset[s] * a.set_stride : 0);
   const uint64_t id = a.sk.noise_id ? a.sk.noise_id[s] : (uint64_t)s;
-  // (1) modes k = 0..M: M/2 Philox calls (see mp_mode)
+  // (1) modes k = 0..M: M/2 Philox calls (see mp_call)
   const float sr = sqrtf((float)M), s2 = sqrtf(2.0f * M);
   // a compile-time trip count, so that the filter loads of every pass are
   // issued together ahead of the Philox rounds
@@ -1462,9 +1475,9 @@ template <int M>
 hipError_t launch_mp(const smk_skewers& sk, const int32_t* list, const int32_t* count, const float* filt,
                      const int32_t* fset, int64_t set_stride, const float* scale, uint64_t seed,
                      const uint64_t* seed_dev, const float* noise, const int64_t* noise_off, const float2* tw,
-                     const float2* twr, float* delta_s, hipStream_t s) {
+                     const float2* twr, float* delta_s, int n, hipStream_t s) {
   constexpr int T = mp_T(M);
-  const int nblk = (sk.n + T - 1) / T;
+  const int nblk = (n + T - 1) / T;
   if (nblk == 0) return hipSuccess;
   hipLaunchKernelGGL((k_missing_power<M, T>), dim3(nblk), dim3(T * (M / elems_per_thread(M))), 0, s, sk, list,
                      count, filt, fset, set_stride, scale, seed, seed_dev, noise, noise_off, tw, twr, delta_s);
@@ -1659,19 +1672,25 @@ extern "C" int smk_forest_missing_power_sets(smk_forest_plan* plan, const smk_sk
                      counts + N_CLASS);
   SMK_LAUNCH_CHECK();
   const int64_t* foff = filt_off;
+  // skewers per class: a class with none is not launched (600 skewers of one
+  // class: 89 us with all six launches, 44 with the one); in graph mode they
+  // are not known here
+  int32_t have[N_CLASS + 1];
+  for (int c = 0; c < N_CLASS; ++c) have[c] = sk->n;
   if (plan->seed_dev == nullptr) {
     // (in graph mode the batch was checked by an eager call; a skewer that
     // fails the checks is left out of every class list and gets no delta_s)
-    int32_t bad = 0;
-    SMK_HIP_CHECK(hipMemcpyAsync(&bad, counts + N_CLASS, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+    SMK_HIP_CHECK(hipMemcpyAsync(have, counts, sizeof(have), hipMemcpyDeviceToHost, s));
     SMK_HIP_CHECK(hipStreamSynchronize(s));
+    const int32_t bad = have[N_CLASS];
     SMK_REQUIRE((bad & 2) == 0, SMK_ERR_RANGE, "a filter set index is outside [0, %d)", (int)n_sets);
     SMK_REQUIRE(bad == 0, SMK_ERR_RANGE, "a skewer needs an FFT longer than %d", 256 << (N_CLASS - 1));
   }
   const int64_t stride = filt_set ? set_stride : 0;
 #define SMK_MP(C, M)                                                                                            \
   SMK_HIP_CHECK(launch_mp<M>(*sk, lists + (int64_t)C * sk->n, counts + C, filt + foff[C], filt_set, stride,     \
-                             scale, seed, plan->seed_dev, noise, noise_off, plan->tw[C], plan->twr[C], delta_s, s))
+                             scale, seed, plan->seed_dev, noise, noise_off, plan->tw[C], plan->twr[C], delta_s,   \
+                             have[C], s))
   SMK_MP(0, 128);
   SMK_MP(1, 256);
   SMK_MP(2, 512);
