@@ -108,6 +108,77 @@ template <bool INV> struct DFT<16, INV> {
   }
 };
 
+// the DFT of R points of which the upper half is 0 (those entries of a are
+// not read): the first stage of a transform of zero-padded input
+template <int R, bool INV> struct DFTHalf;
+template <bool INV> struct DFTHalf<4, INV> {
+  static __device__ __forceinline__ void run(double2* a) {
+    const double2 u = a[0], v = a[1], w = mul_mi<INV>(a[1]);
+    a[0] = cadd(u, v);
+    a[1] = cadd(u, w);
+    a[2] = csub(u, v);
+    a[3] = csub(u, w);
+  }
+};
+template <bool INV> struct DFTHalf<8, INV> {
+  static __device__ __forceinline__ void run(double2* a) {
+    const double r = 0.70710678118654752440084436210484904;
+    double2 e[4] = {a[0], a[2]};
+    double2 o[4] = {a[1], a[3]};
+    DFTHalf<4, INV>::run(e);
+    DFTHalf<4, INV>::run(o);
+    double2 o1, o3;
+    if (INV) {
+      o1 = make_double2(r * (o[1].x - o[1].y), r * (o[1].x + o[1].y));
+      o3 = make_double2(-r * (o[3].x + o[3].y), r * (o[3].x - o[3].y));
+    } else {
+      o1 = make_double2(r * (o[1].x + o[1].y), r * (o[1].y - o[1].x));
+      o3 = make_double2(r * (o[3].y - o[3].x), -r * (o[3].x + o[3].y));
+    }
+    const double2 o2 = mul_mi<INV>(o[2]);
+    a[0] = cadd(e[0], o[0]);
+    a[4] = csub(e[0], o[0]);
+    a[1] = cadd(e[1], o1);
+    a[5] = csub(e[1], o1);
+    a[2] = cadd(e[2], o2);
+    a[6] = csub(e[2], o2);
+    a[3] = cadd(e[3], o3);
+    a[7] = csub(e[3], o3);
+  }
+};
+template <bool INV> struct DFTHalf<16, INV> {
+  static __device__ __forceinline__ void run(double2* a) {
+    const double c1 = 0.92387953251128675612818318939678829;  // cos(pi/8)
+    const double s1 = 0.38268343236508977172845998403039887;  // sin(pi/8)
+    const double h = 0.70710678118654752440084436210484904;
+    double2 t[4][4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      double2 u[4] = {a[q], a[q + 4]};
+      DFTHalf<4, INV>::run(u);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) t[q][r] = u[r];
+    }
+    const double sg = INV ? 1.0 : -1.0;
+    const double2 w[4][4] = {
+        {{1, 0}, {1, 0}, {1, 0}, {1, 0}},
+        {{1, 0}, {c1, sg * s1}, {h, sg * h}, {s1, sg * c1}},
+        {{1, 0}, {h, sg * h}, {0, sg}, {-h, sg * h}},
+        {{1, 0}, {s1, sg * c1}, {-h, sg * h}, {-c1, -sg * s1}}};
+#pragma unroll
+    for (int q = 1; q < 4; ++q)
+#pragma unroll
+      for (int r = 1; r < 4; ++r) t[q][r] = cmul(t[q][r], w[q][r]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      double2 u[4] = {t[0][r], t[1][r], t[2][r], t[3][r]};
+      DFT<4, INV>::run(u);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) a[r + 4 * q] = u[q];
+    }
+  }
+};
+
 // radix of stage S of an M-point FFT with E points per thread: the largest
 // of 16, 8, 4, 2 dividing both E and what remains of M
 __host__ __device__ constexpr int stage_radix(int M, int E, int S) {
@@ -178,8 +249,9 @@ __device__ __forceinline__ void stage_twiddles(double2 (&w)[E / R][R], int p, co
 // Stockham stage: butterfly j = p + P b takes points j + r M/R (register
 // slots b + r B), multiplies point r by w[b][r] (stage_twiddles; none for
 // Ns = 1), outputs to points (j / Ns) Ns R + j % Ns + r Ns (the last stage
-// keeps them in registers: slot b + r B holds point j + r M/R).
-template <int M, int E, int R, int Ns, bool INV, bool LAST>
+// keeps them in registers: slot b + r B holds point j + r M/R).  HALF: the
+// upper half of the points is 0.
+template <int M, int E, int R, int Ns, bool INV, bool LAST, bool HALF = false>
 __device__ __forceinline__ void stage(double2 (&v)[E], double2* __restrict__ line, int p,
                                       const double2 (&w)[E / R][R]) {
   constexpr int P = M / E;
@@ -189,12 +261,13 @@ __device__ __forceinline__ void stage(double2 (&v)[E], double2* __restrict__ lin
     const int j = p + P * b;
     double2 a[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) a[r] = v[b + r * B];
+    for (int r = 0; r < (HALF ? R / 2 : R); ++r) a[r] = v[b + r * B];
     if (Ns > 1) {
 #pragma unroll
       for (int r = 1; r < R; ++r) a[r] = cmul(a[r], w[b][r]);
     }
-    DFT<R, INV>::run(a);
+    if constexpr (HALF) DFTHalf<R, INV>::run(a);
+    else DFT<R, INV>::run(a);
     if (LAST) {
 #pragma unroll
       for (int r = 0; r < R; ++r) v[b + r * B] = a[r];
@@ -209,7 +282,7 @@ __device__ __forceinline__ void stage(double2 (&v)[E], double2* __restrict__ lin
 // The stages from S on; w holds stage S's twiddles.  The next stage's
 // twiddles are loaded before the exchange's barriers, so that their latency
 // overlaps the exchange.
-template <int M, int E, bool INV, int S, int Ns>
+template <int M, int E, bool INV, int S, int Ns, bool HALF = false>
 __device__ __forceinline__ void stages(double2 (&v)[E], double2* __restrict__ line, int p,
                                        const double2* __restrict__ twM, int TW,
                                        const double2 (&w)[E / stage_radix(M, E, S)][stage_radix(M, E, S)]) {
@@ -219,7 +292,7 @@ __device__ __forceinline__ void stages(double2 (&v)[E], double2* __restrict__ li
   if constexpr (S < NS) {
     constexpr int R = stage_radix(M, E, S);
     constexpr bool LAST = S + 1 == NS;
-    stage<M, E, R, Ns, INV, LAST>(v, line, p, w);
+    stage<M, E, R, Ns, INV, LAST, HALF>(v, line, p, w);
     if constexpr (!LAST) {
       constexpr int R1 = stage_radix(M, E, S + 1);
       double2 w1[E / R1][R1];
@@ -235,13 +308,14 @@ __device__ __forceinline__ void stages(double2 (&v)[E], double2* __restrict__ li
 
 // In-register FFT of one M-point line over the M / E threads p of the block
 // (every thread of the block must call it: it holds block barriers).  On
-// entry and exit thread p holds points p + P e.  Unnormalised.
-template <int M, int E, bool INV>
+// entry and exit thread p holds points p + P e.  Unnormalised.  HALF: the
+// points from M / 2 on are 0 (their entries of v are not read).
+template <int M, int E, bool INV, bool HALF = false>
 __device__ __forceinline__ void fft(double2 (&v)[E], double2* __restrict__ line, int p,
                                     const double2* __restrict__ twM, int TW) {
   constexpr int R0 = stage_radix(M, E, 0);
   double2 w0[E / R0][R0];   // stage 0 has Ns = 1: no twiddles
-  stages<M, E, INV, 0, 1>(v, line, p, twM, TW, w0);
+  stages<M, E, INV, 0, 1, HALF>(v, line, p, twM, TW, w0);
 }
 
 // w_n = exp(-i pi n^2 / N), n^2 mod 2N exact (n < 2^31 / N)
@@ -333,24 +407,25 @@ __device__ __forceinline__ void bluestein_table(int N, double2* __restrict__ T, 
 
 // Bluestein with the chirp w (N values) and FFT_M(b) / M (M values) read
 // from a table made once per length (bluestein_table): one register tile,
-// two transforms.  in(n) may read LDS that `line` aliases (all of it is read
-// before the first exchange); emit may write there too (the line is free
-// once the last transform's final stage runs in registers).
+// two transforms, X_k of k = p + (M / E) e < N at x[e] of thread p.  in(n) may
+// read LDS that `line` aliases (all of it is read before the first exchange);
+// the line is free once the last transform's final stage runs in registers.
 // KEEP bit 0: the chirp's transform is loaded before the first FFT (its
 // latency overlaps that FFT); bit 1: the chirp is kept from the input for
-// the output.  2 E more registers each, for kernels whose occupancy does not
-// drop by them.
-constexpr int KEEP_B = 1, KEEP_W = 2;
-template <int M, int E, int KEEP = 0, class In, class Emit>
-__device__ __forceinline__ void bluestein_tab(int N, int nout, In in, Emit emit, double2* __restrict__ line,
-                                              const double2* __restrict__ twM, int TW,
-                                              const double2* __restrict__ wtab, const double2* __restrict__ btab) {
-  constexpr int P = M / E;
+// the output.  4 E and 2 E more registers, for kernels whose occupancy does
+// not drop by them.  LATE_B: no load of the chirp's transform is moved ahead
+// of the first FFT's end, where the registers are the kernel's most.
+constexpr int KEEP_B = 1, KEEP_W = 2, LATE_B = 4;
+// (the general form: x before the multiplication by w, wk the chirp if kept)
+template <int M, int E, int KEEP, class In>
+__device__ __forceinline__ void bluestein_core(double2 (&va)[E], double2 (&wk)[E / 2], int N, In in,
+                                               double2* __restrict__ line, const double2* __restrict__ twM, int TW,
+                                               const double2* __restrict__ wtab, const double2* __restrict__ btab) {
+  constexpr int P = M / E, H = E / 2;   // N <= M / 2: points of the lower half only, in and out
   const int p = threadIdx.x;
-  double2 va[E];
-  [[maybe_unused]] double2 wk[E], bk[E];
+  [[maybe_unused]] double2 bk[E];
 #pragma unroll
-  for (int e = 0; e < E; ++e) {
+  for (int e = 0; e < H; ++e) {
     const int n = p + P * e;
     if constexpr ((KEEP & KEEP_W) != 0) {
       wk[e] = n < N ? wtab[n] : make_double2(0.0, 0.0);
@@ -364,13 +439,36 @@ __device__ __forceinline__ void bluestein_tab(int N, int nout, In in, Emit emit,
     for (int e = 0; e < E; ++e) bk[e] = btab[p + P * e];
   }
   __syncthreads();
-  fft<M, E, false>(va, line, p, twM, TW);
+  fft<M, E, false, true>(va, line, p, twM, TW);
+  if constexpr ((KEEP & LATE_B) != 0) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int e = 0; e < E; ++e) va[e] = cmul(va[e], (KEEP & KEEP_B) ? bk[e] : btab[p + P * e]);
   fft<M, E, true>(va, line, p, twM, TW);
+}
+
+template <int M, int E, int KEEP = 0, class In>
+__device__ __forceinline__ void bluestein_regs(double2 (&x)[E / 2], int N, In in, double2* __restrict__ line,
+                                               const double2* __restrict__ twM, int TW,
+                                               const double2* __restrict__ wtab, const double2* __restrict__ btab) {
+  double2 va[E], wk[E / 2];
+  bluestein_core<M, E, KEEP>(va, wk, N, in, line, twM, TW, wtab, btab);
 #pragma unroll
-  for (int e = 0; e < E; ++e) {
-    const int k = p + P * e;
+  for (int e = 0; e < E / 2; ++e) {
+    const int k = (int)threadIdx.x + M / E * e;
+    x[e] = cmul(va[e], (KEEP & KEEP_W) ? wk[e] : wtab[k < N ? k : N - 1]);
+  }
+}
+
+// bluestein_regs, then emit(k, X_k) for k < nout (nout <= N)
+template <int M, int E, int KEEP = 0, class In, class Emit>
+__device__ __forceinline__ void bluestein_tab(int N, int nout, In in, Emit emit, double2* __restrict__ line,
+                                              const double2* __restrict__ twM, int TW,
+                                              const double2* __restrict__ wtab, const double2* __restrict__ btab) {
+  double2 va[E], wk[E / 2];
+  bluestein_core<M, E, KEEP>(va, wk, N, in, line, twM, TW, wtab, btab);
+#pragma unroll
+  for (int e = 0; e < E / 2; ++e) {
+    const int k = (int)threadIdx.x + M / E * e;
     if (k < nout) emit(k, cmul(va[e], (KEEP & KEEP_W) ? wk[e] : wtab[k]));
   }
 }

@@ -735,11 +735,25 @@ __global__ __launch_bounds__(M / 8) __attribute__((amdgpu_waves_per_eu(2))) void
   }
 }
 
-// LDS of k_p1d_blue_pair<M>: the line, the two forests' pk (NJ each,
-// NJ = M/4 + 1 >= N/2 + 1), the bins, then the edges and the bin runs
-__host__ __device__ constexpr size_t pair_fixed_bytes(int M) {
-  return blue_line_bytes_m(M) + (size_t)(M / 4 + 1) * 16 + (size_t)(((M / 4 + 1) + 1) & ~1) * 4;
-}
+// LDS of k_p1d_blue_pair<M>: the line, and in it past the outputs (N <= M/2)
+// the two forests' pk (NJ each, NJ = M/4 + 1 >= N/2 + 1) and the bins; then
+// the edges and the bin runs
+__host__ __device__ constexpr size_t pair_fixed_bytes(int M) { return blue_line_bytes_m(M); }
+// Points per thread of k_p1d_blue_pair<M>.  One block of 512 threads fills a
+// CU's registers at M = 4096, which leaves every barrier and load bare; with
+// 16 points on 256 threads two blocks fit, and an FFT has three stages instead
+// of four.  10000 pairs of 1025 to 1500 points: the forward pass 794 -> 660 us;
+// M = 2048 takes 390 either way (513 to 1020 points), 428 before with its pk
+// outside the line.
+constexpr int pair_E(int M) { return M == 4096 ? 16 : 8; }
+// The same of k_p1d_adjoint_blue_pair<M>, and what it keeps in registers.  The
+// FGPA part on the transform's registers instead of x and A in LDS (100 KB at
+// M = 4096, one block per CU; two passes over the pixels and two reductions):
+// with the forward pass 10000 pairs of 1025 to 1500 points 1916 -> 1505 us, of
+// 513 to 1020 1048 -> 900.  M = 4096 with 8 points and all kept: 1610; M = 2048
+// with 16: as with 8.
+constexpr int adj_pair_E(int M) { return M == 4096 ? 16 : 8; }
+constexpr int adj_pair_keep(int M) { return f64::KEEP_W | (M == 4096 ? f64::LATE_B : f64::KEEP_B); }
 
 // The members (s1, s2) of pair w that take M's size class: each must still
 // have a table of this size class, the second one of the same length and
@@ -829,15 +843,17 @@ __device__ __forceinline__ void desc_members(const Args& a, const PairDesc& d, i
 // b takes pairs pair_lo + b + k gridDim.x, with the members' descriptors
 // loaded a pair ahead and the pair list entry two pairs ahead.
 template <int M>
-__global__ __launch_bounds__(M / 8) __attribute__((amdgpu_waves_per_eu(2))) void k_p1d_blue_pair(P1dArgs a) {
-  constexpr int NT = M / 8;
+__global__ __launch_bounds__(M / pair_E(M)) __attribute__((amdgpu_waves_per_eu(2))) void k_p1d_blue_pair(P1dArgs a) {
+  constexpr int E = pair_E(M), NT = M / E;
   constexpr int NJ = M / 4 + 1;
+  static_assert((size_t)(f64::line_len(M) - M / 2) * 16 >= (size_t)NJ * 16 + (size_t)(NJ + 1) * 4,
+                "a pair's pk and bins must fit past the outputs in the line");
   extern __shared__ double dyn[];
   double2* line = reinterpret_cast<double2*>(dyn);
-  double* pk1 = reinterpret_cast<double*>(reinterpret_cast<char*>(dyn) + blue_line_bytes_m(M));
+  double* pk1 = reinterpret_cast<double*>(line + M / 2);
   double* pk2 = pk1 + NJ;
   int* bins = reinterpret_cast<int*>(pk2 + NJ);
-  double* ledges = reinterpret_cast<double*>(bins + ((NJ + 1) & ~1));
+  double* ledges = reinterpret_cast<double*>(reinterpret_cast<char*>(dyn) + pair_fixed_bytes(M));
   int* bfirst = reinterpret_cast<int*>(ledges + a.nb + 1);
   int* blast = bfirst + a.nb;
   for (int i = threadIdx.x; i <= a.nb; i += NT) ledges[i] = a.edges[i];
@@ -878,7 +894,7 @@ __global__ __launch_bounds__(M / 8) __attribute__((amdgpu_waves_per_eu(2))) void
     const double inv2 = s2 >= 0 ? 1.0 / a.fmean[set2] : 0.0;
     const int nj = nq / 2 + 1;
     const double2* T = a.tables + tb;
-    f64::bluestein_tab<M, 8, (M >= 4096 ? f64::KEEP_B | f64::KEEP_W : 0)>(
+    f64::bluestein_tab<M, E>(
         nq, nq,
         [&](int q) {
           double acc1 = 0.0, acc2 = 0.0;
@@ -1380,19 +1396,18 @@ __global__ __launch_bounds__(M / 8) __attribute__((amdgpu_waves_per_eu(2))) void
 // Hermitian spectrum H (H_0 = Re c_0, H_j = c_j / 2 and H_{N-j} = conj(c_j)
 // / 2 for 0 < j < N/2, H_{N/2} = Re c_{N/2} for even N), a real sequence, so
 // the DFT of H1 + i H2 is A1 + i A2.  Without saved modes, X1 and X2 come from
-// one DFT of delta_F1 + i delta_F2 as in k_p1d_blue_pair.  LDS: x1, x2 (M/2
-// doubles each), the line (c1 and c2 over its start), the edges.
+// one DFT of delta_F1 + i delta_F2 as in k_p1d_blue_pair.  The FGPA part
+// (adj_fgpa) of both forests runs on the registers that hold A, with one block
+// reduction of fourteen sums.  LDS: the line (c1 and c2 over its start), the
+// edges.
 template <int M>
-__global__ __launch_bounds__(M / 8) __attribute__((amdgpu_waves_per_eu(2))) void k_p1d_adjoint_blue_pair(
+__global__ __launch_bounds__(M / adj_pair_E(M)) __attribute__((amdgpu_waves_per_eu(2))) void k_p1d_adjoint_blue_pair(
     AdjArgs a) {
-  constexpr int NT = M / 8;
+  constexpr int E = adj_pair_E(M), NT = M / E;
   extern __shared__ double dyn[];
-  double* x1 = dyn;
-  double* x2 = dyn + M / 2;
-  double2* line = reinterpret_cast<double2*>(reinterpret_cast<char*>(dyn) + 2 * adj_blue_x_bytes(M));
-  double* ledges = reinterpret_cast<double*>(reinterpret_cast<char*>(dyn) + 2 * adj_blue_x_bytes(M) +
-                                             blue_line_bytes_m(M));
-  __shared__ double red[7 * (NT / 64)];
+  double2* line = reinterpret_cast<double2*>(dyn);
+  double* ledges = reinterpret_cast<double*>(reinterpret_cast<char*>(dyn) + blue_line_bytes_m(M));
+  __shared__ double red[14 * (NT / 64)], sums[14];
   for (int i = threadIdx.x; i <= a.nb; i += NT) ledges[i] = a.edges[i];
   const smk_skewers& sk = a.sk;
   const int m = a.regroup;
@@ -1429,11 +1444,13 @@ __global__ __launch_bounds__(M / 8) __attribute__((amdgpu_waves_per_eu(2))) void
     const bool two = s2 >= 0;
     const int nq = nf1 / m;
     const int nj = nq / 2 + 1;
-    const double fm1 = a.fmean[set1], fm2 = a.fmean[set2];
     __syncthreads();
-    load_delta_f<NT>(a.flux, o1, 0, nf1, m, 1.0 / fm1, x1);
-    if (two) load_delta_f<NT>(a.flux, o2, 0, nf2, m, 1.0 / fm2, x2);
-    __syncthreads();
+    // F of regrouped point q of the forest at o: the mean of its m pixels
+    const auto point = [&](int64_t o, int q) {
+      double acc = 0.0;
+      for (int r = 0; r < m; ++r) acc += a.flux[o + (int64_t)q * m + r];
+      return acc / m;
+    };
     const double* gp1 = a.gp + (int64_t)set1 * a.nb;
     const double* gp2 = a.gp + (int64_t)set2 * a.nb;
     const double2* T = a.tables + tb;
@@ -1457,8 +1474,11 @@ __global__ __launch_bounds__(M / 8) __attribute__((amdgpu_waves_per_eu(2))) void
         c2[j] = cc;
       }
     } else {
-      f64::bluestein_tab<M, 8>(nq, nq, [&](int n) { return make_double2(x1[n], two ? x2[n] : 0.0); },
-                               [&](int j, double2 Z) { line[j] = Z; }, line, a.tw, BLUE_MMAX, T, T + nq);
+      const double inv1 = 1.0 / a.fmean[set1], inv2 = 1.0 / a.fmean[set2];
+      f64::bluestein_tab<M, E>(
+          nq, nq,
+          [&](int n) { return make_double2(point(o1, n) * inv1 - 1.0, two ? point(o2, n) * inv2 - 1.0 : 0.0); },
+          [&](int j, double2 Z) { line[j] = Z; }, line, a.tw, BLUE_MMAX, T, T + nq);
       __syncthreads();
       // the split reads line[j] and line[N - j]: into registers first, then
       // the block writes c1, c2 over the line's start
@@ -1495,25 +1515,78 @@ __global__ __launch_bounds__(M / 8) __attribute__((amdgpu_waves_per_eu(2))) void
       const double2 v = c[nq - n];
       return make_double2(0.5 * v.x, -0.5 * v.y);
     };
-    double saf1 = 0.0, saf2 = 0.0;
-    f64::bluestein_tab<M, 8, f64::KEEP_B | f64::KEEP_W>(
-        nq, nq,
+    double2 Z[E / 2];   // A of both forests at q = threadIdx.x + NT e
+    f64::bluestein_regs<M, E, adj_pair_keep(M)>(
+        Z, nq,
         [&](int n) {
           const double2 h1 = herm(c1, n), h2 = herm(c2, n);
           return make_double2(h1.x - h2.y, h1.y + h2.x);   // H1 + i H2
         },
-        [&](int q, double2 Z) {
-          saf1 += Z.x * (x1[q] + 1.0) * fm1;
-          x1[q] = Z.x;
-          if (two) {
-            saf2 += Z.y * (x2[q] + 1.0) * fm2;
-            x2[q] = Z.y;
-          }
-        },
         line, a.tw, BLUE_MMAX, T, T + nq);
-    __syncthreads();
-    adj_fgpa<NT>(a, set1, o1, nf1, nq, saf1, x1, red, a.out + (int64_t)s1 * 7);
-    if (two) adj_fgpa<NT>(a, set2, o2, nf2, nq, saf2, x2, red, a.out + (int64_t)s2 * 7);
+    // the FGPA part (adj_fgpa) of both forests where A is, in registers: seven
+    // sums each
+    double v[14];
+#pragma unroll
+    for (int k = 0; k < 14; ++k) v[k] = 0.0;
+    const double4 pr1 = prow(a.abcg, a.rows, set1), pr2 = prow(a.abcg, a.rows, set2);
+    const float* ep = a.eta ? a.eta : a.delta;
+    const auto pixel = [&](double* s, const double4& p, float dv, float ev, double F, double Aq) {
+      const double e = a.eta ? (double)ev : 0.0;
+      const double gf = (double)dv + p.z * e;
+      const double T1 = exp(p.y * p.w * gf);
+      const double dfa = -T1 * F, dfb = -p.x * T1 * F * p.w * gf, dfc = -p.x * T1 * F * p.y * p.w * e;
+      s[4] += dfa; s[5] += dfb; s[6] += dfc;
+      s[1] += Aq * dfa; s[2] += Aq * dfb; s[3] += Aq * dfc;
+    };
+    if (m == 1) {
+      // a pixel per point: the loads of all points together, at a clamped
+      // index past the end
+      float dv[2][E / 2], ev[2][E / 2];
+      double fv[2][E / 2];
+      const int64_t o2c = two ? o2 : o1;
+#pragma unroll
+      for (int e = 0; e < E / 2; ++e) {
+        const int q = (int)threadIdx.x + NT * e, i = q < nq ? q : nq - 1;
+        dv[0][e] = a.delta[o1 + i];
+        ev[0][e] = ep[o1 + i];
+        fv[0][e] = a.flux[o1 + i];
+        dv[1][e] = a.delta[o2c + i];
+        ev[1][e] = ep[o2c + i];
+        fv[1][e] = a.flux[o2c + i];
+      }
+#pragma unroll
+      for (int e = 0; e < E / 2; ++e) {
+        if ((int)threadIdx.x + NT * e < nq) {
+          v[0] += Z[e].x * fv[0][e];
+          v[7] += Z[e].y * fv[1][e];
+          pixel(v, pr1, dv[0][e], ev[0][e], fv[0][e], Z[e].x);
+          pixel(v + 7, pr2, dv[1][e], ev[1][e], fv[1][e], Z[e].y);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < E / 2; ++e) {
+        const int q = (int)threadIdx.x + NT * e;
+        if (q < nq) {
+          for (int r = 0; r < m; ++r) {
+            const int64_t i = (int64_t)q * m + r;
+            pixel(v, pr1, a.delta[o1 + i], ep[o1 + i], a.flux[o1 + i], Z[e].x / m);
+            if (two) pixel(v + 7, pr2, a.delta[o2 + i], ep[o2 + i], a.flux[o2 + i], Z[e].y / m);
+          }
+          v[0] += Z[e].x * point(o1, q);
+          if (two) v[7] += Z[e].y * point(o2, q);
+        }
+      }
+    }
+    // the pixels past the last whole point: no A
+    for (int i = nq * m + (int)threadIdx.x; i < nf1; i += NT)
+      pixel(v, pr1, a.delta[o1 + i], ep[o1 + i], a.flux[o1 + i], 0.0);
+    if (two)
+      for (int i = nq * m + (int)threadIdx.x; i < nf2; i += NT)
+        pixel(v + 7, pr2, a.delta[o2 + i], ep[o2 + i], a.flux[o2 + i], 0.0);
+    reduce_k<NT, 14>(v, red, sums);
+    if (threadIdx.x < 7) a.out[(int64_t)s1 * 7 + threadIdx.x] = sums[threadIdx.x];
+    else if (two && threadIdx.x < 14) a.out[(int64_t)s2 * 7 + threadIdx.x - 7] = sums[threadIdx.x];
   }
 }
 
@@ -1935,8 +2008,8 @@ int launch_p1d_blue_pair(P1dArgs a, int lo, int hi, size_t tail, hipStream_t st)
   a.pair_hi = hi;
   const size_t lds = pair_fixed_bytes(M) + tail;
   SMK_HIP_CHECK(hipFuncSetAttribute((const void*)k_p1d_blue_pair<M>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  const int grid = resident_grid((const void*)k_p1d_blue_pair<M>, M / 8, lds, hi - lo);
-  hipLaunchKernelGGL(k_p1d_blue_pair<M>, dim3(grid), dim3(M / 8), lds, st, a);
+  const int grid = resident_grid((const void*)k_p1d_blue_pair<M>, M / pair_E(M), lds, hi - lo);
+  hipLaunchKernelGGL(k_p1d_blue_pair<M>, dim3(grid), dim3(M / pair_E(M)), lds, st, a);
   SMK_LAUNCH_CHECK();
   return SMK_OK;
 }
@@ -1978,11 +2051,11 @@ int launch_adj_blue_pair(AdjArgs a, int lo, int hi, size_t tail, hipStream_t st)
   if (hi <= lo) return SMK_OK;
   a.pair_lo = lo;
   a.pair_hi = hi;
-  const size_t lds = 2 * adj_blue_x_bytes(M) + blue_line_bytes_m(M) + tail;
+  const size_t lds = blue_line_bytes_m(M) + tail;
   SMK_HIP_CHECK(hipFuncSetAttribute((const void*)k_p1d_adjoint_blue_pair<M>,
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  const int grid = resident_grid((const void*)k_p1d_adjoint_blue_pair<M>, M / 8, lds, hi - lo);
-  hipLaunchKernelGGL(k_p1d_adjoint_blue_pair<M>, dim3(grid), dim3(M / 8), lds, st, a);
+  const int grid = resident_grid((const void*)k_p1d_adjoint_blue_pair<M>, M / adj_pair_E(M), lds, hi - lo);
+  hipLaunchKernelGGL(k_p1d_adjoint_blue_pair<M>, dim3(grid), dim3(M / adj_pair_E(M)), lds, st, a);
   SMK_LAUNCH_CHECK();
   return SMK_OK;
 }
