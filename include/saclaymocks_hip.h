@@ -286,7 +286,7 @@ int smk_forest_plan_destroy(smk_forest_plan* plan);
 int smk_forest_plan_set_graph_mode(smk_forest_plan* plan, const uint64_t* seed_dev);
 /* Kernel instance of smk_forest_step for batches whose FFTs are at most 2048
  * points (the planner's choice, no counterpart in the reference): one wave
- * per skewer with at least 4 (0, the default) or 3 (1) waves per SIMD, two
+ * per skewer with at least 3 (0, the default) or 4 (1) waves per SIMD, two
  * waves per skewer with at least 4 (2) or 5 (3).  0 and 1 give the same
  * bits, as do 2 and 3; the two pairs transform the missing power with
  * different register tiles, so their delta_s and F differ by float32

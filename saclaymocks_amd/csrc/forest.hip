@@ -1116,6 +1116,7 @@ struct StepArgs {
   float* delta_s;
   int32_t* status;
   int32_t* queue;
+  int32_t n_static;      // skewers that go round the blocks ahead of the queue
   int32_t max_class;
   double hx, hy, hz;
   int32_t ctab_cap;      // z cells the per-skewer column table holds (0: no table)
@@ -1210,6 +1211,25 @@ __device__ __forceinline__ void step_missing_power(const StepArgs& a, int s, int
   __syncthreads();
 }
 
+constexpr int STEP_RUN = 4;   // skewers per queue slot
+
+// the block's skewer after s (see k_forest_step); the same value in every lane,
+// so scalar registers hold all per-skewer terms
+__device__ __forceinline__ int step_next(const StepArgs& a, int s, int& left, int q_next, int* s_next) {
+  __syncthreads();   // the LDS of this skewer is free
+  if (left > 0) {
+    --left;
+    return s + 1;
+  }
+  if (s < a.n_static && s + (int)gridDim.x < a.n_static) return s + (int)gridDim.x;
+  if (a.n_static >= a.sk.n) return a.sk.n;
+  if (threadIdx.x == 0) *s_next = q_next;
+  __syncthreads();
+  s = a.n_static + __builtin_amdgcn_readfirstlane(*s_next);
+  left = STEP_RUN - 1;
+  return s;
+}
+
 // MAXC: the longest length class of the batch (classes above it are
 // flagged); NT threads per block
 template <int MAXC, int NT, int OCC>
@@ -1225,18 +1245,16 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(OCC))) void 
   const float* __restrict__ fd = b.delta;
   const float* __restrict__ fe = b.eta[2];
   const double D = b.cell;
-  // the queue slot of the next skewer is taken while this one is processed
-  // (its atomic's latency overlaps the work); every slot goes to one block
-  int q_next = 0;
-  if (tid == 0) q_next = atomicAdd(a.queue, 1);
-  for (;;) {
-    if (tid == 0) s_next = q_next;
-    __syncthreads();
-    // the same value in every lane: scalar registers for all per-skewer terms
-    const int s = __builtin_amdgcn_readfirstlane(s_next);
-    __syncthreads();
-    if (s >= sk.n) break;
-    if (tid == 0) q_next = atomicAdd(a.queue, 1);
+  // Skewers [0, n_static) go round the blocks, the rest from a queue in runs
+  // of STEP_RUN; a run is taken while the block's skewer before it is
+  // processed (its atomic's latency overlaps the work) and goes to one block.
+  // The queue's atomics on one address take 11.7 ns each, so that with one
+  // per skewer they bounded the step: 200000 skewers took 2.34 ms at any length.
+  int s = (int)blockIdx.x, left = 0, q_next = 0;   // left: skewers of the run after s
+  for (; s < sk.n; s = step_next(a, s, left, q_next, &s_next)) {
+    // the last of a run, or of the static part: the next run
+    if (tid == 0 && left == 0 && s + (int)gridDim.x >= a.n_static && a.n_static < sk.n)
+      q_next = atomicAdd(a.queue, STEP_RUN);
     const int n = sk.npix[s];
     int c = 0;
     for (int nzc = 256; nzc < n + 50 && c < N_CLASS; nzc <<= 1) ++c;
@@ -1708,6 +1726,17 @@ extern "C" int smk_forest_missing_power(smk_forest_plan* plan, const smk_skewers
                                        workspace, delta_s, stream);
 }
 
+// Skewers that go round the blocks: 70% of a large batch, the queue evens out
+// the rest; all of a batch of few per block, where the queue's runs would be
+// the unevenness.  200000 skewers of 300 to 1500 pixels take 1071 us with 70%
+// and runs of 4, 1110 with 90% and 1218 with all, 1120 with runs of 2 and 1415
+// with runs of 1; 2394 with every skewer in the queue.  3000 to 30000: within
+// 3% of all round the blocks (205 us for 30000, 424 with every one queued).
+static int step_static(int n, int nblk) {
+  const int64_t rounds = n / nblk;
+  return rounds < 10 ? n : (int)(rounds * 7 / 10) * nblk;
+}
+
 extern "C" size_t smk_forest_step_workspace_bytes(void) { return 256; }
 
 extern "C" int smk_forest_step(smk_forest_plan* plan, const smk_skewers* sk, const smk_box_view* box,
@@ -1773,10 +1802,12 @@ extern "C" int smk_forest_step(smk_forest_plan* plan, const smk_skewers* sk, con
     SMK_REQUIRE(h == 0, SMK_ERR_RANGE, "a filter set index is outside [0, %d)", (int)n_sets);
   }
   // kernel instance for classes up to 3 (nz <= 2048, n <= 1998): one wave
-  // per skewer with at least 4 waves per SIMD (variant 0: some registers
-  // spill) or 3 (variant 1: none spill), two waves per skewer with at least
-  // 4 (variant 2) or 5 (variant 3: some spill); four waves per skewer with
-  // all six classes.  Skewers of a class above max_npix's are flagged
+  // per skewer with at least 3 waves per SIMD (variant 0: no register spills)
+  // or 4 (variant 1: some do), two waves per skewer with at least 4 (variant
+  // 2) or 5 (variant 3: some spill); four waves per skewer with all six
+  // classes.  200000 skewers of 300 to 1500 pixels: 1071, 1236, 1279 and 1347
+  // us; 30000: 203, 266, 216 and 243; 200000 of 100 to 200: 622, 566, 818 and
+  // 761.  Skewers of a class above max_npix's are flagged
   // (a.max_class)
   const bool small = c <= 3;
   const int var = plan->step_variant;
@@ -1794,14 +1825,17 @@ extern "C" int smk_forest_step(smk_forest_plan* plan, const smk_skewers* sk, con
   int dev = 0, ncu = 0, per_cu = 0;
   SMK_HIP_CHECK(hipGetDevice(&dev));
   SMK_HIP_CHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-  void (*const small_kern[SMK_FOREST_STEP_NVAR])(StepArgs) = {k_forest_step<3, 64, 4>, k_forest_step<3, 64, 3>,
+  void (*const small_kern[SMK_FOREST_STEP_NVAR])(StepArgs) = {k_forest_step<3, 64, 3>, k_forest_step<3, 64, 4>,
                                                                 k_forest_step<3, 128, 4>, k_forest_step<3, 128, 5>};
   void (*kern)(StepArgs) = small ? small_kern[var] : k_forest_step<N_CLASS - 1, NT_L, 1>;
   SMK_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, nt, lds));
   const int64_t want = (int64_t)ncu * (per_cu > 0 ? per_cu : 1);
   const int nblk = (int)(want < sk->n ? want : sk->n);
-  hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, s, a.queue, 1);
-  SMK_LAUNCH_CHECK();
+  a.n_static = step_static(sk->n, nblk);
+  if (a.n_static < sk->n) {
+    hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, s, a.queue, 1);
+    SMK_LAUNCH_CHECK();
+  }
   hipLaunchKernelGGL(kern, dim3(nblk), dim3(nt), lds, s, a);
   SMK_LAUNCH_CHECK();
   return SMK_OK;
