@@ -476,7 +476,7 @@ __device__ __forceinline__ void bluestein_tab(int N, int nout, In in, Emit emit,
 // Two independent M-point FFTs (va on line la, vb on line lb) in lockstep:
 // each stage's butterflies of both, then one pair of barriers around both
 // exchanges, so the two transforms share every barrier and every twiddle.
-template <int M, int E, bool INV, int S, int Ns>
+template <int M, int E, bool INV, int S, int Ns, bool HALF = false>
 __device__ __forceinline__ void stages2(double2 (&va)[E], double2 (&vb)[E], double2* __restrict__ la,
                                         double2* __restrict__ lb, int p, const double2* __restrict__ twM, int TW,
                                         const double2 (&w)[E / stage_radix(M, E, S)][stage_radix(M, E, S)]) {
@@ -486,8 +486,8 @@ __device__ __forceinline__ void stages2(double2 (&va)[E], double2 (&vb)[E], doub
   if constexpr (S < NS) {
     constexpr int R = stage_radix(M, E, S);
     constexpr bool LAST = S + 1 == NS;
-    stage<M, E, R, Ns, INV, LAST>(va, la, p, w);
-    stage<M, E, R, Ns, INV, LAST>(vb, lb, p, w);
+    stage<M, E, R, Ns, INV, LAST, HALF>(va, la, p, w);
+    stage<M, E, R, Ns, INV, LAST, HALF>(vb, lb, p, w);
     if constexpr (!LAST) {
       constexpr int R1 = stage_radix(M, E, S + 1);
       double2 w1[E / R1][R1];
@@ -504,12 +504,12 @@ __device__ __forceinline__ void stages2(double2 (&va)[E], double2 (&vb)[E], doub
   }
 }
 
-template <int M, int E, bool INV>
+template <int M, int E, bool INV, bool HALF = false>
 __device__ __forceinline__ void fft2(double2 (&va)[E], double2 (&vb)[E], double2* __restrict__ la,
                                      double2* __restrict__ lb, int p, const double2* __restrict__ twM, int TW) {
   constexpr int R0 = stage_radix(M, E, 0);
   double2 w0[E / R0][R0];   // stage 0 has Ns = 1: no twiddles
-  stages2<M, E, INV, 0, 1>(va, vb, la, lb, p, twM, TW, w0);
+  stages2<M, E, INV, 0, 1, HALF>(va, vb, la, lb, p, twM, TW, w0);
 }
 
 // bluestein_tab for two inputs in lockstep on the lines la and lb, of
@@ -525,12 +525,12 @@ __device__ __forceinline__ void bluestein_tab2(int Na, int Nb, In in, EmitA emit
                                                const double2* __restrict__ twM, int TW,
                                                const double2* __restrict__ wa, const double2* __restrict__ ba,
                                                const double2* __restrict__ wb, const double2* __restrict__ bb) {
-  constexpr int P = M / E;
+  constexpr int P = M / E, H = E / 2;   // Na, Nb <= M / 2: points of the lower half only, in and out
   const int p = threadIdx.x;
   const int nmax = Na > Nb ? Na : Nb;
   double2 va[E], vb[E];
 #pragma unroll
-  for (int e = 0; e < E; ++e) {
+  for (int e = 0; e < H; ++e) {
     const int n = p + P * e;
     va[e] = vb[e] = make_double2(0.0, 0.0);
     if (n < nmax) {
@@ -552,7 +552,7 @@ __device__ __forceinline__ void bluestein_tab2(int Na, int Nb, In in, EmitA emit
     for (int e = 0; e < E; ++e) bk[e] = ba[p + P * e];
   }
   __syncthreads();
-  fft2<M, E, false>(va, vb, la, lb, p, twM, TW);
+  fft2<M, E, false, true>(va, vb, la, lb, p, twM, TW);
 #pragma unroll
   for (int e = 0; e < E; ++e) {
     const double2 x = (KEEP & KEEP_B) ? bk[e] : ba[p + P * e];
@@ -561,7 +561,7 @@ __device__ __forceinline__ void bluestein_tab2(int Na, int Nb, In in, EmitA emit
   }
   fft2<M, E, true>(va, vb, la, lb, p, twM, TW);
 #pragma unroll
-  for (int e = 0; e < E; ++e) {
+  for (int e = 0; e < H; ++e) {
     const int k = p + P * e;
     if (SAME) {
       if (k < Na) {
