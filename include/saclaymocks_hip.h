@@ -305,8 +305,9 @@ int smk_forest_missing_power(smk_forest_plan* plan, const smk_skewers* sk, const
  * skewers, the device-drawn missing power (smk_forest_missing_power_sets,
  * merge_spectra.py:303-322), trilinear delta and eta_zz along the line of
  * sight (smk_forest_gather) and the FGPA (merge_spectra.py:335-339), with
- * delta_s kept on chip.  Each block takes skewers from a work queue in the
- * workspace (smk_forest_step_workspace_bytes(), cleared by the call).
+ * delta_s kept on chip.  The blocks take turns; the last skewers of a large
+ * batch come from a work queue in the workspace
+ * (smk_forest_step_workspace_bytes(), cleared by the call).
  *   filt, filt_off, set_stride, n_sets, filt_set, scale, seed: as
  *               smk_forest_missing_power_sets (device-drawn modes only; the
  *               plan's graph mode applies)

@@ -1086,7 +1086,8 @@ __global__ void k_classify(smk_skewers sk, const int32_t* __restrict__ fset, int
 
 // ------------------------------------------------------ fused forest step
 // One persistent launch for a batch of plane-parallel skewers: each block
-// takes skewers from a device work queue and, per skewer, (1) draws the
+// takes its turns of the skewers (the last of a large batch from a device
+// queue) and, per skewer, (1) draws the
 // missing-power Fourier modes into LDS (one Philox call per two modes),
 // (2) folds them for the C2R transform and inverse-FFTs them in LDS, so that
 // delta_s stays in LDS, (3) interpolates delta and eta_zz trilinearly along
