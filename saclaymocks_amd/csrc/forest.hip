@@ -1269,8 +1269,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(OCC))) void 
       continue;
     }
     if (c == 0) step_missing_power<0, NT>(a, s, n, seed, sh);
-    else if (c == 1) step_missing_power<1, NT>(a, s, n, seed, sh);
-    else if (c == 2) step_missing_power<2, NT>(a, s, n, seed, sh);
+    else if (c == 1 || MAXC <= 1) step_missing_power<1, NT>(a, s, n, seed, sh);
+    else if (c == 2 || MAXC <= 2) step_missing_power<(MAXC < 2 ? MAXC : 2), NT>(a, s, n, seed, sh);
     else if (c == 3 || MAXC <= 3) step_missing_power<(MAXC < 3 ? MAXC : 3), NT>(a, s, n, seed, sh);
     else if (c == 4 || MAXC <= 4) step_missing_power<(MAXC < 4 ? MAXC : 4), NT>(a, s, n, seed, sh);
     else step_missing_power<MAXC, NT>(a, s, n, seed, sh);
@@ -1812,9 +1812,17 @@ extern "C" int smk_forest_step(smk_forest_plan* plan, const smk_skewers* sk, con
   // (a.max_class)
   const bool small = c <= 3;
   const int var = plan->step_variant;
+  // variant 0 has instances for batches without the longer classes, of the same
+  // register tiles (the same bits), with fewer registers and less LDS: 95 and
+  // 121 registers, 5 and 4 waves per SIMD, none spilled.  200000 skewers of 100
+  // to 200 pixels 630 -> 491 us, of 200 to 410 762 -> 558, of 300 to 900
+  // 891 -> 749; forced to 6 and 5 waves 494, 570 and 804.
+  const bool short_batch = var == 0 && c <= 2;
   constexpr int NT_L = 256;
   const int nt = small ? (var >= 2 ? 128 : 64) : NT_L;
-  const int mp_float2 = small ? (nt == 128 ? step_lds_max(3, 128) : step_lds_max(3, 64))
+  const int mp_float2 = small ? (nt == 128 ? step_lds_max(3, 128)
+                                 : short_batch ? (c <= 1 ? step_lds_max(1, 64) : step_lds_max(2, 64))
+                                               : step_lds_max(3, 64))
                               : step_lds_max(N_CLASS - 1, NT_L);
   // column table: the z cells of the longest forest (n pixels span at most
   // n dr / D + 2 cells; 2 more for the rounding of the positions), up to
@@ -1829,6 +1837,7 @@ extern "C" int smk_forest_step(smk_forest_plan* plan, const smk_skewers* sk, con
   void (*const small_kern[SMK_FOREST_STEP_NVAR])(StepArgs) = {k_forest_step<3, 64, 3>, k_forest_step<3, 64, 4>,
                                                                 k_forest_step<3, 128, 4>, k_forest_step<3, 128, 5>};
   void (*kern)(StepArgs) = small ? small_kern[var] : k_forest_step<N_CLASS - 1, NT_L, 1>;
+  if (short_batch) kern = c <= 1 ? k_forest_step<1, 64, 4> : k_forest_step<2, 64, 3>;
   SMK_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, nt, lds));
   const int64_t want = (int64_t)ncu * (per_cu > 0 ? per_cu : 1);
   const int nblk = (int)(want < sk->n ? want : sk->n);
