@@ -509,18 +509,35 @@ __global__ __launch_bounds__(T*(M / E)) void k_z_r2c(const float* __restrict__ n
 
   if (noise == nullptr) {
     // four cells per Philox call: cells 4q..4q+3 of the whole box
-    constexpr int Q = M / 2;
-    for (int q = tid; q < T * Q; q += NT) {
-      const int tt = q / Q, qq = q % Q;
-      const uint64_t LL_ = L0 + tt;
-      if (LL_ < n_pencils) {
-        U4 u = philox4x32_10(LL_ * (uint64_t)Q + qq, seed);
-        float n0, n1, n2, n3;
-        box_muller_hw(u.x, u.y, n0, n1);
-        box_muller_hw(u.z, u.w, n2, n3);
-        float2* ln = lds + tt * LL;
-        ln[lds_pos<M>(2 * qq)] = make_float2(n0, n1);
-        ln[lds_pos<M>(2 * qq + 1)] = make_float2(n2, n3);
+    if constexpr (M % 2 == 0) {
+      constexpr int Q = M / 2;
+      for (int q = tid; q < T * Q; q += NT) {
+        const int tt = q / Q, qq = q % Q;
+        const uint64_t LL_ = L0 + tt;
+        if (LL_ < n_pencils) {
+          U4 u = philox4x32_10(LL_ * (uint64_t)Q + qq, seed);
+          float n0, n1, n2, n3;
+          box_muller_hw(u.x, u.y, n0, n1);
+          box_muller_hw(u.z, u.w, n2, n3);
+          float2* ln = lds + tt * LL;
+          ln[lds_pos<M>(2 * qq)] = make_float2(n0, n1);
+          ln[lds_pos<M>(2 * qq + 1)] = make_float2(n2, n3);
+        }
+      }
+    } else {
+      // every other pencil begins in the middle of a call: each point takes
+      // its half of the call its two cells are in
+      for (int q = tid; q < T * M; q += NT) {
+        const int tt = q / M, n = q % M;
+        const uint64_t LL_ = L0 + tt;
+        if (LL_ < n_pencils) {
+          const uint64_t g = LL_ * (uint64_t)M + n;
+          const U4 u = philox4x32_10(g / 2, seed);
+          float n0, n1;
+          if (g % 2 == 0) box_muller_hw(u.x, u.y, n0, n1);
+          else box_muller_hw(u.z, u.w, n0, n1);
+          lds[tt * LL + lds_pos<M>(n)] = make_float2(n0, n1);
+        }
       }
     }
     __syncthreads();
