@@ -1212,10 +1212,11 @@ __device__ __forceinline__ void step_missing_power(const StepArgs& a, int s, int
   __syncthreads();
 }
 
-constexpr int STEP_RUN = 4;   // skewers per queue slot
+constexpr int step_run(int nt) { return nt < 256 ? 4 : 1; }   // skewers per queue slot
 
 // the block's skewer after s (see k_forest_step); the same value in every lane,
 // so scalar registers hold all per-skewer terms
+template <int RUN>
 __device__ __forceinline__ int step_next(const StepArgs& a, int s, int& left, int q_next, int* s_next) {
   __syncthreads();   // the LDS of this skewer is free
   if (left > 0) {
@@ -1227,7 +1228,7 @@ __device__ __forceinline__ int step_next(const StepArgs& a, int s, int& left, in
   if (threadIdx.x == 0) *s_next = q_next;
   __syncthreads();
   s = a.n_static + __builtin_amdgcn_readfirstlane(*s_next);
-  left = STEP_RUN - 1;
+  left = RUN - 1;
   return s;
 }
 
@@ -1247,15 +1248,15 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(OCC))) void 
   const float* __restrict__ fe = b.eta[2];
   const double D = b.cell;
   // Skewers [0, n_static) go round the blocks, the rest from a queue in runs
-  // of STEP_RUN; a run is taken while the block's skewer before it is
+  // of step_run; a run is taken while the block's skewer before it is
   // processed (its atomic's latency overlaps the work) and goes to one block.
   // The queue's atomics on one address take 11.7 ns each, so that with one
   // per skewer they bounded the step: 200000 skewers took 2.34 ms at any length.
   int s = (int)blockIdx.x, left = 0, q_next = 0;   // left: skewers of the run after s
-  for (; s < sk.n; s = step_next(a, s, left, q_next, &s_next)) {
+  for (; s < sk.n; s = step_next<step_run(NT)>(a, s, left, q_next, &s_next)) {
     // the last of a run, or of the static part: the next run
     if (tid == 0 && left == 0 && s + (int)gridDim.x >= a.n_static && a.n_static < sk.n)
-      q_next = atomicAdd(a.queue, STEP_RUN);
+      q_next = atomicAdd(a.queue, step_run(NT));
     const int n = sk.npix[s];
     int c = 0;
     for (int nzc = 256; nzc < n + 50 && c < N_CLASS; nzc <<= 1) ++c;
@@ -1733,9 +1734,14 @@ extern "C" int smk_forest_missing_power(smk_forest_plan* plan, const smk_skewers
 // and runs of 4, 1110 with 90% and 1218 with all, 1120 with runs of 2 and 1415
 // with runs of 1; 2394 with every skewer in the queue.  3000 to 30000: within
 // 3% of all round the blocks (205 us for 30000, 424 with every one queued).
-static int step_static(int n, int nblk) {
+// Blocks of 256 threads (skewers of more than 1998 pixels) are a few per CU
+// and their skewers long, so that a run is one skewer and the queue pays from
+// three per block: 8000 skewers of 300 to 7000 pixels take 255 us, 295 with
+// runs of 4, 275 with every one queued; 4000 142, 159 with all round the
+// blocks, 160 queued; 1000 74 with the queue and 50 without.
+static int step_static(int n, int nblk, int run) {
   const int64_t rounds = n / nblk;
-  return rounds < 10 ? n : (int)(rounds * 7 / 10) * nblk;
+  return rounds < (run > 1 ? 10 : 3) ? n : (int)(rounds * 7 / 10) * nblk;
 }
 
 extern "C" size_t smk_forest_step_workspace_bytes(void) { return 256; }
@@ -1809,7 +1815,9 @@ extern "C" int smk_forest_step(smk_forest_plan* plan, const smk_skewers* sk, con
   // classes.  200000 skewers of 300 to 1500 pixels: 1071, 1236, 1279 and 1347
   // us; 30000: 203, 266, 216 and 243; 200000 of 100 to 200: 622, 566, 818 and
   // 761.  Skewers of a class above max_npix's are flagged
-  // (a.max_class)
+  // (a.max_class).  The instance of all classes needs its two waves per SIMD
+  // asked for: with three registers more than the 256 that they leave, 30000
+  // skewers of 3000 pixels took 1497 us instead of 815
   const bool small = c <= 3;
   const int var = plan->step_variant;
   // variant 0 has instances for batches without the longer classes, of the same
@@ -1836,12 +1844,12 @@ extern "C" int smk_forest_step(smk_forest_plan* plan, const smk_skewers* sk, con
   SMK_HIP_CHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
   void (*const small_kern[SMK_FOREST_STEP_NVAR])(StepArgs) = {k_forest_step<3, 64, 3>, k_forest_step<3, 64, 4>,
                                                                 k_forest_step<3, 128, 4>, k_forest_step<3, 128, 5>};
-  void (*kern)(StepArgs) = small ? small_kern[var] : k_forest_step<N_CLASS - 1, NT_L, 1>;
+  void (*kern)(StepArgs) = small ? small_kern[var] : k_forest_step<N_CLASS - 1, NT_L, 2>;
   if (short_batch) kern = c <= 1 ? k_forest_step<1, 64, 4> : k_forest_step<2, 64, 3>;
   SMK_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, nt, lds));
   const int64_t want = (int64_t)ncu * (per_cu > 0 ? per_cu : 1);
   const int nblk = (int)(want < sk->n ? want : sk->n);
-  a.n_static = step_static(sk->n, nblk);
+  a.n_static = step_static(sk->n, nblk, step_run(nt));
   if (a.n_static < sk->n) {
     hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, s, a.queue, 1);
     SMK_LAUNCH_CHECK();
