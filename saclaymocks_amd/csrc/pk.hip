@@ -519,6 +519,7 @@ extern "C" int smk_pk_table(const smk_pk_spline* spline, const float* kx, const 
   SMK_REQUIRE(nxs >= 0 && ny > 0 && nzh > 0 && vcell > 0.0f, SMK_ERR_ARG, "bad table shape");
   const uint64_t nmodes = (uint64_t)nxs * (uint64_t)ny * (uint64_t)nzh;
   if (nmodes == 0) return SMK_OK;
+  SMK_REQUIRE((nmodes + 255) / 256 <= 0x7fffffffull, SMK_ERR_ARG, "table too large for one launch");
   TableArgs a;
   a.sp = *spline;
   a.r_step = 1.0 / spline->g_step;
