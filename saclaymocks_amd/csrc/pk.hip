@@ -63,7 +63,8 @@ __device__ __forceinline__ float sqrt_f32(float x) {
 
 struct TableArgs {
   smk_pk_spline sp;
-  double r_step, r_lo, r_vcell;   // 1 / sp.g_step, -sp.g_lo / sp.g_step, 1 / vcell
+  double r_step, r_lo;            // 1 / sp.g_step, -sp.g_lo / sp.g_step
+  double vcell, r_vcell;          // vcell, 1 / vcell
   const float *kx, *ky, *kz;
   uint32_t ny, nzh, nch;          // nch: 64-mode pieces of a row
   float* out;
@@ -79,19 +80,16 @@ __device__ __forceinline__ uint32_t guess_bin(double k, double r_step, double r_
   return g < last ? g : last;
 }
 
-// sqrt(max(P, 0) / vcell), P the cubic c at d; the float32 quotient is rounded
-// once: 1 / vcell is exact to 2^-53, and a quotient of float32s no nearer than
-// 2^-49 to the middle of two
-__device__ __forceinline__ float table_value(const TableArgs& a, const double* c, double d) {
-  const double p = ((c[0] * d + c[1]) * d + c[2]) * d + c[3];
-  return sqrt_f32((float)((double)fmaxf((float)p, 0.0f) * a.r_vcell));
+// max(P, 0) in float32, P the cubic c at d
+__device__ __forceinline__ float table_power(const double* c, double d) {
+  return fmaxf((float)(((c[0] * d + c[1]) * d + c[2]) * d + c[3]), 0.0f);
 }
 
-__device__ __forceinline__ float table_global(const TableArgs& a, double k) {
+__device__ __forceinline__ float power_global(const TableArgs& a, double k) {
   int iv = a.sp.guess[guess_bin(k, a.r_step, a.r_lo, (uint32_t)a.sp.n_guess - 1)];
   while (iv + 1 < a.sp.n_int && a.sp.x[iv + 1] <= k) ++iv;
   while (iv > 0 && a.sp.x[iv] > k) --iv;
-  return table_value(a, a.sp.c + 4 * (int64_t)iv, k - a.sp.x[iv]);
+  return table_power(a.sp.c + 4 * (int64_t)iv, k - a.sp.x[iv]);
 }
 
 constexpr int TABLE_ROWS = 4;  // rows that a wave's lanes have at a time
@@ -180,7 +178,7 @@ __global__ __launch_bounds__(LDS ? 1024 : 256) __attribute__((amdgpu_waves_per_e
       }
 #pragma unroll
       for (int u = 0; u < TABLE_ROWS; ++u)
-        r[u] = table_value(a, reinterpret_cast<const double*>(cb + 4 * at[u]), k[u] - x0[u]);
+        r[u] = table_power(reinterpret_cast<const double*>(cb + 4 * at[u]), k[u] - x0[u]);
     }
     if (!lds) {
       // the loads of all rows ahead of what waits for them
@@ -203,20 +201,34 @@ __global__ __launch_bounds__(LDS ? 1024 : 256) __attribute__((amdgpu_waves_per_e
         }
       }
 #pragma unroll
-      for (int u = 0; u < TABLE_ROWS; ++u) r[u] = table_value(a, a.sp.c + 4 * (int64_t)iv[u], k[u] - x0[u]);
+      for (int u = 0; u < TABLE_ROWS; ++u) r[u] = table_power(a.sp.c + 4 * (int64_t)iv[u], k[u] - x0[u]);
     } else if (off) {
 #pragma unroll 1
       for (int u = 0; u < TABLE_ROWS; ++u) {
-        const float v = table_global(a, u == 0 ? k[0] : (u == 1 ? k[1] : (u == 2 ? k[2] : k[3])));
+        const float v = power_global(a, u == 0 ? k[0] : (u == 1 ? k[1] : (u == 2 ? k[2] : k[3])));
         r[0] = u == 0 ? v : r[0];
         r[1] = u == 1 ? v : r[1];
         r[2] = u == 2 ? v : r[2];
         r[3] = u == 3 ? v : r[3];
       }
     }
+    // the quotient through 1 / vcell, which is exact to 2^-53: rounded once where
+    // it is normal, as a quotient of float32s is then no nearer than 2^-49 to the
+    // middle of two; a subnormal one may be the middle itself and is divided
+    float q[TABLE_ROWS];
+    bool sub = false;
+#pragma unroll
+    for (int u = 0; u < TABLE_ROWS; ++u) {
+      q[u] = (float)((double)r[u] * a.r_vcell);
+      sub |= __builtin_amdgcn_classf(q[u], 0x080);
+    }
+    if (sub) {
+#pragma unroll
+      for (int u = 0; u < TABLE_ROWS; ++u) q[u] = (float)((double)r[u] / a.vcell);
+    }
 #pragma unroll
     for (int u = 0; u < TABLE_ROWS; ++u)
-      if (l < a.nzh && row + (uint64_t)u < a.nrows) a.out[(row + (uint64_t)u) * a.nzh + l] = r[u];
+      if (l < a.nzh && row + (uint64_t)u < a.nrows) a.out[(row + (uint64_t)u) * a.nzh + l] = sqrt_f32(q[u]);
     // the next piece of this wave
     group += a.dgroup;
     i += a.di;
@@ -524,7 +536,8 @@ extern "C" int smk_pk_table(const smk_pk_spline* spline, const float* kx, const 
   a.sp = *spline;
   a.r_step = 1.0 / spline->g_step;
   a.r_lo = -spline->g_lo / spline->g_step;
-  a.r_vcell = 1.0 / (double)vcell;
+  a.vcell = (double)vcell;
+  a.r_vcell = 1.0 / a.vcell;
   a.kx = kx;
   a.ky = ky;
   a.kz = kz;
