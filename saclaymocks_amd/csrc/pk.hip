@@ -8,6 +8,7 @@
 #include <math.h>
 
 #include "fft_core.h"
+#include "route.h"
 #include "smk_internal.h"
 
 using namespace smk;
@@ -95,10 +96,16 @@ __device__ __forceinline__ float power_global(const TableArgs& a, double k) {
 constexpr int TABLE_ROWS = 4;  // rows that a wave's lanes have at a time
 constexpr int SEGS = 1760;     // segments in LDS: two blocks of 1024 threads per CU
 constexpr int BINS = 4096;     // bins of the guess table in LDS
-// Tables from here on take the LDS kernel, whose blocks first load 20 to 80 KB
-// each: 2.5 million modes take 15.9 us with and 14.5 without, 3.7 million 19.2
-// and 19.0, 6.2 million 25.9 and 27.2.
-constexpr uint64_t LDS_MODES = 4u << 20;
+// A thread per mode, the spline in global memory: tables of few modes or of
+// rows that would leave many lanes of k_pk_table idle (smk_route::pk_table).
+__global__ __launch_bounds__(256) void k_pk_modes(TableArgs a, uint64_t nmodes) {
+  const uint64_t m = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+  if (m >= nmodes) return;
+  const uint64_t row = m / a.nzh;
+  const float kx = a.kx[row / a.ny], ky = a.ky[row % a.ny], kz = a.kz[m % a.nzh];
+  const float k = sqrt_f32(add_rn(add_rn(mul_rn(kx, kx), mul_rn(ky, ky)), mul_rn(kz, kz)));
+  a.out[m] = sqrt_f32((float)((double)power_global(a, (double)k) / a.vcell));
+}
 
 // A wave has 64 neighbouring modes of TABLE_ROWS rows at a time, a lane one
 // column of them: k from the float32 axes as numpy's sqrt((kx*kx + ky*ky) + kz*kz),
@@ -548,7 +555,13 @@ extern "C" int smk_pk_table(const smk_pk_spline* spline, const float* kx, const 
   a.nrows = (uint64_t)nxs * (uint64_t)ny;
   a.ngroup = (a.nrows + TABLE_ROWS - 1) / TABLE_ROWS;
   const hipStream_t st = (hipStream_t)stream;
-  const bool lds = nmodes >= LDS_MODES;
+  const smk_route::PkTable route = smk_route::pk_table(nmodes, (uint64_t)nzh);
+  if (route == smk_route::PK_MODES) {
+    hipLaunchKernelGGL(k_pk_modes, dim3((uint32_t)((nmodes + 255) / 256)), dim3(256), 0, st, a, nmodes);
+    SMK_LAUNCH_CHECK();
+    return SMK_OK;
+  }
+  const bool lds = route == smk_route::PK_ROWS_LDS;
   // two blocks of 16 waves per CU; or as many waves as there are pieces, of which fewer than 2^18
   const uint64_t blocks = lds ? 512 : (a.ngroup * a.nch + 3) / 4, waves = blocks * (lds ? 16 : 4);
   a.dgroup = waves / a.nch;
