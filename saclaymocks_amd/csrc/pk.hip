@@ -428,10 +428,17 @@ __device__ __forceinline__ void store_row(const RsdArgs& a, int i, double acc, d
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
   __syncthreads();
   if (threadIdx.x == 0) a.out[i] = (((red[0] + red[1]) + red[2]) + red[3]) / 2.0 / M_PI;
-  __syncthreads();
 }
 
-// One block per k_par row (models 0 and 1).
+// One block per k_par row by row_sum: rows too short or too few for what
+// follows (smk_route::p1d_fast, p1d_cut_rows).
+template <int MODEL>
+__global__ __launch_bounds__(256) void k_p1d_rows(RsdArgs a) {
+  __shared__ double red[4];
+  store_row(a, blockIdx.x, row_sum<MODEL>(a, a.k_par[blockIdx.x], 0, a.n_perp), red);
+}
+
+// One block per k_par row by row_fast (models 0 and 1).
 template <int MODEL>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k_p1d_rsd_rows(RsdArgs a) {
   __shared__ double red[4];
@@ -456,7 +463,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k
 // 20000 rows of 20000 points: 1.6 ms with every point evaluated, 0.21 with
 // whole waves passing over the points beyond, row by row, bound by the
 // 3.2 GB of k_perp that the rows read from L2; 0.09 with 8 rows to a block.
-// Fewer rows than 8192 go fewer to a block, so that the blocks fill the card.
 __global__ __launch_bounds__(256) void k_p1d_cut_rows(RsdArgs a, int n_par, int rows) {
   __shared__ double red[4];
   __shared__ int range[2];
@@ -489,7 +495,10 @@ __global__ __launch_bounds__(256) void k_p1d_cut_rows(RsdArgs a, int n_par, int 
   __syncthreads();
   lo = range[0] & ~255;   // whole turns of the block: the sum's order is that of the whole row
   hi = range[1];
-  for (int i = i0; i < i1; ++i) store_row(a, i, row_sum<2>(a, a.k_par[i], lo, hi), red);
+  for (int i = i0; i < i1; ++i) {
+    store_row(a, i, row_sum<2>(a, a.k_par[i], lo, hi), red);
+    __syncthreads();   // red is free
+  }
 }
 
 }  // namespace
@@ -518,12 +527,15 @@ extern "C" int smk_p1d_rsd_rows(const smk_pk_spline* spline, const double* k_par
   a.kny = kny;
   a.out = out;
   const hipStream_t st = (hipStream_t)stream;
-  if (model == 0) hipLaunchKernelGGL(k_p1d_rsd_rows<0>, dim3(n_par), dim3(256), 0, st, a);
-  else if (model == 1) hipLaunchKernelGGL(k_p1d_rsd_rows<1>, dim3(n_par), dim3(256), 0, st, a);
-  else {
-    const int rows = n_par < 2048 ? 1 : (n_par < 8192 ? n_par / 1024 : 8);   // 1024 blocks or more
+  const int rows = model == 2 ? smk_route::p1d_cut_rows(n_par, n_perp) : 1;
+  const bool fast = smk_route::p1d_fast(model, n_par, n_perp);
+  void (*const whole)(RsdArgs) = model == 0   ? (fast ? k_p1d_rsd_rows<0> : k_p1d_rows<0>)
+                                 : model == 1 ? (fast ? k_p1d_rsd_rows<1> : k_p1d_rows<1>)
+                                              : k_p1d_rows<2>;
+  if (model == 2 && rows > 0)
     hipLaunchKernelGGL(k_p1d_cut_rows, dim3((n_par + rows - 1) / rows), dim3(256), 0, st, a, n_par, rows);
-  }
+  else
+    hipLaunchKernelGGL(whole, dim3(n_par), dim3(256), 0, st, a);
   SMK_LAUNCH_CHECK();
   return SMK_OK;
 }

@@ -31,4 +31,35 @@ constexpr PkTable pk_table(uint64_t modes, uint64_t nzh) {
   return modes >= PK_LDS_MODES ? PK_ROWS_LDS : PK_ROWS;
 }
 
+// ------------------------------------------- rows of the missing 1D power
+// Whether models 0 and 1 take the sum of fewer instructions (row_fast), which
+// first fills its tables and finds its segments: it needs points to a row to
+// pay for that, and more rows than two per CU, as with fewer the latency of a
+// point decides, which it does not shorten.  Us, row_sum against row_fast, by
+// points of a row:
+//              model 1:  200         400         600         900         2500        20000
+//   512 rows             7.1, 7.6    7.3, 8.4    8.9, 10.0   10.7, 11.8  21.9, 22.7  144, 147
+//   1024 rows            7.3, 7.9    9.4, 10.4   12.0, 11.8  15.5, 14.6  33.6, 24.3  234, 149
+//   2048 rows            11.0, 12.2  15.4, 15.7  19.3, 19.1  25.3, 21.9  57.2, 34.1  400, 162
+//   8192 rows            34.7, 35.6  49.9, 45.3  63.5, 55.2  85.0, 66.1  197, 110    1399, 519
+//              model 0:  600         1500        2500        5000        10000       20000
+//   400 rows             7.2, 7.7    8.3, 9.9    11.5, 13.0  20.1, 21.9  36.4, 38.3  68.8, 63.3
+//   768 rows             7.4, 8.0    9.6, 11.1   12.9, 13.7  22.5, 23.3  41.4, 40.1  78.9, 64.7
+//   2048 rows            9.5, 12.2   17.2, 17.9  26.4, 22.9  45.2, 38.0  85.5, 62.5  164, 98.5
+//   12000 rows           37.8, 50.5  81.4, 80.7  130, 114    248, 176    479, 254    931, 379
+constexpr bool p1d_fast(int model, int n_par, int n_perp) {
+  if (model == 0) return n_perp >= (n_par > 1024 ? 1500 : n_par > 512 ? 8000 : 15000);
+  return model == 1 && n_par > 512 && n_perp >= (n_par > 2560 ? 350 : n_par > 1024 ? 550 : 750);
+}
+
+// Rows per block of model 2 (k_p1d_cut_rows), so that the blocks fill the card:
+// 1024 blocks or more, 4096 where a row has less than a point per thread.  0:
+// a few short rows, as they are, without the range of k_perp found first (100
+// to 512 rows of 900 points 7.3 us against 8.0; 600 the same either way).
+constexpr int p1d_cut_rows(int n_par, int n_perp) {
+  if (n_par <= 512 && n_perp <= 1024) return 0;
+  const int rows = n_par / (n_perp < 200 ? 4096 : 1024);
+  return rows < 1 ? 1 : rows < 8 ? rows : 8;
+}
+
 }  // namespace smk_route
