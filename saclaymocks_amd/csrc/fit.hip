@@ -23,6 +23,7 @@
 
 #include "fft64.h"
 #include "fft_core.h"
+#include "route.h"
 #include "smk_internal.h"
 
 using namespace smk;
@@ -124,23 +125,14 @@ __device__ __forceinline__ double wave_sum(double v) {
 // the per-skewer FGPA kernels run one wave per skewer (a forest of ~10^3
 // pixels is ~16 loads per lane; a block per skewer spent its time on block
 // barriers and the skewer's descriptor loads), k_fgpa_flux several where the
-// skewers are few or long (flux_waves)
+// skewers are few or long (smk_route::flux_waves)
 constexpr int FLUX_WAVES = FIT_THREADS / 64;
 __device__ __forceinline__ int flux_wave() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); }
 int grid_for_waves(int n, int w = 1) {
   const int b = (n + FLUX_WAVES / w - 1) / (FLUX_WAVES / w);
   return b < 1 ? 1 : (b < 65536 ? b : 65536);
 }
-// Waves of k_fgpa_flux to a skewer.  Few skewers leave waves idle if each has
-// one, and a long one is a long chain on one wave: 600 skewers of 7500 pixels
-// take 60.8, 34.7 and 22.6 us with 1, 2 and 8 (16 at the copy rate), 3000 of
-// 8000 149, 124 and 122, 1500 of 1500 15.2, 13.9 and 13.2.  Short ones do not
-// fill eight: 3000 of 700 take 13.0, 11.5 and 16.2, 2000 of 650 8.8, 8.7 and
-// 11.1, and many short ones fill the card alone: 6000 of 1000 23.8, 24.3, 32.6.
-int flux_waves(const smk_skewers& sk) {
-  if (sk.npix_total >= 1400 * (int64_t)sk.n) return 8;
-  return sk.n < 4096 ? 2 : 1;
-}
+int flux_waves(const smk_skewers& sk) { return smk_route::flux_waves(sk.n, sk.npix_total, sk.pset == nullptr); }
 
 // F for every pixel, in FP64 so that chi2(theta) is smooth to FP64 rounding
 // (the optimisers' line searches need that); per-skewer sum of F over the

@@ -62,4 +62,34 @@ constexpr int p1d_cut_rows(int n_par, int n_perp) {
   return rows < 1 ? 1 : rows < 8 ? rows : 8;
 }
 
+// ------------------------------------------------------------- FGPA flux
+// Waves that a skewer of k_fgpa_flux and k_fgpa_flux_jac gets (eight waves to a
+// block).  Few skewers leave the card idle with one wave each, and a long one
+// is a long chain on one wave; but eight waves share a barrier per skewer,
+// which many skewers pay for.  One wave each also leaves a part of the last of
+// the blocks' rounds over the 256 CUs idle, which two waves halve.  Us with 1,
+// 2 and 8 waves, one parameter set per skewer:
+//             700 pixels        1400              3000             6500
+//     600     7.8  7.5  7.5     9.7  7.5  7.6     18   12   9.9    35   24   16
+//    1500     7.3  7.3  8.2     11.2 11.1 10.6    20.5 18.7 16.6   37   34   28
+//    2000     7.8  7.7  9.9     12.6 11.6 13.0    22   20   20     40   37   38
+//    3000     10.9 9.8  13.6    17.6 14.9 17.6    31   26   28     78   67   67
+//    4000     11.9 12.3 17.4    18.6 18.3 22      34.5 34   36     94   101  89
+//    5000     14.8 14.2 20.8    23.4 21.9 26.5    45   41   45     125  116  110
+//   10000     23   23.5 38      38   38   52      103  103  114    224  227  215
+//   20000     42   43   74      95   97   131     203  199  223    442  434  414
+// and with parameters per pixel 6500 pixels take 59, 43, 34.5 (1500 skewers),
+// 117, 106, 104 (3000) and 309, 329, 322 (10000).
+constexpr int flux_waves(int64_t n, int64_t pixels, bool per_pixel) {
+  const int64_t mean = pixels / (n > 0 ? n : 1);
+  const int64_t round = 8 * 256;   // skewers, one wave each, in a round of the CUs
+  const bool idle = 20 * n < 17 * ((n + round - 1) / round * round);   // one wave each use less than 85% of the rounds
+  if (n <= round) {
+    if (mean >= (n <= 1200 ? 1400 : n <= 1536 ? 2000 : 8000)) return 8;
+    return mean >= (n <= 1200 || per_pixel ? 600 : 1400) ? 2 : 1;
+  }
+  if (mean >= 6000 && (idle || !per_pixel)) return 8;
+  return idle && mean >= (n <= 4096 ? 600 : 1000) ? 2 : 1;
+}
+
 }  // namespace smk_route
