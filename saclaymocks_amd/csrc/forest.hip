@@ -24,6 +24,7 @@
 #include <vector>
 
 #include "fft_core.h"
+#include "route.h"
 #include "smk_internal.h"
 
 using namespace smk;
@@ -512,8 +513,12 @@ __global__ __launch_bounds__(NT)
       }
       gather_out(a, s, off + i, g0 + i, -1000000.0f, 0.0f, 0.0f);
     }
+    // pixels to begin with: what fitted last, or twice that if it fitted at once
+    // (beginning with NT every time, pixels a cell apart at dmax 1 took 1.2 times
+    // k_gather's time in three or four rounds of barriers a part, now 0.8)
+    int most = NT;
     for (int f = f0; f < f1;) {
-      const int n = f1 - f < NT ? f1 - f : NT;
+      const int n = f1 - f < most ? f1 - f : most;
       // ---- the thread's pixel and its cell
       const LosPixel q = los_pixel(a, l, g0 + f + (tid < n ? tid : 0));
       int64_t sx = 0, sy = 0, sz = 0;
@@ -618,6 +623,7 @@ __global__ __launch_bounds__(NT)
         nl = (nl + 1) / 2;
         __syncthreads();
       }
+      most = nl < n ? nl : (2 * most < NT ? 2 * most : NT);
       const int rows = WX * WY;
       const int ps = rows | 1;   // plane stride, odd: planes start in different LDS banks
       if (nk > 0) {
@@ -1582,17 +1588,13 @@ static void launch_radial_nt(hipStream_t st, const GatherArgs& a) {
                      gg_lds_bytes<G>(DM, NT), st, a, span);
 }
 
-// k_gather_radial or k_gather.  One field fits k_gather's L1 (761 us against
-// 661 for 2000 skewers at dmax 3, but 34 against 45 for 30), and so does one
-// cell per pixel (dmax 0).  A block of k_gather_radial does one skewer at a
-// time, so short skewers leave it idle: with seven fields and 2e6 pixels in
-// all, dmax 1 takes 488 us against 685 at 50 pixels per skewer and 1005
-// against 790 at 20; dmax 2 13.0 ms against 15.9 and dmax 3 21.5 against 44.1
-// at 2.
+// k_gather_radial or k_gather (smk_route::gather_radial).  One field fits
+// k_gather's L1: 761 us against 661 for 2000 skewers at dmax 3, but 34 against
+// 45 for 30.
 template <int NF, int DM>
 static void launch_gather_dm(hipStream_t st, const GatherArgs& a) {
   if constexpr (NF >= 7 && DM >= 1) {
-    if (a.npix_total >= (DM == 1 ? 40 : 2) * (int64_t)a.sk.n) {
+    if (smk_route::gather_radial(DM, a.sk.n, a.npix_total, a.sk.dr / a.box.cell)) {
       launch_radial_nt<NF, DM, 256>(st, a);
       return;
     }

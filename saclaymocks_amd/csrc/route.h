@@ -92,4 +92,24 @@ constexpr int flux_waves(int64_t n, int64_t pixels, bool per_pixel) {
   return idle && mean >= (n <= 4096 ? 600 : 1000) ? 2 : 1;
 }
 
+// ------------------------------------------- smoothing along radial lines
+// Whether the smoothing over (2 dmax + 1)^3 cells of seven or more fields takes
+// k_gather_radial (a tube of cells per run of pixels) or k_gather (a thread per
+// pixel, each its own cells), for lines of `pixels` pixels in all and pixels
+// `cells` cells apart.
+//
+// One cell per pixel (dmax 0) fits k_gather's L1.  A block of k_gather_radial
+// does one skewer at a time, so short skewers leave it idle: with seven fields
+// and 2e6 pixels in all, dmax 1 takes 488 us against 685 at 50 pixels per
+// skewer and 1005 against 790 at 20; dmax 2 13.0 ms against 15.9 and dmax 3 21.5
+// against 44.1 at 2.  And with pixels cells apart a tube holds few of them: a
+// million pixels along x or y, dmax 1, take 0.37 of k_gather's time at a half
+// of a cell, 0.45 at one, 0.8 at two, 0.9 at two and a half, 1.1 at three, 1.4
+// at four and 2.2 at eight (along z 0.9, 0.85, 0.85, 0.85, 0.8, 0.6, 0.8; dmax 2
+// 0.8 at the most, dmax 3 0.45).
+constexpr bool gather_radial(int dmax, int64_t n, int64_t pixels, double cells) {
+  if (dmax < 1 || pixels < (dmax == 1 ? 40 : 2) * n) return false;
+  return dmax > 1 || (cells <= 2.75 && cells >= -2.75);
+}
+
 }  // namespace smk_route
