@@ -435,6 +435,9 @@ template <int G> constexpr size_t gg_lds_bytes(int DM, int NT) {
   return (size_t)((gg_cap(DM, NT) + 1) & ~1) * (4 + 8 * (G - 1));
 }
 
+// the window arrays and the line below, at the most
+constexpr size_t GG_STATIC_BYTES = 9 * GG_NK * sizeof(int) + 512;
+
 // NF fields: 7 (delta and the six eta_ij) or 10 (those and the three
 // velocities); DM the stencil radius.  Block b takes the packed pixels
 // [b span, (b+1) span), in parts of at most NT pixels of one skewer.
@@ -445,6 +448,8 @@ __global__ __launch_bounds__(NT)
   constexpr int G = NF == 10 ? 3 : 2;
   constexpr int CAP = gg_cap(DM, NT), CAP2 = (CAP + 1) & ~1;
   static_assert(W * (W * W | 1) + W <= CAP, "one pixel must fit");
+  static_assert(gg_lds_bytes<G>(DM, NT) + GG_STATIC_BYTES <= 160 * 1024, "a CU's LDS must hold the tube");
+  static_assert(CAP * GG_NK < (1 << 20), "the cell's indices by multiplication must be exact");
   extern __shared__ double gg_lds[];
   double* ge = gg_lds;
   double* gv = gg_lds + CAP2;   // with velocities only
