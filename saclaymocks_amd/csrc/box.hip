@@ -203,8 +203,9 @@ extern "C" int smk_box_plan_create(smk_box_plan** plan, int nx, int ny, int nz, 
   SMK_REQUIRE(p != nullptr, SMK_ERR_OOM, "host allocation failed");
   p->nx = nx; p->ny = ny; p->nz = nz; p->m = nz / 2; p->nzh = nz / 2 + 1; p->cell = cell;
   for (int k = 0; k < SMK_PASS_COUNT; ++k) {
-    p->vid[k] = k == SMK_PASS_Z_R2C   ? default_pencil(p->m, false)
-                : k == SMK_PASS_Z_C2R ? default_pencil(p->m, true)
+    const int64_t np = (int64_t)nx * ny;
+    p->vid[k] = k == SMK_PASS_Z_R2C   ? smk_route::box_pencil(p->m, false, np)
+                : k == SMK_PASS_Z_C2R ? smk_route::box_pencil(p->m, true, np)
                                       : default_strided(k == SMK_PASS_Y_FWD || k == SMK_PASS_Y_INV ? ny : nx, k);
   }
   p->n_partial = strided_blocks_max(nx, MODE_SPECTRAL, (uint64_t)p->nzh, (uint32_t)ny);

@@ -6,6 +6,7 @@
 
 #include "fft_core.h"
 #include "fft_lengths.h"
+#include "route.h"
 #include "smk_internal.h"
 
 namespace smk_box {
@@ -490,13 +491,15 @@ __global__ __launch_bounds__(T*(N / E)) __attribute__((amdgpu_waves_per_eu(2))) 
 // Output: trans == 0 -> numpy layout K[x][y][kz]; trans == 1 -> K[x][kz][y]
 // (the store phase then runs with lanes ordered pencil-fastest, i.e. along y).
 // Pencils pencil0 .. n_pencils-1 (a launch may cover a slab of the box).
-template <int M, int E, int T>
+// SWB: 0, or LINE_PADDED for padded LDS lines where the length has none (LdsMap).
+template <int M, int E, int T, int SWB>
 __global__ __launch_bounds__(T*(M / E)) void k_z_r2c(const float* __restrict__ noise, uint64_t seed,
                                                      float2* __restrict__ K, const float2* __restrict__ tw,
                                                      const float2* __restrict__ twr, uint64_t pencil0,
                                                      uint64_t n_pencils, int trans, uint32_t ny) {
   constexpr int P = M / E;
-  constexpr int LL = lds_line_len(M);
+  constexpr int LL = lds_line_len(M, SWB);
+  using LM = LdsMap<M, 0, SWB>;
   constexpr int NT = T * P;
   __shared__ float2 lds[T * LL];
   const int tid = threadIdx.x;
@@ -520,8 +523,8 @@ __global__ __launch_bounds__(T*(M / E)) void k_z_r2c(const float* __restrict__ n
           box_muller_hw(u.x, u.y, n0, n1);
           box_muller_hw(u.z, u.w, n2, n3);
           float2* ln = lds + tt * LL;
-          ln[lds_pos<M>(2 * qq)] = make_float2(n0, n1);
-          ln[lds_pos<M>(2 * qq + 1)] = make_float2(n2, n3);
+          ln[LM::slot(2 * qq, 0)] = make_float2(n0, n1);
+          ln[LM::slot(2 * qq + 1, 0)] = make_float2(n2, n3);
         }
       }
     } else {
@@ -536,12 +539,12 @@ __global__ __launch_bounds__(T*(M / E)) void k_z_r2c(const float* __restrict__ n
           float n0, n1;
           if (g % 2 == 0) box_muller_hw(u.x, u.y, n0, n1);
           else box_muller_hw(u.z, u.w, n0, n1);
-          lds[tt * LL + lds_pos<M>(n)] = make_float2(n0, n1);
+          lds[tt * LL + LM::slot(n, 0)] = make_float2(n0, n1);
         }
       }
     }
     __syncthreads();
-    lds_gather<M, P, E>(v, line, p);
+    lds_gather<M, P, E, 0, SWB>(v, line, p);
     __syncthreads();
   } else {
     const float2* src = reinterpret_cast<const float2*>(noise) + L * M;
@@ -549,9 +552,9 @@ __global__ __launch_bounds__(T*(M / E)) void k_z_r2c(const float* __restrict__ n
     for (int e = 0; e < E; ++e) v[e] = valid ? src[p + P * e] : make_float2(0.f, 0.f);
   }
 
-  fft_line_e<M, E, false>(v, line, p, tw);
+  fft_line_e<M, E, false, 0, SWB>(v, line, p, tw);
 
-  lds_scatter<M, P, E>(v, line, p);
+  lds_scatter<M, P, E, 0, SWB>(v, line, p);
   __syncthreads();
   // store phase: (ts, ps) is the lane's (pencil, point) role
   const int ts = trans ? tid % T : t;
@@ -572,15 +575,15 @@ __global__ __launch_bounds__(T*(M / E)) void k_z_r2c(const float* __restrict__ n
 #pragma unroll
   for (int e = 0; e < E; ++e) {
     const int k = ps + P * e;
-    const float2 zk = sl[lds_pos<M>(k)];
-    const float2 zc = cconj(sl[lds_pos<M>((M - k) % M)]);
+    const float2 zk = sl[LM::slot(k, 0)];
+    const float2 zc = cconj(sl[LM::slot((M - k) % M, 0)]);
     const float2 ze = cscale(cadd(zk, zc), 0.5f);
     const float2 zo = mul_mi<false>(cscale(csub(zk, zc), 0.5f));
     const float2 x = cadd(ze, cmul(twr[k], zo));
     if (vs) dst[k * sk] = x;
   }
   if (ps == 0 && vs) {
-    const float2 z0 = sl[lds_pos<M>(0)];
+    const float2 z0 = sl[LM::slot(0, 0)];
     dst[(uint64_t)M * sk] = make_float2(z0.x - z0.y, 0.0f);
   }
 }
@@ -610,6 +613,7 @@ __global__ __launch_bounds__(T*(M / E)) void k_z_c2r(const float2* __restrict__ 
                                                      int slot_mask) {
   constexpr int P = M / E;
   constexpr int LL = lds_line_len(M);
+  using LM = LdsMap<M, 0, 0>;
   __shared__ float2 xnyq[T];
   const int tid = threadIdx.x;
   const int p = tid % P, t = tid / P;
@@ -632,7 +636,7 @@ __global__ __launch_bounds__(T*(M / E)) void k_z_c2r(const float2* __restrict__ 
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       const int k = p1 + P * e;
-      v[e] = c2r_fold(v[e], (k == 0) ? xnyq[t] : line[lds_pos<M>(M - k)], k, twr1);
+      v[e] = c2r_fold(v[e], (k == 0) ? xnyq[t] : line[LM::slot(M - k, 0)], k, twr1);
     }
     __syncthreads();
     fft_line_e<M, E, true>(v, line, p, tw);
@@ -641,21 +645,21 @@ __global__ __launch_bounds__(T*(M / E)) void k_z_c2r(const float2* __restrict__ 
     float* lf = ldf + t * LL;
     float xr[E];
 #pragma unroll
-    for (int e = 0; e < E; ++e) lf[lds_pos<M>(p + P * e)] = v[e].x;
+    for (int e = 0; e < E; ++e) lf[LM::slot(p + P * e, 0)] = v[e].x;
     __syncthreads();
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       const int k = p1 + P * e;
-      xr[e] = (k == 0) ? xnyq[t].x : lf[lds_pos<M>(M - k)];
+      xr[e] = (k == 0) ? xnyq[t].x : lf[LM::slot(M - k, 0)];
     }
     __syncthreads();
 #pragma unroll
-    for (int e = 0; e < E; ++e) lf[lds_pos<M>(p + P * e)] = v[e].y;
+    for (int e = 0; e < E; ++e) lf[LM::slot(p + P * e, 0)] = v[e].y;
     __syncthreads();
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       const int k = p1 + P * e;
-      const float xi = (k == 0) ? xnyq[t].y : lf[lds_pos<M>(M - k)];
+      const float xi = (k == 0) ? xnyq[t].y : lf[LM::slot(M - k, 0)];
       v[e] = c2r_fold(v[e], make_float2(xr[e], xi), k, twr1);
     }
     __syncthreads();
@@ -906,27 +910,30 @@ inline bool pencil_variant_ok(int m, int vid, bool c2r) {
   return vid >= 0 && vid < SMK_NPVAR && pencil_E(m, vid) != 0 && (c2r || pencil_XCH(vid) == 0);
 }
 
-// The z passes' variant a plan starts with (ms against variant 0): R2C of 320
-// complex points 0.43 against 0.65 and 384 1.94 against 2.18; C2R of 320 1.00
-// against 1.17, 384 8.7 against 8.9 and 768 32.5 against 35.4.
-constexpr int default_pencil(int m, bool c2r) {
-  return c2r ? (m == 320 ? 1 : m == 384 || m == 768 ? 2 : 0) : (m == 320 || m == 384 ? 1 : 0);
+template <int M, int VID, int SWB>
+hipError_t launch_z_r2c_swb(const float* noise, uint64_t seed, float2* K, const float2* tw, const float2* twr,
+                            uint64_t p0, uint64_t np, int trans, uint32_t ny, hipStream_t s) {
+  constexpr int E = pencil_E(M, VID);
+  constexpr int T = pencil_T(M, E);
+  const uint64_t nblk = (np - p0 + T - 1) / T;
+  if (nblk > 0x7fffffffull) return hipErrorInvalidConfiguration;
+  hipLaunchKernelGGL((k_z_r2c<M, E, T, SWB>), dim3((uint32_t)nblk), dim3(T * (M / E)), 0, s, noise, seed, K, tw, twr,
+                     p0, np, trans, ny);
+  return hipGetLastError();
 }
 
 template <int M, int VID>
 hipError_t launch_z_r2c_v(const float* noise, uint64_t seed, float2* K, const float2* tw, const float2* twr,
                           uint64_t p0, uint64_t np, int trans, uint32_t ny, hipStream_t s) {
-  constexpr int E = pencil_E(M, VID);
-  if constexpr (E == 0) {
+  if constexpr (pencil_E(M, VID) == 0) {
     return hipErrorInvalidValue;
   } else {
-    constexpr int T = pencil_T(M, E);
     if (np <= p0) return hipSuccess;
-    const uint64_t nblk = (np - p0 + T - 1) / T;
-    if (nblk > 0x7fffffffull) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL((k_z_r2c<M, E, T>), dim3((uint32_t)nblk), dim3(T * (M / E)), 0, s, noise, seed, K, tw, twr,
-                       p0, np, trans, ny);
-    return hipGetLastError();
+    if constexpr (M == 1280) {
+      if (smk_route::box_r2c_padded(VID, trans != 0, (int64_t)np))
+        return launch_z_r2c_swb<M, VID, LINE_PADDED>(noise, seed, K, tw, twr, p0, np, trans, ny, s);
+    }
+    return launch_z_r2c_swb<M, VID, 0>(noise, seed, K, tw, twr, p0, np, trans, ny, s);
   }
 }
 

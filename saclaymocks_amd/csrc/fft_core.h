@@ -302,14 +302,17 @@ __host__ __device__ constexpr int elems_per_thread(int n) {
 }
 
 // LDS line stride (in float2): one pad slot every 32 points breaks the
-// power-of-two strides of the early Stockham stages across banks.  The
-// 2560-point line is left unpadded so that four lines fill exactly 80 KiB and
-// two blocks share one CU's 160 KiB.
+// power-of-two strides of the early Stockham stages across banks.  The 1280-
+// and 2560-point lines are left unpadded so that eight and four of them fill
+// exactly 80 KiB and two blocks share one CU's 160 KiB.
 __host__ __device__ constexpr bool lds_padded(int n) { return n != 2560 && n != 1280; }
 template <int N> __host__ __device__ constexpr int lds_pos(int pos) {
   return lds_padded(N) ? pos + (pos >> 5) : pos;
 }
-__host__ __device__ constexpr int lds_line_len(int n) { return lds_padded(n) ? n + (n >> 5) + 1 : n; }
+constexpr int LINE_PADDED = -1;   // for SWB (see LdsMap)
+__host__ __device__ constexpr int lds_line_len(int n, int swb = 0) {
+  return lds_padded(n) || swb == LINE_PADDED ? n + (n >> 5) + 1 : n;
+}
 
 // A zero the compiler cannot see through.  Adding it to a table pointer at
 // the start of each stage keeps that stage's loads inside the stage: without
@@ -322,15 +325,16 @@ __device__ __forceinline__ int opaque_zero() {
   return z;
 }
 
-// Slot of point `pos` in an LDS line.  Padded lines (every length but 2560)
-// insert one slot every 32 points.  The unpadded 2560-point line instead
-// XORs bits [SWS, SWS + SWB) of the position with the lane's swizzle `sw`
+// Slot of point `pos` in an LDS line.  Padded lines (every length but 1280 and
+// 2560, and these with SWB = LINE_PADDED, of lds_line_len(N, LINE_PADDED)
+// slots) insert one slot every 32 points.  The unpadded lines instead
+// XOR bits [SWS, SWS + SWB) of the position with the lane's swizzle `sw`
 // (its line index within the block, shifted by SWS): the lines of a block
 // start a multiple of 64 banks apart and the lanes of a wave interleave them.
 // fold(slot(x), C) = slot(x + C) for a compile-time C that is a multiple of G,
 // which turns the LDS addresses of a stage into one base plus immediates.
 template <int N, int SWS, int SWB> struct LdsMap {
-  static constexpr bool padded = lds_padded(N);
+  static constexpr bool padded = lds_padded(N) || SWB == LINE_PADDED;
   static constexpr int G = padded ? 32 : (1 << (SWS + SWB));
   static __device__ __forceinline__ uint32_t slot(uint32_t pos, uint32_t sw) {
     if constexpr (padded) return pos + (pos >> 5);

@@ -112,4 +112,29 @@ constexpr bool gather_radial(int dmax, int64_t n, int64_t pixels, double cells) 
   return dmax > 1 || (cells <= 2.75 && cells >= -2.75);
 }
 
+// -------------------------------------------------------------- box passes
+// The variant (box_kernels.h) of a z pass that a plan starts with, for pencils
+// of m complex points: ms against variant 0, R2C of 320 points 0.43 against 0.65
+// and 384 1.94 against 2.18; C2R of 320 1.00 against 1.17, 384 8.7 against 8.9
+// and 768 32.5 against 35.4; of 1280 the C2R takes us with variant 1 and 0
+//   pencils   64^2      200^2     320^2     512^2       640^2
+//             27  36    191  246  475  592  1190  1410  1850  2140
+// and the R2C into [x][kz][y] with 1 and 0, with lines padded (p) and not
+//   1p        32        242       755       2935        4920
+//   0p        52        330       820       2190        3980
+//   0         37        271       725       2640        4570
+// (in the numpy layout, with the x and y passes, 1 and 0 not padded: 59 66,
+// 708 762, 1280 1400, 3410 3700, 5385 5720).
+constexpr int box_pencil(int m, bool c2r, int64_t pencils) {
+  if (m == 1280) return c2r || pencils < 70000 ? 1 : 0;
+  return c2r ? (m == 320 ? 1 : m == 384 || m == 768 ? 2 : 0) : (m == 320 || m == 384 ? 1 : 0);
+}
+
+// Whether an R2C of 1280 points pads its LDS lines: one that stores with the
+// lanes along y reads one point of several lines, which unpadded lie in the same
+// banks, but more of these fit a CU.
+constexpr bool box_r2c_padded(int variant, bool trans, int64_t pencils) {
+  return trans && (variant == 1 || pencils >= 200000);
+}
+
 }  // namespace smk_route
