@@ -184,8 +184,10 @@ struct smk_box_plan {
   float* ky;
   float* kz;
   uint64_t n_partial;
-  // pass variants, indexed by SMK_PASS_*
+  // pass variants, indexed by SMK_PASS_*; and the spectral pass's without an aux
+  // field, the same once it has been set
   int vid[SMK_PASS_COUNT];
+  int vid_no_aux;
 };
 
 extern "C" int smk_fft_length_supported(int n) { return length_supported(n) ? 1 : 0; }
@@ -206,8 +208,9 @@ extern "C" int smk_box_plan_create(smk_box_plan** plan, int nx, int ny, int nz, 
     const int64_t np = (int64_t)nx * ny;
     p->vid[k] = k == SMK_PASS_Z_R2C   ? smk_route::box_pencil(p->m, false, np)
                 : k == SMK_PASS_Z_C2R ? smk_route::box_pencil(p->m, true, np)
-                                      : default_strided(k == SMK_PASS_Y_FWD || k == SMK_PASS_Y_INV ? ny : nx, k);
+                                      : smk_route::box_strided(k == SMK_PASS_Y_FWD || k == SMK_PASS_Y_INV ? ny : nx, k, true);
   }
+  p->vid_no_aux = smk_route::box_strided(nx, SMK_PASS_X_SPECTRAL, false);
   p->n_partial = strided_blocks_max(nx, MODE_SPECTRAL, (uint64_t)p->nzh, (uint32_t)ny);
 
   auto upload = [](void** dst, const void* src, size_t bytes) -> hipError_t {
@@ -430,7 +433,7 @@ namespace {
 
 // Arguments of the spectral x pass over kz planes [k0, k1).
 StridedArgs spectral_args(const smk_box_plan* p, const float2* in, float2* out, float2* aux, const double* pk,
-                          int aux_kind, double aux_coef, double* partial, uint32_t k0) {
+                          int aux_kind, double aux_coef, double* partial, int vx, uint32_t k0) {
   StridedArgs a = tr_x_args(p, in, out);
   a.in = in + (uint64_t)k0 * a.in_so;
   a.out = out + (uint64_t)k0 * a.out_so;
@@ -450,7 +453,7 @@ StridedArgs spectral_args(const smk_box_plan* p, const float2* in, float2* out, 
   a.write_delta = 1;
   a.nz_nyq = (uint32_t)p->m;
   a.kz0 = k0;
-  a.partial = partial + strided_blocks(p->nx, MODE_SPECTRAL, p->vid[SMK_PASS_X_SPECTRAL], k0, (uint32_t)p->ny);
+  a.partial = partial + strided_blocks(p->nx, MODE_SPECTRAL, vx, k0, (uint32_t)p->ny);
   return a;
 }
 
@@ -502,7 +505,8 @@ extern "C" int smk_grf_box(smk_box_plan* p, uint64_t seed, const float* noise, c
   double* partial = (double*)((char*)workspace + nbox * kb);
   const uint64_t np = (uint64_t)p->nx * p->ny;
   const bool has_aux = aux_kind != SMK_AUX_NONE;
-  const int vzr = p->vid[SMK_PASS_Z_R2C], vyf = p->vid[SMK_PASS_Y_FWD], vx = p->vid[SMK_PASS_X_SPECTRAL];
+  const int vzr = p->vid[SMK_PASS_Z_R2C], vyf = p->vid[SMK_PASS_Y_FWD];
+  const int vx = has_aux ? p->vid[SMK_PASS_X_SPECTRAL] : p->vid_no_aux;
   const int vyi = p->vid[SMK_PASS_Y_INV], vz = p->vid[SMK_PASS_Z_C2R];
 
   int rc = harvest_timing(p);
@@ -529,7 +533,7 @@ extern "C" int smk_grf_box(smk_box_plan* p, uint64_t seed, const float* noise, c
     SMK_HIP_RET(timed(p, 1, s, [&] {
       return launch_strided<MODE_FWD>(p->ny, vyf, tr_y_fwd_args(p, A1, A2), (uint64_t)p->nzh, s);
     }));
-    const StridedArgs a = spectral_args(p, A2, A1, has_aux ? A3 : nullptr, pk_params, aux_kind, aux_coef, partial, 0);
+    const StridedArgs a = spectral_args(p, A2, A1, has_aux ? A3 : nullptr, pk_params, aux_kind, aux_coef, partial, vx, 0);
     SMK_HIP_RET(timed(p, 2, s, [&] { return launch_strided<MODE_SPECTRAL>(p->nx, vx, a, (uint64_t)p->nzh, s); }));
     if (var_out) {
       hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(1024), 0, s, partial, nb_spec, var_out, slots);
@@ -589,7 +593,7 @@ extern "C" int smk_grf_box(smk_box_plan* p, uint64_t seed, const float* noise, c
     for (int i = 0; i < S; ++i) {
       const uint32_t k0 = slab_bound((uint32_t)p->nzh, S, i, 8), k1 = slab_bound((uint32_t)p->nzh, S, i + 1, 8);
       if (k1 <= k0) continue;
-      const StridedArgs a = spectral_args(p, A2, A1, has_aux ? A3 : nullptr, pk_params, aux_kind, aux_coef, partial,
+      const StridedArgs a = spectral_args(p, A2, A1, has_aux ? A3 : nullptr, pk_params, aux_kind, aux_coef, partial, vx,
                                           k0);
       SMK_HIP_RET(timed(p, 2, s1, [&] {
         return launch_strided<MODE_SPECTRAL>(p->nx, vx, a, (uint64_t)(k1 - k0), s1);
@@ -664,6 +668,7 @@ extern "C" int smk_box_set_variant(smk_box_plan* p, int kind, int vid) {
   SMK_REQUIRE(variant_valid(p, kind, vid), SMK_ERR_UNSUPPORTED, "variant %d does not exist for pass kind %d", vid,
               kind);
   p->vid[kind] = vid;
+  if (kind == SMK_PASS_X_SPECTRAL) p->vid_no_aux = vid;
   return SMK_OK;
 }
 
@@ -681,6 +686,7 @@ extern "C" int smk_box_autotune(smk_box_plan* p, uint64_t seed, const float* noi
   const int nv = SMK_NVAR > SMK_NPVAR ? SMK_NVAR : SMK_NPVAR;
   int saved[SMK_PASS_COUNT];
   memcpy(saved, p->vid, sizeof(saved));
+  const int saved_no_aux = p->vid_no_aux;
   // variants are timed in the sequential schedule (one pass at a time); the
   // workspace of either schedule is large enough for it
   const int saved_nslab = p->nslab;
@@ -705,6 +711,7 @@ extern "C" int smk_box_autotune(smk_box_plan* p, uint64_t seed, const float* noi
       p->vid[k] = ok ? v : 0;
       any = any || ok;
     }
+    p->vid_no_aux = p->vid[SMK_PASS_X_SPECTRAL];
     if (!any) continue;
     for (int r = 0; r <= reps && rc == SMK_OK; ++r) {
       rc = smk_grf_box(p, seed, noise, pk_params, aux_kind, aux_coef, delta_out, aux_out, workspace, var_out,
@@ -737,9 +744,11 @@ extern "C" int smk_box_autotune(smk_box_plan* p, uint64_t seed, const float* noi
   p->nslab = saved_nslab;
   if (rc) {
     memcpy(p->vid, saved, sizeof(saved));
+    p->vid_no_aux = saved_no_aux;
     return rc;
   }
   for (int k = 0; k < NK; ++k) p->vid[k] = best[k];
+  p->vid_no_aux = best[SMK_PASS_X_SPECTRAL];
   return rc2;
 }
 

@@ -3,6 +3,8 @@
 #pragma once
 #include <cstdint>
 
+#include "../../include/saclaymocks_hip.h"
+
 namespace smk_route {
 
 // ------------------------------------------------------------ P(k) tables
@@ -135,6 +137,53 @@ constexpr int box_pencil(int m, bool c2r, int64_t pencils) {
 // banks, but more of these fit a CU.
 constexpr bool box_r2c_padded(int variant, bool trans, int64_t pencils) {
   return trans && (variant == 1 || pencils >= 200000);
+}
+
+// The variant of an x or y pass of n points that a plan starts with.  What
+// decides is the lines per block that half of a CU's LDS holds (the transposed
+// runs are 8 B per line) against the waves that the register tile leaves: the
+// split exchange buys lines, the half tile waves.  Measured per pass, in ms
+// against variant 0, at 320^3, 384^3, ... 1280 x 1280 x 512 and 2560 x 1280 x 768:
+//   y, x forward   320 18 (0.051, 0.056)  384 18 (0.114, 0.128)
+//                  512 17 (0.327, 0.362)  640 17 (0.482, 0.518)
+//                  768 17 (0.750, 0.875)  1024 3 (1.17, 1.59)
+//                  1280 6 (4.34, 4.68)    1536 3 (2.37, 3.04)
+//                  2048 3 (3.48, 4.94)
+//   y inverse      320 18 (0.147, 0.165)  384 18 (0.251, 0.273)
+//                  640 6 (1.02, 1.11)     768 18 (1.81, 2.05)
+//                  1024 3 (2.60, 2.81)    1280 6 (9.1, 10.4)
+//                  1536 6 (5.41, 5.79)    2048 3 (7.9, 11.9)
+//   x inverse      as forward; in the numpy layout 1280 17 (2.42, 2.55 the
+//                  whole inverse), 2560 4 (4.86, 5.26)
+//   x spectral     320 18 (0.153, 0.164)  384 17 (0.263, 0.288)
+//                  512 16 (0.530, 0.634)  640 10 (1.12, 1.55)
+//                  768 3 (1.85, 2.00)     1024 14 (2.57, 2.94)
+//                  1280 12 (3.53, 4.57)   1536 3 (5.95, 7.18)
+//                  2048 14 (5.68, 6.44)   2560 1 (13.2, 17.0)
+// Without an aux field the spectral pass has two line FFTs instead of three or
+// four, and the variants that keep a second register tile for it lose: us of the
+// pass with 16 or 14 against 0, 512^3 390, 342; 1024 x 512 x 512 939, 822; 2048 x
+// 512 x 256 920, 856 (320, 384, 640, 768, 1280, 1536 and 2560 win without one too).
+// Of the other lengths the general ones have variant 0 only; 4096 has others,
+// which were not measured.
+constexpr int box_strided(int n, int kind, bool aux) {
+  const bool p2 = n == 1024 || n == 2048;
+  switch (kind) {
+    case SMK_PASS_X_SPECTRAL:
+      if (!aux && (p2 || n == 512)) return 0;
+      return n == 320 ? 18 : n == 384 ? 17 : n == 512 ? 16 : n == 640 ? 10 : n == 768 || n == 1536 ? 3 : p2 ? 14
+             : n == 1280 ? 12 : n == 2560 ? 1 : 0;
+    case SMK_PASS_Y_INV:
+      return n == 320 || n == 384 || n == 768 ? 18 : n == 640 || n == 1280 || n == 1536 ? 6 : p2 ? 3 : 0;
+    case SMK_PASS_X_INV:
+      if (n == 1280) return 17;
+      if (n == 2560) return 4;
+      [[fallthrough]];
+    case SMK_PASS_Y_FWD:
+    case SMK_PASS_X_FWD:
+      return n == 320 || n == 384 ? 18 : n == 512 || n == 640 || n == 768 ? 17 : n == 1280 ? 6 : p2 || n == 1536 ? 3 : 0;
+    default: return 0;
+  }
 }
 
 }  // namespace smk_route
