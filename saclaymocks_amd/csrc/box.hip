@@ -208,9 +208,9 @@ extern "C" int smk_box_plan_create(smk_box_plan** plan, int nx, int ny, int nz, 
     const int64_t np = (int64_t)nx * ny;
     p->vid[k] = k == SMK_PASS_Z_R2C   ? smk_route::box_pencil(p->m, false, np)
                 : k == SMK_PASS_Z_C2R ? smk_route::box_pencil(p->m, true, np)
-                                      : smk_route::box_strided(k == SMK_PASS_Y_FWD || k == SMK_PASS_Y_INV ? ny : nx, k, true);
+                                      : smk_route::box_strided(k, nx, ny, nz, true);
   }
-  p->vid_no_aux = smk_route::box_strided(nx, SMK_PASS_X_SPECTRAL, false);
+  p->vid_no_aux = smk_route::box_strided(SMK_PASS_X_SPECTRAL, nx, ny, nz, false);
   p->n_partial = strided_blocks_max(nx, MODE_SPECTRAL, (uint64_t)p->nzh, (uint32_t)ny);
 
   auto upload = [](void** dst, const void* src, size_t bytes) -> hipError_t {

@@ -160,30 +160,65 @@ constexpr bool box_r2c_padded(int variant, bool trans, int64_t pencils) {
 //                  768 3 (1.85, 2.00)     1024 14 (2.57, 2.94)
 //                  1280 12 (3.53, 4.57)   1536 3 (5.95, 7.18)
 //                  2048 14 (5.68, 6.44)   2560 1 (13.2, 17.0)
+//
+// The split exchange pays for its barriers with longer runs, that is where the
+// passes are bound by memory, not where the work box lies in the caches; and it
+// leaves lanes idle where the inner extent is no multiple of its lines.  So each
+// holds from a size of the work box on (MB of nx ny (nz / 2 + 1) complex
+// numbers).  Us against variant 0 on both sides, boxes of n x a x c or a x n x c:
+//   y forward, numpy layout  512 17: 160^2 (53 MB) 79, 75   250x300 219, 213   400^2 571, 592
+//                            768 17: 160^2 (80) 108, 103    250x300 327, 315   400^2 805, 839
+//                            1024 3: 128^2 (68) 89, 86      200^2 243, 242     250x300 549, 597
+//                            2048 3: 64^2 (34) 62, 63       transposed 64^2 32, 27  200^2 183, 204
+//   y inverse, transposed    768 18: 100^2 (31) 29, 22      250x300 127, 116   400^2 252, 249
+//                            1024 3: 64^2 (17) 26, 20       256^2 (270) 178, 166  400^2 366, 366
+//                            1536 6: 100^2 (63) 53, 42      200^2 155, 143     400^2 550, 583
+//   x inverse, numpy layout  512 17: 160^2 (53) 125, 121    250x300 254, 260
+//   x spectral               384 17: 100^2 (16) 45, 34      256^2 (101) 114, 112  400^2 264, 269
+//                            768 3:  32^2 (3) 35, 32        128^2 (51) 73, 79
+// With ny a multiple of 128 the points of an x line are a multiple of 1 KB apart,
+// in few of the memory's channels, and longer runs pay sooner: x forward of 512
+// and 768 x 256 x 256 143, 166 and 217, 257.
+//
 // Without an aux field the spectral pass has two line FFTs instead of three or
 // four, and the variants that keep a second register tile for it lose: us of the
 // pass with 16 or 14 against 0, 512^3 390, 342; 1024 x 512 x 512 939, 822; 2048 x
 // 512 x 256 920, 856 (320, 384, 640, 768, 1280, 1536 and 2560 win without one too).
 // Of the other lengths the general ones have variant 0 only; 4096 has others,
 // which were not measured.
-constexpr int box_strided(int n, int kind, bool aux) {
-  const bool p2 = n == 1024 || n == 2048;
-  switch (kind) {
-    case SMK_PASS_X_SPECTRAL:
-      if (!aux && (p2 || n == 512)) return 0;
-      return n == 320 ? 18 : n == 384 ? 17 : n == 512 ? 16 : n == 640 ? 10 : n == 768 || n == 1536 ? 3 : p2 ? 14
-             : n == 1280 ? 12 : n == 2560 ? 1 : 0;
-    case SMK_PASS_Y_INV:
-      return n == 320 || n == 384 || n == 768 ? 18 : n == 640 || n == 1280 || n == 1536 ? 6 : p2 ? 3 : 0;
-    case SMK_PASS_X_INV:
-      if (n == 1280) return 17;
-      if (n == 2560) return 4;
-      [[fallthrough]];
-    case SMK_PASS_Y_FWD:
-    case SMK_PASS_X_FWD:
-      return n == 320 || n == 384 ? 18 : n == 512 || n == 640 || n == 768 ? 17 : n == 1280 ? 6 : p2 || n == 1536 ? 3 : 0;
-    default: return 0;
+struct BoxDefault {
+  int n, variant;
+  int mb[2];   // from this size of the work box on: y, x forward; y, x inverse; both the same for the spectral pass
+};
+
+constexpr int box_strided(int kind, int nx, int ny, int nz, bool aux) {
+  constexpr BoxDefault forward[] = {{320, 18, {45, 45}},  {384, 18, {95, 45}},  {512, 17, {250, 250}},
+                                    {640, 17, {100, 60}}, {768, 17, {300, 300}}, {1024, 3, {250, 90}},
+                                    {1280, 6, {0, 0}},    {1536, 3, {20, 20}},  {2048, 3, {160, 30}}};
+  constexpr BoxDefault y_inverse[] = {{320, 18, {45, 45}}, {384, 18, {150, 150}}, {640, 6, {0, 0}},
+                                      {768, 18, {450, 450}}, {1024, 3, {250, 250}}, {1280, 6, {0, 0}},
+                                      {1536, 6, {460, 460}}, {2048, 3, {160, 160}}};
+  constexpr BoxDefault x_inverse[] = {{320, 18, {45, 45}}, {384, 18, {60, 60}},  {512, 17, {150, 150}},
+                                      {640, 17, {45, 45}}, {768, 17, {75, 75}},  {1024, 3, {90, 90}},
+                                      {1280, 17, {80, 80}}, {1536, 3, {20, 20}}, {2048, 3, {60, 60}},
+                                      {2560, 4, {30, 30}}};
+  constexpr BoxDefault spectral[] = {{320, 18, {45, 45}}, {384, 17, {200, 200}}, {512, 16, {0, 0}}, {640, 10, {0, 0}},
+                                     {768, 3, {30, 30}},  {1024, 14, {0, 0}},    {1280, 12, {0, 0}},
+                                     {1536, 3, {20, 20}}, {2048, 14, {0, 0}},    {2560, 1, {0, 0}}};
+  const bool x = kind == SMK_PASS_X_FWD || kind == SMK_PASS_X_INV;
+  const int n = kind == SMK_PASS_Y_FWD || kind == SMK_PASS_Y_INV ? ny : nx;
+  const bool aliased = x && (n == 512 || n == 768) && ny % 128 == 0;
+  if (kind == SMK_PASS_X_SPECTRAL && !aux && (n == 512 || n == 1024 || n == 2048)) return 0;
+  const BoxDefault* t = kind == SMK_PASS_Y_INV ? y_inverse : kind == SMK_PASS_X_INV ? x_inverse
+                        : kind == SMK_PASS_X_SPECTRAL ? spectral : forward;
+  const int len = kind == SMK_PASS_Y_INV ? 8 : kind == SMK_PASS_X_INV || kind == SMK_PASS_X_SPECTRAL ? 10 : 9;
+  const double mb = 8e-6 * nx * ny * (nz / 2 + 1);
+  for (int i = 0; i < len; ++i) {
+    if (t[i].n != n) continue;
+    const int from = t[i].mb[x ? 1 : 0];
+    return mb >= (aliased && from > 100 ? 100 : from) ? t[i].variant : 0;
   }
+  return 0;
 }
 
 }  // namespace smk_route

@@ -8,7 +8,7 @@ from route_rules import build
 @pytest.fixture(scope="module")
 def rule(tmp_path_factory):
     return build(tmp_path_factory.mktemp("rule"),
-                 "int spectral(int n, int aux) { return box_strided(n, SMK_PASS_X_SPECTRAL, aux); }").spectral
+                 "int spectral(int n, int aux) { return box_strided(SMK_PASS_X_SPECTRAL, n, 512, 512, aux); }").spectral
 
 
 @pytest.mark.parametrize("n,with_aux,without", [(512, 16, 0), (1024, 14, 0), (2048, 14, 0), (640, 10, 10), (1280, 12, 12),
