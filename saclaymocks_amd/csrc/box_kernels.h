@@ -528,18 +528,19 @@ __global__ __launch_bounds__(T*(M / E)) void k_z_r2c(const float* __restrict__ n
         }
       }
     } else {
-      // every other pencil begins in the middle of a call: each point takes
-      // its half of the call its two cells are in
-      for (int q = tid; q < T * M; q += NT) {
-        const int tt = q / M, n = q % M;
-        const uint64_t LL_ = L0 + tt;
-        if (LL_ < n_pencils) {
-          const uint64_t g = LL_ * (uint64_t)M + n;
-          const U4 u = philox4x32_10(g / 2, seed);
-          float n0, n1;
-          if (g % 2 == 0) box_muller_hw(u.x, u.y, n0, n1);
-          else box_muller_hw(u.z, u.w, n0, n1);
-          lds[tt * LL + LM::slot(n, 0)] = make_float2(n0, n1);
+      // every other pencil begins in the middle of a call, so the calls run
+      // through the block's pencils, whose points follow each other
+      const uint64_t g0 = L0 * (uint64_t)M;
+      const int lead = (int)(g0 & 1);
+      for (int q = tid; q < (T * M + lead + 1) / 2; q += NT) {
+        const U4 u = philox4x32_10(g0 / 2 + (uint64_t)q, seed);
+        float2 n[2];
+        box_muller_hw(u.x, u.y, n[0].x, n[0].y);
+        box_muller_hw(u.z, u.w, n[1].x, n[1].y);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int i = 2 * q + h - lead, tt = i / M;
+          if (i >= 0 && i < T * M && L0 + tt < n_pencils) lds[tt * LL + LM::slot(i - tt * M, 0)] = n[h];
         }
       }
     }
