@@ -731,21 +731,22 @@ __global__ __launch_bounds__(M / 8) __attribute__((amdgpu_waves_per_eu(2))) void
 // the two forests' pk (NJ each, NJ = M/4 + 1 >= N/2 + 1) and the bins; then
 // the edges and the bin runs
 __host__ __device__ constexpr size_t pair_fixed_bytes(int M) { return blue_line_bytes_m(M); }
-// Points per thread of k_p1d_blue_pair<M>.  One block of 512 threads fills a
+// Points per thread of k_p1d_blue_pair<M, E>.  One block of 512 threads fills a
 // CU's registers at M = 4096, which leaves every barrier and load bare; with
 // 16 points on 256 threads two blocks fit, and an FFT has three stages instead
 // of four.  10000 pairs of 1025 to 1500 points: the forward pass 794 -> 660 us;
 // M = 2048 takes 390 either way (513 to 1020 points), 428 before with its pk
-// outside the line.
-constexpr int pair_E(int M) { return M == 4096 ? 16 : 8; }
-// The same of k_p1d_adjoint_blue_pair<M>, and what it keeps in registers.  The
+// outside the line.  Where every pair has a CU of its own nothing shares it, and
+// 512 threads are the sooner done (smk_route::fit_pair_points).
+//
+// The same of k_p1d_adjoint_blue_pair<M, E>, and what it keeps in registers.  The
 // FGPA part on the transform's registers instead of x and A in LDS (100 KB at
 // M = 4096, one block per CU; two passes over the pixels and two reductions):
 // with the forward pass 10000 pairs of 1025 to 1500 points 1916 -> 1505 us, of
 // 513 to 1020 1048 -> 900.  M = 4096 with 8 points and all kept: 1610; M = 2048
 // with 16: as with 8.
-constexpr int adj_pair_E(int M) { return M == 4096 ? 16 : 8; }
-constexpr int adj_pair_keep(int M) { return f64::KEEP_W | (M == 4096 ? f64::LATE_B : f64::KEEP_B); }
+constexpr int pair_keep(int M, int E) { return M == 4096 && E == 8 ? f64::KEEP_B | f64::KEEP_W : 0; }
+constexpr int adj_pair_keep(int M, int E) { return f64::KEEP_W | (E == 16 ? f64::LATE_B : f64::KEEP_B); }
 
 // The members (s1, s2) of pair w that take M's size class: each must still
 // have a table of this size class, the second one of the same length and
@@ -834,9 +835,9 @@ __device__ __forceinline__ void desc_members(const Args& a, const PairDesc& d, i
 // pairs [pair_lo, pair_hi) are those of M's size class.  Persistent: block
 // b takes pairs pair_lo + b + k gridDim.x, with the members' descriptors
 // loaded a pair ahead and the pair list entry two pairs ahead.
-template <int M>
-__global__ __launch_bounds__(M / pair_E(M)) __attribute__((amdgpu_waves_per_eu(2))) void k_p1d_blue_pair(P1dArgs a) {
-  constexpr int E = pair_E(M), NT = M / E;
+template <int M, int E>
+__global__ __launch_bounds__(M / E) __attribute__((amdgpu_waves_per_eu(2))) void k_p1d_blue_pair(P1dArgs a) {
+  constexpr int NT = M / E;
   constexpr int NJ = M / 4 + 1;
   static_assert((size_t)(f64::line_len(M) - M / 2) * 16 >= (size_t)NJ * 16 + (size_t)(NJ + 1) * 4,
                 "a pair's pk and bins must fit past the outputs in the line");
@@ -886,7 +887,7 @@ __global__ __launch_bounds__(M / pair_E(M)) __attribute__((amdgpu_waves_per_eu(2
     const double inv2 = s2 >= 0 ? 1.0 / a.fmean[set2] : 0.0;
     const int nj = nq / 2 + 1;
     const double2* T = a.tables + tb;
-    f64::bluestein_tab<M, E>(
+    f64::bluestein_tab<M, E, pair_keep(M, E)>(
         nq, nq,
         [&](int q) {
           double acc1 = 0.0, acc2 = 0.0;
@@ -1392,10 +1393,10 @@ __global__ __launch_bounds__(M / 8) __attribute__((amdgpu_waves_per_eu(2))) void
 // (adj_fgpa) of both forests runs on the registers that hold A, with one block
 // reduction of fourteen sums.  LDS: the line (c1 and c2 over its start), the
 // edges.
-template <int M>
-__global__ __launch_bounds__(M / adj_pair_E(M)) __attribute__((amdgpu_waves_per_eu(2))) void k_p1d_adjoint_blue_pair(
+template <int M, int E>
+__global__ __launch_bounds__(M / E) __attribute__((amdgpu_waves_per_eu(2))) void k_p1d_adjoint_blue_pair(
     AdjArgs a) {
-  constexpr int E = adj_pair_E(M), NT = M / E;
+  constexpr int NT = M / E;
   extern __shared__ double dyn[];
   double2* line = reinterpret_cast<double2*>(dyn);
   double* ledges = reinterpret_cast<double*>(reinterpret_cast<char*>(dyn) + blue_line_bytes_m(M));
@@ -1508,7 +1509,7 @@ __global__ __launch_bounds__(M / adj_pair_E(M)) __attribute__((amdgpu_waves_per_
       return make_double2(0.5 * v.x, -0.5 * v.y);
     };
     double2 Z[E / 2];   // A of both forests at q = threadIdx.x + NT e
-    f64::bluestein_regs<M, E, adj_pair_keep(M)>(
+    f64::bluestein_regs<M, E, adj_pair_keep(M, E)>(
         Z, nq,
         [&](int n) {
           const double2 h1 = herm(c1, n), h2 = herm(c2, n);
@@ -1556,17 +1557,32 @@ __global__ __launch_bounds__(M / adj_pair_E(M)) __attribute__((amdgpu_waves_per_
         }
       }
     } else {
+      // m pixels per point, the loads of two of them together (the second at
+      // the first's index past the last), and the point's mean of F from them
+      const int64_t o2c = two ? o2 : o1;
 #pragma unroll
       for (int e = 0; e < E / 2; ++e) {
         const int q = (int)threadIdx.x + NT * e;
         if (q < nq) {
-          for (int r = 0; r < m; ++r) {
-            const int64_t i = (int64_t)q * m + r;
-            pixel(v, pr1, a.delta[o1 + i], ep[o1 + i], a.flux[o1 + i], Z[e].x / m);
-            if (two) pixel(v + 7, pr2, a.delta[o2 + i], ep[o2 + i], a.flux[o2 + i], Z[e].y / m);
+          double f1 = 0.0, f2 = 0.0;
+          for (int r = 0; r < m; r += 2) {
+            const bool both = r + 1 < m;
+            const int64_t i = (int64_t)q * m + r, j = both ? i + 1 : i;
+            const float d1[2] = {a.delta[o1 + i], a.delta[o1 + j]}, d2[2] = {a.delta[o2c + i], a.delta[o2c + j]};
+            const float e1[2] = {ep[o1 + i], ep[o1 + j]}, e2[2] = {ep[o2c + i], ep[o2c + j]};
+            const double F1[2] = {a.flux[o1 + i], a.flux[o1 + j]}, F2[2] = {a.flux[o2c + i], a.flux[o2c + j]};
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              if (h == 0 || both) {
+                f1 += F1[h];
+                f2 += F2[h];
+                pixel(v, pr1, d1[h], e1[h], F1[h], Z[e].x / m);
+                if (two) pixel(v + 7, pr2, d2[h], e2[h], F2[h], Z[e].y / m);
+              }
+            }
           }
-          v[0] += Z[e].x * point(o1, q);
-          if (two) v[7] += Z[e].y * point(o2, q);
+          v[0] += Z[e].x * (f1 / m);
+          if (two) v[7] += Z[e].y * (f2 / m);
         }
       }
     }
@@ -1993,17 +2009,25 @@ int resident_grid(const void* kern, int threads, size_t lds, int n) {
   return n < g ? (n > 0 ? n : 1) : (int)g;
 }
 
-template <int M>
-int launch_p1d_blue_pair(P1dArgs a, int lo, int hi, size_t tail, hipStream_t st) {
+template <int M, int E>
+int launch_p1d_blue_pair_e(P1dArgs a, int lo, int hi, size_t tail, hipStream_t st) {
   if (hi <= lo) return SMK_OK;
   a.pair_lo = lo;
   a.pair_hi = hi;
   const size_t lds = pair_fixed_bytes(M) + tail;
-  SMK_HIP_CHECK(hipFuncSetAttribute((const void*)k_p1d_blue_pair<M>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  const int grid = resident_grid((const void*)k_p1d_blue_pair<M>, M / pair_E(M), lds, hi - lo);
-  hipLaunchKernelGGL(k_p1d_blue_pair<M>, dim3(grid), dim3(M / pair_E(M)), lds, st, a);
+  SMK_HIP_CHECK(hipFuncSetAttribute((const void*)(k_p1d_blue_pair<M, E>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  const int grid = resident_grid((const void*)(k_p1d_blue_pair<M, E>), M / E, lds, hi - lo);
+  hipLaunchKernelGGL((k_p1d_blue_pair<M, E>), dim3(grid), dim3(M / E), lds, st, a);
   SMK_LAUNCH_CHECK();
   return SMK_OK;
+}
+
+template <int M>
+int launch_p1d_blue_pair(P1dArgs a, int lo, int hi, size_t tail, hipStream_t st) {
+  if constexpr (M == 4096) {
+    if (smk_route::fit_pair_points(hi - lo) == 16) return launch_p1d_blue_pair_e<M, 16>(a, lo, hi, tail, st);
+  }
+  return launch_p1d_blue_pair_e<M, 8>(a, lo, hi, tail, st);
 }
 
 template <int M>
@@ -2038,18 +2062,26 @@ int launch_adj_blue(const AdjArgs& a, dim3 grid, size_t tail, hipStream_t st) {
   return SMK_OK;
 }
 
-template <int M>
-int launch_adj_blue_pair(AdjArgs a, int lo, int hi, size_t tail, hipStream_t st) {
+template <int M, int E>
+int launch_adj_blue_pair_e(AdjArgs a, int lo, int hi, size_t tail, hipStream_t st) {
   if (hi <= lo) return SMK_OK;
   a.pair_lo = lo;
   a.pair_hi = hi;
   const size_t lds = blue_line_bytes_m(M) + tail;
-  SMK_HIP_CHECK(hipFuncSetAttribute((const void*)k_p1d_adjoint_blue_pair<M>,
+  SMK_HIP_CHECK(hipFuncSetAttribute((const void*)(k_p1d_adjoint_blue_pair<M, E>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  const int grid = resident_grid((const void*)k_p1d_adjoint_blue_pair<M>, M / adj_pair_E(M), lds, hi - lo);
-  hipLaunchKernelGGL(k_p1d_adjoint_blue_pair<M>, dim3(grid), dim3(M / adj_pair_E(M)), lds, st, a);
+  const int grid = resident_grid((const void*)(k_p1d_adjoint_blue_pair<M, E>), M / E, lds, hi - lo);
+  hipLaunchKernelGGL((k_p1d_adjoint_blue_pair<M, E>), dim3(grid), dim3(M / E), lds, st, a);
   SMK_LAUNCH_CHECK();
   return SMK_OK;
+}
+
+template <int M>
+int launch_adj_blue_pair(AdjArgs a, int lo, int hi, size_t tail, hipStream_t st) {
+  if constexpr (M == 4096) {
+    if (smk_route::fit_pair_points(hi - lo) == 16) return launch_adj_blue_pair_e<M, 16>(a, lo, hi, tail, st);
+  }
+  return launch_adj_blue_pair_e<M, 8>(a, lo, hi, tail, st);
 }
 
 template <int M>

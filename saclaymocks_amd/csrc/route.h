@@ -114,6 +114,11 @@ constexpr bool gather_radial(int dmax, int64_t n, int64_t pixels, double cells) 
   return dmax > 1 || (cells <= 2.75 && cells >= -2.75);
 }
 
+// ------------------------------------------- the fit's transforms in pairs
+// Points per thread of the pair kernels of 4096 points: with 16, two blocks fit
+// a CU; with 8, one of twice the threads.
+constexpr int fit_pair_points(int pairs) { return pairs > 256 ? 16 : 8; }
+
 // -------------------------------------------------------------- box passes
 // The variant (box_kernels.h) of a z pass that a plan starts with, for pencils
 // of m complex points: ms against variant 0, R2C of 320 points 0.43 against 0.65
