@@ -1599,7 +1599,7 @@ static void launch_radial_nt(hipStream_t st, const GatherArgs& a) {
 template <int NF, int DM>
 static void launch_gather_dm(hipStream_t st, const GatherArgs& a) {
   if constexpr (NF >= 7 && DM >= 1) {
-    if (smk_route::gather_radial(DM, a.sk.n, a.npix_total, a.sk.dr / a.box.cell)) {
+    if (smk_route::gather_radial(DM, NF, a.sk.n, a.npix_total, a.sk.dr / a.box.cell)) {
       launch_radial_nt<NF, DM, 256>(st, a);
       return;
     }

@@ -101,16 +101,34 @@ constexpr int flux_waves(int64_t n, int64_t pixels, bool per_pixel) {
 // `cells` cells apart.
 //
 // One cell per pixel (dmax 0) fits k_gather's L1.  A block of k_gather_radial
-// does one skewer at a time, so short skewers leave it idle: with seven fields
-// and 2e6 pixels in all, dmax 1 takes 488 us against 685 at 50 pixels per
-// skewer and 1005 against 790 at 20; dmax 2 13.0 ms against 15.9 and dmax 3 21.5
-// against 44.1 at 2.  And with pixels cells apart a tube holds few of them: a
+// does the skewers of its 256 or more pixels one after the other, each in 10 us
+// or more however short it is.  With seven fields and 2e6 pixels in all dmax 1
+// takes 488 us against 685 at 50 pixels per skewer and 1005 against 790 at 20;
+// dmax 2 13.0 ms against 15.9 and dmax 3 21.5 against 44.1 at 2.  A batch that
+// does not fill the card waits for the block with the most skewers; k_gather
+// then takes as long as one pixel does, which its fields and cells decide.  Us,
+// k_gather_radial against k_gather, 30000 pixels in skewers of
+//                 5          20        45       100      300
+//   dmax 1, 7                          58, 29   37, 24   23, 23
+//           10                         61, 46   39, 39
+//   dmax 2, 7     555, 267   160, 115  80, 83
+//           10    587, 399
+//   dmax 3, 7     887, 696
+// (800000 pixels of dmax 1 in skewers of 45 218, 211; of dmax 2 in skewers of 5
+// 2312, 1790).
+//
+// And with pixels cells apart a tube holds few of them: a
 // million pixels along x or y, dmax 1, take 0.37 of k_gather's time at a half
 // of a cell, 0.45 at one, 0.8 at two, 0.9 at two and a half, 1.1 at three, 1.4
 // at four and 2.2 at eight (along z 0.9, 0.85, 0.85, 0.85, 0.8, 0.6, 0.8; dmax 2
 // 0.8 at the most, dmax 3 0.45).
-constexpr bool gather_radial(int dmax, int64_t n, int64_t pixels, double cells) {
-  if (dmax < 1 || pixels < (dmax == 1 ? 40 : 2) * n) return false;
+constexpr bool gather_radial(int dmax, int fields, int64_t n, int64_t pixels, double cells) {
+  if (dmax < 1) return false;
+  const bool fills = pixels >= 200000, ten = fields >= 10;
+  const int64_t mean = dmax == 1   ? (fills ? (ten ? 40 : 60) : (ten ? 100 : 150))
+                       : dmax == 2 ? (fills ? (ten ? 2 : 10) : (ten ? 10 : 30))
+                                   : (fills ? 2 : (ten ? 4 : 8));
+  if (pixels < mean * n) return false;
   return dmax > 1 || (cells <= 2.75 && cells >= -2.75);
 }
 
