@@ -68,9 +68,10 @@ constexpr int p1d_cut_rows(int n_par, int n_perp) {
 // Waves that a skewer of k_fgpa_flux and k_fgpa_flux_jac gets (eight waves to a
 // block).  Few skewers leave the card idle with one wave each, and a long one
 // is a long chain on one wave; but eight waves share a barrier per skewer,
-// which many skewers pay for.  One wave each also leaves a part of the last of
-// the blocks' rounds over the 256 CUs idle, which two waves halve.  Us with 1,
-// 2 and 8 waves, one parameter set per skewer:
+// which many skewers pay for.  One or two waves each also leave a part of the
+// last round of blocks over the 256 CUs idle: the lower the share in use with
+// the better of them, the sooner eight win.  Us with 1, 2 and 8 waves, one
+// parameter set per skewer:
 //             700 pixels        1400              3000             6500
 //     600     7.8  7.5  7.5     9.7  7.5  7.6     18   12   9.9    35   24   16
 //    1500     7.3  7.3  8.2     11.2 11.1 10.6    20.5 18.7 16.6   37   34   28
@@ -81,17 +82,28 @@ constexpr int p1d_cut_rows(int n_par, int n_perp) {
 //   10000     23   23.5 38      38   38   52      103  103  114    224  227  215
 //   20000     42   43   74      95   97   131     203  199  223    442  434  414
 // and with parameters per pixel 6500 pixels take 59, 43, 34.5 (1500 skewers),
-// 117, 106, 104 (3000) and 309, 329, 322 (10000).
+// 117, 106, 104 (3000) and 309, 329, 322 (10000).  Of eight waves against two,
+// 2100 skewers (68% of the rounds in use) of 3000 pixels take 0.92 of the time,
+// 2500 (81%) 0.98 and 2700 (88%) 1.02; of 4500 0.87, 0.93 and 0.98; 6300
+// (77%) of 4500 0.93.
+constexpr int64_t rounds_used(int64_t n, int64_t round) { return 100 * n / ((n + round - 1) / round * round); }
+
 constexpr int flux_waves(int64_t n, int64_t pixels, bool per_pixel) {
-  const int64_t mean = pixels / (n > 0 ? n : 1);
-  const int64_t round = 8 * 256;   // skewers, one wave each, in a round of the CUs
-  const bool idle = 20 * n < 17 * ((n + round - 1) / round * round);   // one wave each use less than 85% of the rounds
-  if (n <= round) {
-    if (mean >= (n <= 1200 ? 1400 : n <= 1536 ? 2000 : 8000)) return 8;
-    return mean >= (n <= 1200 || per_pixel ? 600 : 1400) ? 2 : 1;
-  }
-  if (mean >= 6000 && (idle || !per_pixel)) return 8;
-  return idle && mean >= (n <= 4096 ? 600 : 1000) ? 2 : 1;
+  if (n <= 0) return 1;
+  const int64_t mean = pixels / n;
+  const int64_t one = rounds_used(n, 8 * 256), two = rounds_used(n, 4 * 256), used = one > two ? one : two;
+  // eight
+  if (mean >= (n <= 1200 || (n <= 1536 && per_pixel) ? 1400 : n <= 1536 ? 2000 : 6000) &&
+      (n <= 4096 || one < 85 || !per_pixel))
+    return 8;
+  if (n <= 4096 && mean >= (used < 77 ? 2000 : used < 84 ? 3000 : used < 87 || (n > 3072 && used < 92) ? 4500 : 6000))
+    return 8;
+  if (n > 4096 && one < 82 && mean >= 4500) return 8;
+  // two
+  if (n <= 1024 || (n > 2048 && n <= 3072)) return mean >= 600 ? 2 : 1;
+  if (n <= 2048) return mean >= (per_pixel ? 600 : 1400) ? 2 : 1;
+  if (n <= 4096) return per_pixel && mean >= 1000 ? 2 : 1;
+  return one < 85 && two > one + 5 && mean >= 1000 ? 2 : 1;
 }
 
 // ------------------------------------------- smoothing along radial lines
