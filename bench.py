@@ -213,8 +213,8 @@ def forest_bench(delta, eta, shape, cell, steps, warmup, n_skewers):
             "ms_gather_gauss343": ms_gauss,
             "pixels_per_s": npx * steps / dt,
             "mean_flux": float(f.double().mean().item()),
-            # waves wait on memory and barriers most of their life (SQ counters),
-            # so neither HBM nor VALU issue is saturated: both fractions are given
+            # VALU issue is the nearer limit (SQ counters: in 63 to 70 % of its
+            # slots); the bytes against HBM are given beside it
             "roofline": {"bound": "valu", "alg_bytes": alg, "achieved": alg / (ms * 1e-3) / 1e9,
                          "peak": HBM_PEAK_GBPS, "unit": "GB/s", "frac": alg / (ms * 1e-3) / 1e9 / HBM_PEAK_GBPS,
                          "valu": forest_valu_roofline(ms, int(np.argmin(ms_var)))}}
@@ -279,7 +279,7 @@ def qso_bench(delta, eta, shape, cell, steps, warmup, nslice=16):
             "cells_per_s": cells / (ms * 1e-3),
             "roofline": {"bound": "hbm", "alg_bytes": alg, "achieved": alg / (ms * 1e-3) / 1e9,
                          "peak": HBM_PEAK_GBPS, "unit": "GB/s", "frac": alg / (ms * 1e-3) / 1e9 / HBM_PEAK_GBPS,
-                         "limiter": "HBM: the fields against a bound; then the FP64 draw of the cells left"}}
+                         "limiter": "VALU issue of the filter (86 %; its read of the fields 72 % of a read kernel's rate); then the FP64 draw of the cells left"}}
 
 
 P1D_BETA, P1D_DX, P1D_ZREF, P1D_DK = 1.6, 2.19, 2.2, 0.001

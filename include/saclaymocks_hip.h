@@ -548,8 +548,11 @@ int smk_qso_draw(const smk_qso_params* p, const float* p1, const float* p2, cons
                  int64_t* count, void* stream);
 
 /* The same draw (the same records) with a scratch buffer for a bit mask of
- * the cells that a bound on the first condition does not rule out: four times
- * faster where few cells pass it, as fast where all do.  scratch: device
+ * the cells that a bound on the first condition does not rule out.  In a slice
+ * of 6e8 cells four times faster where up to one cell in a hundred is drawn,
+ * slower where one in fourteen or more is (1.4 times at one in seven); in slices
+ * below 6.5e6 cells its three launches cost more than they save, and a caller
+ * better passes none.  scratch: device
  * memory, 8-byte aligned, of at least smk_qso_scratch_bytes (0.13 bytes per
  * cell on long columns), or NULL: smk_qso_draw.  Calls that share a scratch
  * buffer must not overlap. */
@@ -591,7 +594,7 @@ int smk_pk_table(const smk_pk_spline* spline, const float* kx, const float* ky, 
  *      D2 = k^3 P(k) G^2 / (2 pi^2)                 (P_RSD_Prats)
  *   2  exp(-dx^2 k^2) for k < kny, else 0           (PW2cut)
  * prats = {q1, q2, kp, kv, av, bv, G}; dx, kny used by model 2.
- * One block per k_par, FP64, deterministic.  out: device double [n_par]. */
+ * FP64, deterministic: a k_par is summed by one block, whatever the launch.  out: device double [n_par]. */
 int smk_p1d_rsd_rows(const smk_pk_spline* spline, const double* k_par, int n_par, const double* k_perp, int n_perp,
                      double beta, int model, const double* prats, double dx, double kny, double* out,
                      void* stream);

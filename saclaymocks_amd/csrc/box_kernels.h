@@ -694,7 +694,8 @@ __global__ __launch_bounds__(T*(M / E)) void k_z_c2r(const float2* __restrict__ 
 // form XCH (0 float2 line, 1 float line with the split exchange), in
 // spectral mode where the aux spectrum waits (TILES, see k_strided), and the
 // swizzle shift SWS of unpadded lines.  Variant 0 exists for every length;
-// the others for n >= 512, where the passes are long enough to tune.
+// the others for the tuned lengths from 512 on, 17 and 18 from 256 on
+// (smk_route::box_strided says which a plan starts with).
 struct SVar {
   int e, t, xch, tiles, sws, occ;
 };
@@ -728,7 +729,7 @@ constexpr int half_tile(int n) {
   return (e0 % 2 == 0 && plan_ok(n, e0 / 2) && n / (e0 / 2) <= 512) ? e0 / 2 : 0;
 }
 
-// Variants (n >= 512; "swz" ones only for the unpadded 1280- and 2560-point
+// Variants (tuned lengths, n >= 512; "swz" ones only for the unpadded 1280- and 2560-point
 // lines, whose LDS exchange needs a swizzle; the stash ones only in spectral
 // mode):
 //   0  E0, float2 exchange            5  E0, split exchange, SWS 3 (swz)

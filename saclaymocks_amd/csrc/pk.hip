@@ -574,7 +574,7 @@ extern "C" int smk_pk_table(const smk_pk_spline* spline, const float* kx, const 
     return SMK_OK;
   }
   const bool lds = route == smk_route::PK_ROWS_LDS;
-  // two blocks of 16 waves per CU; or as many waves as there are pieces, of which fewer than 2^18
+  // two blocks of 16 waves per CU; or as many waves as there are pieces, four to a block: fewer than 2^18 blocks
   const uint64_t blocks = lds ? 512 : (a.ngroup * a.nch + 3) / 4, waves = blocks * (lds ? 16 : 4);
   a.dgroup = waves / a.nch;
   a.dch = (uint32_t)(waves % a.nch);

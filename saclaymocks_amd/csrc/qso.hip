@@ -206,15 +206,17 @@ __global__ __launch_bounds__(256) void k_qso_draw(smk_qso_params p, const float*
 // draw_cell would draw is left out.
 //
 // Measured on a slice of 160 x 2560 x 1536 cells: k_qso_draw 7.7 ms, bound by
-// its FP64 lookups per cell; this way 1.67, of which the filter 1.55 (4.9 TB/s,
-// the card's copy rate) and the bounds 0.05 (0.16 with one per 8 columns; found
+// its FP64 lookups per cell; this way 1.67, of which the filter 1.55 (its VALU
+// issues in 86% of the slots, 8.2e8 instructions; 4.9 TB/s, 72% of the rate of a
+// kernel that only reads) and the bounds 0.05 (0.16 with one per 8 columns; found
 // inside the filter's blocks 0.7, as a block waits for a few lanes' chains).
 // With 10 and 100 times as many cells that pass, 10.4 and 20.5 ms against 1.97
-// and 4.4; only with all of them (75 million quasars) k_qso_draw is the faster,
-// 47 against 63.  draw_cell has a kernel of its own since in the filter's loop
-// it took 216 registers (2 waves per SIMD, 9.4 ms), as a call from there 7.0.  In k_qso_masked's loop the compiler keeps its
-// constants in registers, 199 of them if it may; 128 were faster at every
-// density.  A bit per cell never overflows; a list of cells did, or was as
+// and 4.4; with a quasar in 5% of all cells k_qso_draw is still the slower, with
+// one in 7% or more it is the faster, 47 against 65 at 15%.  draw_cell has a
+// kernel of its own since in the filter's loop it took 216 registers (2 waves
+// per SIMD, 9.4 ms), as a call from there 7.0.  In k_qso_masked's loop the
+// compiler keeps its constants in registers, 199 of them if it may; 128 were
+// faster at every density.  A bit per cell never overflows; a list of cells did, or was as
 // large as a field.
 constexpr int CHUNK = 128;        // cells along z of one bound: two waves
 constexpr int BCOLS = 32;         // columns of one bound

@@ -8,8 +8,7 @@ pi / DX), both clipped at 0 and splined (p1d_missing.py:113-186).  The RSD
 variant integrates the 3-D spectrum (1 + beta mu^2)^2 P(k) [D_NL(k, mu)]
 over k_perp for every k_par (powerspectrum.py:36-49); at the reference's
 default grid (k_max = 20, dk = 0.001) that is 2 x 4e8 evaluations of the
-spline, which smk_p1d_rsd_rows does on the device, one block per k_par row,
-in FP64.  The O(n) pieces (the 1-D cumulative trapezoid, the scipy spline
+spline, which smk_p1d_rsd_rows does on the device, in FP64.  The O(n) pieces (the 1-D cumulative trapezoid, the scipy spline
 fits of the rows) stay on the host as in the reference.
 """
 import ctypes
